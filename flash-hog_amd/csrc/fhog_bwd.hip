@@ -31,21 +31,11 @@ constexpr int kThreads = 64 * kWaves;
 constexpr int kStages = 4;  // 3 stages: 2.6 % slower at B4 N2048 H16
 
 // Waves per SIMD the register allocator is asked to allow: two for 2-byte
-// types at D = 64 and 128 (at D = 128 the dQ kernel takes 238 VGPRs and the
-// dK/dV kernel, in two column passes, 242; first backward at B4 N2048 H16
-// causal 495 -> 403-417 us), one otherwise.
+// types at D = 64 and 128 (at D = 128 the dQ kernel takes 238 VGPRs), one
+// otherwise.
 template <typename T, int D> struct Occupancy {
   static constexpr int value = (sizeof(T) == 2 && D <= 128) ? 2 : 1;
 };
-// Whether the dK/dV kernel runs as two passes over halves of the output
-// columns (each forming the full scores): at D = 256 all columns'
-// accumulators beside the resident K and V spilled 740 bytes per lane; for
-// 2-byte types at D = 128 they took 401 registers (one wave per SIMD) against
-// 242 per pass (two waves).
-template <typename T, int D> struct KSplit {
-  static constexpr bool value = D > 128 || (sizeof(T) == 2 && D == 128);
-};
-
 
 template <typename T, int D, bool CAUSAL>
 __global__ void __launch_bounds__(kThreads)
@@ -212,17 +202,15 @@ bwd_q_kernel(BwdParams<T> p, int chunk) {
 // dword DMAs and, once they have landed, rewrites them in LDS as the initial
 // values of the S and dP accumulators (-L / scale and -D).
 //
-// With KSplit (2-byte types at D = 128 and 256) the launcher runs the kernel
-// twice, for output column blocks [C0, C0 + DTO) with C0 = 0 and D / 64, each
-// pass forming the full scores again, so that the dK and dV accumulators of
-// half the columns fit beside the resident K and V.
-template <typename T, int D, bool CAUSAL, int C0>
+// It serves 2-byte types at D = 64; every other type and head dim, and small
+// grids at D = 64, run bwd_pair_kernel (fhog_bwd_pair.hip).
+template <typename T, int D, bool CAUSAL>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(Occupancy<T, D>::value, Occupancy<T, D>::value)))
 bwd_k_kernel(BwdParams<T> p, int chunk) {
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 16;
-  constexpr int DTO = KSplit<T, D>::value ? D / 64 : D / 32;  // 32-column output blocks of this pass
+  constexpr int DT = D / 32;
   constexpr int BKB = 32 * kWaves;
   constexpr int BQ = 32;
   constexpr int NST = kStages;
@@ -263,9 +251,9 @@ bwd_k_kernel(BwdParams<T> p, int chunk) {
   const int qt_begin = CAUSAL ? max(0, kb * BKB - p.coff) / BQ : 0;
   const int total = nqt > qt_begin ? (nqt - qt_begin) * grp : 0;
 
-  f32x16 acc_dk[DTO], acc_dv[DTO];
+  f32x16 acc_dk[DT], acc_dv[DT];
 #pragma unroll
-  for (int dt = 0; dt < DTO; ++dt) acc_dk[dt] = acc_dv[dt] = zero16();
+  for (int dt = 0; dt < DT; ++dt) acc_dk[dt] = acc_dv[dt] = zero16();
 
   if (total > 0) {
     V8<T> kf[KS], vf[KS];
@@ -399,9 +387,9 @@ bwd_k_kernel(BwdParams<T> p, int chunk) {
           const V8<T> oP = cvt8<T>(s ? hi8(P) : lo8(P));
           const V8<T> oS = cvt8<T>(vdS);
 #pragma unroll
-          for (int dt = 0; dt < DTO; ++dt) {
-            acc_dv[dt] = mma<T>(fr.trf(sa, kTile, C0 + dt, s), oP, acc_dv[dt]);
-            acc_dk[dt] = mma<T>(fr.trf(sa, 0, C0 + dt, s), oS, acc_dk[dt]);
+          for (int dt = 0; dt < DT; ++dt) {
+            acc_dv[dt] = mma<T>(fr.trf(sa, kTile, dt, s), oP, acc_dv[dt]);
+            acc_dk[dt] = mma<T>(fr.trf(sa, 0, dt, s), oS, acc_dk[dt]);
           }
         }
       }
@@ -412,10 +400,10 @@ bwd_k_kernel(BwdParams<T> p, int chunk) {
     T* dk = p.dk + kbase + (long)kj * rsk;
     T* dv = p.dv + kbase + (long)kj * rsk;
 #pragma unroll
-    for (int dt = 0; dt < DTO; ++dt) {
+    for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
-        const int d = 32 * (C0 + dt) + 8 * a + 4 * g;
+        const int d = 32 * dt + 8 * a + 4 * g;
         f32x4 x, y;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -431,19 +419,27 @@ bwd_k_kernel(BwdParams<T> p, int chunk) {
 
 }  // namespace
 
-// The first backward for 2-byte types at D = 64 has two kernels for each
-// half of its work: dK/dV in bwd_k_kernel above or in bwd_k64_kernel
-// (fhog_bwd_k64.hip: 64 keys per wave at one wave per SIMD, generated sweep),
-// dQ in bwd_q_kernel above or in bwd_q64_kernel (fhog_bwd_q64.hip, the same
-// with 64 queries per wave). A one-wave kernel runs one 256-row block per CU
+// The first backward for 2-byte types at D = 64 has several kernels for each
+// half of its work, all giving the same bits: dK/dV in bwd_k_kernel above, in
+// bwd_k64_kernel (fhog_bwd_k64.hip: 64 keys per wave at one wave per SIMD,
+// generated sweep) or in bwd_pair_kernel (fhog_bwd_pair.hip: two waves per 32
+// keys), dQ in bwd_q_kernel above or in bwd_q64_kernel (fhog_bwd_q64.hip, 64
+// queries per wave). A one-wave kernel runs one 256-row block per CU
 // at a time and gains nothing when a CU is left alone, so it is taken when
 // its grid fills whole rounds of the resident workgroups (or at least six),
 // and the compiled kernel, whose second workgroup per CU runs faster alone,
 // otherwise: first backward at B4 N2048 H16 causal bf16 138.7-140.7 us with
 // both one-wave kernels against 148.5-149.1 with both compiled ones, while
 // at B8 N2048 H12 causal (1.5 rounds) the one-wave dQ kernel took 258
-// against 241 us. FLASH_HOG_BWD (dK/dV) and FLASH_HOG_BWDQ (dQ) = compiled or
-// k64 / q64 force a kernel; read at every launch.
+// against 241 us. The pair kernel does more LDS work per tile but takes half
+// the time per tile of a wave, and its grid has twice the workgroups: it is
+// taken while that grid has at most two workgroups per CU, three when causal
+// (half the pairs). First backward, us, compiled / pair: causal B1 N1024 H12
+// (192 workgroups) 52.4 / 46.5, B1 N4096 H12 (768) 184 / 166, B2 N4096 H16 over
+// 4 key heads (512) 523 / 446, but B2 N2048 H16 (1024) 101 / 108; non-causal
+// B1 N2048 H16 (512) 95.2 / 92.9, but B2 N2048 H12 (768) 121 / 142.
+// FLASH_HOG_BWD (dK/dV) = compiled, k64 or pair and FLASH_HOG_BWDQ (dQ) =
+// compiled or q64 force a kernel; read at every launch.
 inline bool one_wave_grid(int workgroups, int resident) {
   return resident > 0 && workgroups > 0 && (workgroups % resident == 0 || workgroups >= 6 * resident);
 }
@@ -455,11 +451,16 @@ inline bool one_wave_selected(const char* var, const char* name, int nb, int npa
   const int pairs = block_pairing(causal, nb, npairs, resident, 1);
   return one_wave_grid((pairs ? (nb + 1) / 2 : nb) * npairs, resident);
 }
+inline bool pair_selected(int nk, int npairs, bool causal) {
+  const char* v = std::getenv("FLASH_HOG_BWD");
+  if (v != nullptr && std::strcmp(v, "pair") == 0) return true;
+  if (v != nullptr && (std::strcmp(v, "compiled") == 0 || std::strcmp(v, "k64") == 0)) return false;
+  return (long)((nk + 63) / 64) * npairs <= (long)(causal ? 3 : 2) * resident_workgroups(1);
+}
 
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd(const BwdParams<T>& p, hipStream_t stream) {
   const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
-  const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
   const int resident = resident_workgroups(Occupancy<T, D>::value);
   const int nq_pairs = p.batch * p.heads, nk_pairs = p.batch * p.kv_heads;
   hipError_t e = hipSuccess;
@@ -476,17 +477,16 @@ hipError_t launch_bwd(const BwdParams<T>& p, hipStream_t stream) {
   if (e == hipSuccess) e = hipGetLastError();
   if (e != hipSuccess) return e;
   if constexpr (sizeof(T) == 2 && D == 64) {
-    if (one_wave_selected("FLASH_HOG_BWD", "k64", (p.nk + 255) / 256, nk_pairs, CAUSAL))
-      return launch_bwd_k64<T, CAUSAL>(p, stream);
+    if (!pair_selected(p.nk, nk_pairs, CAUSAL)) {
+      if (one_wave_selected("FLASH_HOG_BWD", "k64", (p.nk + 255) / 256, nk_pairs, CAUSAL))
+        return launch_bwd_k64<T, CAUSAL>(p, stream);
+      const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
+      hipLaunchKernelGGL((bwd_k_kernel<T, D, CAUSAL>), dim3(nkb * nk_pairs), dim3(kThreads), 0, stream, p,
+                         grid_chunk(nk_pairs, nkb, resident));
+      return hipGetLastError();
+    }
   }
-  hipLaunchKernelGGL((bwd_k_kernel<T, D, CAUSAL, 0>), dim3(nkb * nk_pairs), dim3(kThreads), 0, stream, p,
-                     grid_chunk(nk_pairs, nkb, resident));
-  if constexpr (KSplit<T, D>::value) {
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL((bwd_k_kernel<T, D, CAUSAL, D / 64>), dim3(nkb * nk_pairs), dim3(kThreads), 0, stream, p,
-                       grid_chunk(nk_pairs, nkb, resident));
-  }
-  return hipGetLastError();
+  return launch_bwd_pair<T, D, CAUSAL>(p, stream);
 }
 
 #define FHOG_INST(T, D, C) template hipError_t launch_bwd<T, D, C>(const BwdParams<T>&, hipStream_t);

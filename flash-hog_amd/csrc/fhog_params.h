@@ -81,6 +81,10 @@ hipError_t launch_bwd_k64(const BwdParams<T>& p, hipStream_t s);
 // (2-byte types, D = 64); launch_bwd selects it for grids of whole rounds.
 template <typename T, bool CAUSAL>
 hipError_t launch_bwd_q64(const BwdParams<T>& p, hipStream_t s);
+// dK and dV of the first backward with two waves per 32 keys (all types and
+// head dims; at 2-byte D = 64 launch_bwd selects it for small grids).
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_bwd_pair(const BwdParams<T>& p, hipStream_t s);
 // Stage 2 with 16 keys per wave (2-byte types, D = 128); launch_bwdbwd selects it.
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwdbwd_stage2_k16(const BwdBwdParams<T>& p, hipStream_t s);
