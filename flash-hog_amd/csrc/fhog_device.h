@@ -546,6 +546,16 @@ inline int grid_chunk(int npairs, int nranks, int resident) {
   return c < 8 ? 8 : (c < npairs ? c : npairs);
 }
 
+// First rank that runs backwards (block nb - 1 - (rank - fold)) in a grid of nb
+// causal blocks, longest first, per (batch, head) pair. A grid of one to two
+// workgroups per CU runs as one round in which workgroups i and i + (number of
+// CUs) share a CU: the second of them take their ranks backwards, so that the
+// shortest blocks sit beside the longest. nb: none does.
+inline int fold_rank(bool causal, int nb, int npairs, int cus) {
+  const long grid = (long)nb * npairs;
+  return causal && cus > 0 && grid > cus && grid <= 2L * cus ? (cus + npairs - 1) / npairs : nb;
+}
+
 // The `pairs` argument of block_pair for a grid of nb causal blocks per
 // (batch, head) pair: mirror pairs when the unpaired grid outnumbers the
 // resident workgroups, skewed ones when the paired grid is exactly one round
