@@ -337,7 +337,8 @@ bwdbwd_q_kernel(BwdBwdParams<T> p, int chunk) {
 // (Q, dO, ddQ) global -> LDS; wave 3 streams the tiles' row statistics and
 // turns them into the four per-query constants (-L log2(e), -D, -dD,
 // -(D dD + B)) in LDS. The loop issues no load the compiler tracks, so its
-// only vector-memory waits are the explicit ones.
+// only vector-memory waits are the explicit ones. It serves 2-byte types at
+// D = 64; other types and head dims run bwdbwd_pair_kernel.
 // ----------------------------------------------------------------------------
 template <typename T, int D, bool CAUSAL, bool PRE>
 __global__ void __launch_bounds__(kThreads)
@@ -417,6 +418,7 @@ bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk) {
       // place as the initial values of the four score accumulators:
       // -L / scale, -dD / scale, -D, -(D dD + B) (-L and -dD when K and ddK carry
       // the scale).
+      static_assert(NST >= 3, "the statistics are finished one tile ahead");
       constexpr int kStatLoads = 4;  // two per lane half
       auto issue_stats = [&](int i, GroupCursor c) {
         // uniform row base plus a per-lane offset; each lane half loads its own tensor
@@ -445,13 +447,10 @@ bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk) {
       // Waits (wave 3) until the statistics of tile i have landed: the DMAs of
       // later tiles, at most NST - 2 of them, may still be in flight.
       auto wait_stats = [&](int i) {
-        if constexpr (NST >= 3) {
-          if (i + NST - 2 < total) {
-            wait_vmem_le<(NST - 2) * kStatLoads>();
-            return;
-          }
-        }
-        wait_vmem_le<0>();
+        if (i + NST - 2 < total)
+          wait_vmem_le<(NST - 2) * kStatLoads>();
+        else
+          wait_vmem_le<0>();
       };
       auto issue = [&](int i, GroupCursor c) {
         if (wave == 3) {
@@ -530,16 +529,13 @@ bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk) {
           issue(i + NST - 1, nxt);
           advance(nxt);
         }
-        // Tile i + 1's statistics are read after the next barrier. With a ring
-        // of three or more stages their DMA went out two or more iterations
-        // ago, and they are finished here, before this tile's work, so that
-        // the LDS round trip overlaps wave 3's own products instead of
-        // delaying the barrier; with two stages, after this tile's work.
-        if constexpr (NST >= 3) {
-          if (wave == 3 && i + 1 < total) {
-            wait_stats(i + 1);
-            finish_stats(i + 1);
-          }
+        // Tile i + 1's statistics are read after the next barrier. Their DMA went
+        // out two or more iterations ago, and they are finished here, before this
+        // tile's work, so that the LDS round trip overlaps wave 3's own products
+        // instead of delaying the barrier.
+        if (wave == 3 && i + 1 < total) {
+          wait_stats(i + 1);
+          finish_stats(i + 1);
         }
         const int q0 = (qt_begin + cur.qt) * BQ;
         const bool active = k0 < p.nk && (!CAUSAL || q0 + BQ - 1 >= k0 - p.coff);
@@ -614,12 +610,6 @@ bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk) {
             }
           }
         }
-        if constexpr (NST < 3) {
-          if (wave == 3 && i + 1 < total) {
-            wait_stats(i + 1);
-            finish_stats(i + 1);
-          }
-        }
       }
     }
 
@@ -661,20 +651,30 @@ inline bool stage1_fused_selected() {
   return v != nullptr && std::strcmp(v, "fused") == 0;
 }
 
-// Stage 2 for bf16 at D = 64 runs bwdbwd_k_kernel below (32 keys per wave,
-// two waves per SIMD) unless FLASH_HOG_STAGE2=k32 selects the kernel with a
-// generated sweep at one wave per SIMD (fhog_bwdbwd_k32.hip). Both give the
-// same results to rounding; at B4 N2048 H16 D64 causal bf16 the compiled
-// kernel is about 10 % faster. Read at every launch.
-inline bool stage2_k32_selected() {
-  const char* v = std::getenv("FLASH_HOG_STAGE2");
-  return v != nullptr && std::strcmp(v, "k32") == 0;
+// Stage 2 runs bwdbwd_pair_kernel (fhog_bwdbwd_pair.hip, two waves per 32 keys)
+// but for 2-byte types at D = 64 on grids that fill the chip, where
+// bwdbwd_k_kernel's one wave per 32 keys is faster; both give the same bits.
+// The pair kernel's grid has twice the workgroups of half the work each, and
+// is taken while it has at most three of them per CU when causal, one
+// otherwise (stage 2, us, k / pair: causal B1 N512 H12 24.8 / 20.2, B1 N2048
+// H12 (384 workgroups) 78.4 / 69.7, B2 N2048 H12 (768) 85.2 / 74.8, B2 N4096
+// H16 over 4 key heads (512) 575 / 511, but B2 N2048 H16 (1024) 93.3 / 95.8 and
+// B1 N8192 H12 (1536) 452 / 497; non-causal B1 N300 over one key head 51.9 /
+// 44.2, but B1 N2048 H12 (384) 79.6 / 82.4, B2 N1000 H12 fp16 43.9 / 48.0).
+// FLASH_HOG_STAGE2 = compiled (bwdbwd_k_kernel) or pair forces either, and k32
+// selects, for bf16, the kernel with a generated sweep at one wave per SIMD
+// (fhog_bwdbwd_k32.hip), which agrees to rounding and is about 10 % slower at B4
+// N2048 H16. Read at every launch.
+inline bool stage2_selected(const char* v, const char* name) { return v != nullptr && std::strcmp(v, name) == 0; }
+inline bool stage2_pair_selected(const char* v, int nk, int npairs, bool causal) {
+  if (stage2_selected(v, "pair")) return true;
+  if (stage2_selected(v, "compiled")) return false;
+  return (long)((nk + 63) / 64) * npairs <= (long)(causal ? 3 : 1) * resident_workgroups(1);
 }
 
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stages) {
   const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
-  const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
   if (stages & 1) {
     hipError_t e;
     if constexpr (sizeof(T) == 2 && D == 64) {
@@ -691,12 +691,14 @@ hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stage
     if (e != hipSuccess) return e;
   }
   if (stages & 2) {
-    if constexpr (sizeof(T) == 2 && D >= 128) {
-      return launch_bwdbwd_stage2_k16<T, D, CAUSAL>(p, stream);
-    } else {
-      if constexpr (std::is_same_v<T, __bf16> && D == 64) {
-        if (stage2_k32_selected()) return launch_bwdbwd_stage2_k32<CAUSAL>(p, stream);
+    if constexpr (sizeof(T) == 2 && D == 64) {
+      const char* variant = std::getenv("FLASH_HOG_STAGE2");
+      if constexpr (std::is_same_v<T, __bf16>) {
+        if (stage2_selected(variant, "k32")) return launch_bwdbwd_stage2_k32<CAUSAL>(p, stream);
       }
+      if (stage2_pair_selected(variant, p.nk, p.batch * p.kv_heads, CAUSAL))
+        return launch_bwdbwd_stage2_pair<T, D, CAUSAL>(p, stream);
+      const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
       // Pair causal key blocks when the grid outnumbers the resident workgroups.
       const int npairs = p.batch * p.kv_heads;
       const int resident = resident_workgroups(Occupancy<T, D>::value);
@@ -711,6 +713,8 @@ hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stage
       else
         hipLaunchKernelGGL((bwdbwd_k_kernel<T, D, CAUSAL, false>), grid, dim3(kThreads), 0, stream, p, pairs, chunk);
       return hipGetLastError();
+    } else {
+      return launch_bwdbwd_stage2_pair<T, D, CAUSAL>(p, stream);
     }
   }
   return hipSuccess;

@@ -85,8 +85,9 @@ hipError_t launch_bwd_q64(const BwdParams<T>& p, hipStream_t s);
 // head dims; at 2-byte D = 64 launch_bwd selects it for small grids).
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd_pair(const BwdParams<T>& p, hipStream_t s);
-// Stage 2 with 16 keys per wave (2-byte types, D = 128); launch_bwdbwd selects it.
+// Stage 2 with two waves per 32 keys (all types and head dims; at 2-byte
+// D = 64 launch_bwdbwd selects it for small grids).
 template <typename T, int D, bool CAUSAL>
-hipError_t launch_bwdbwd_stage2_k16(const BwdBwdParams<T>& p, hipStream_t s);
+hipError_t launch_bwdbwd_stage2_pair(const BwdBwdParams<T>& p, hipStream_t s);
 
 }  // namespace fhog
