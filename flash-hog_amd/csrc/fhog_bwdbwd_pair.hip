@@ -24,7 +24,7 @@
 //
 // Stage 2, us, before -> with this kernel: causal bf16 B2 N8192 H16 D128
 // 2525 -> 2189, B2 N2048 H32 over 8 key heads D128 574 -> 396, B2 N2048 H8
-// D256 278 -> 260; fp32 B2 N2048 H8 D64 565 -> 366, B1 N2048 H8 D128
+// D256 278 -> 213; fp32 B2 N2048 H8 D64 565 -> 366, B1 N2048 H8 D128
 // non-causal 1285 -> 665; D = 64 small grids: B1 N1024 H12 42.4 -> 35.7, B1
 // N4096 H12 161 -> 144. At D = 64 the exchange is two thirds of the operand
 // reads, and grids that fill the chip keep bwdbwd_k_kernel (B4 N2048 H16 147

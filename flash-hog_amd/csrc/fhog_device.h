@@ -340,10 +340,13 @@ template <typename T, int D, int COUNT = SwzTile<T, D>::kLoads, int SWZ = kSwzPa
 // stage to a fixed per-lane offset (shared by every tile of the stage) with
 // the constant in the instruction's offset field; computing addresses from
 // pointers instead leaves the compiler to rebuild the swizzled offsets inside
-// the loop when registers are scarce.
+// the loop when registers are scarce. The swizzle permutes chunks within
+// aligned groups of eight (128 bytes, 64 columns), so the offsets of the first 64
+// columns serve the others with a constant: six registers whatever D, where
+// offsets for every column block took 12 at D = 128 and 24 at D = 256.
 template <typename T, int D> struct SwzFrags {
-  uint32_t row[D / 16];  // row operand of step ks
-  uint32_t tr[D / 32];   // first transposed read of column block dt, step 0 (rows 4 g + i / 4)
+  uint32_t row[4];  // row operand of steps ks = 0..3 (columns 0..63)
+  uint32_t tr[2];   // first transposed read of column blocks dt = 0, 1, step 0 (rows 4 g + i / 4)
   int lane;
 
   __device__ __forceinline__ void init(int lane_id) {
@@ -351,12 +354,12 @@ template <typename T, int D> struct SwzFrags {
     if constexpr (sizeof(T) == 2) {
       const int n = lane & 31, g = lane >> 5;
 #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks)
+      for (int ks = 0; ks < 4; ++ks)
         row[ks] = 2u * (uint32_t)(n * D + 8 * phys_chunk(n, 2 * ks + g));
       const int i = lane & 15;
       const int r = 4 * g + (i >> 2);
 #pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt) {
+      for (int dt = 0; dt < 2; ++dt) {
         const int d = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (i & 3);
         tr[dt] = 2u * (uint32_t)(r * D + 8 * phys_chunk(r, d >> 3) + (d & 7));
       }
@@ -366,8 +369,8 @@ template <typename T, int D> struct SwzFrags {
   // Operand contracting over columns: lane (n, g) gets row n, columns 16 ks + 8 g .. +7.
   __device__ __forceinline__ V8<T> rowf(uint32_t stage, int off, int ks) const {
     if constexpr (sizeof(T) == 2) {
-      const lds_cchar* p = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[ks]));
-      return *reinterpret_cast<const __attribute__((address_space(3))) V8<T>*>(p + off);
+      const lds_cchar* p = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[ks & 3]));
+      return *reinterpret_cast<const __attribute__((address_space(3))) V8<T>*>(p + off + 128 * (ks >> 2));
     } else {
       return frag_row_swz<T, D>(tile_ptr(stage, off), lane & 31, lane >> 5, ks);
     }
@@ -385,9 +388,10 @@ template <typename T, int D> struct SwzFrags {
   // be a multiple of 32, which every ring stage and tile offset here is.
   __device__ __forceinline__ V8<T> trf(uint32_t stage, int off, int dt, int s) const {
     if constexpr (sizeof(T) == 2) {
-      const uint32_t a0 = stage + tr[dt];
-      const lds_cchar* a = reinterpret_cast<const lds_cchar*>((uintptr_t)a0) + off + s * 32 * D;
-      const lds_cchar* b = reinterpret_cast<const lds_cchar*>((uintptr_t)(a0 ^ 16u)) + off + s * 32 * D + 16 * D;
+      const uint32_t a0 = stage + tr[dt & 1];
+      const int o = off + 128 * (dt >> 1) + s * 32 * D;
+      const lds_cchar* a = reinterpret_cast<const lds_cchar*>((uintptr_t)a0) + o;
+      const lds_cchar* b = reinterpret_cast<const lds_cchar*>((uintptr_t)(a0 ^ 16u)) + o + 16 * D;
       const i16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(a));
       const i16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(b));
       return __builtin_shufflevector(__builtin_bit_cast(V4<T>, x), __builtin_bit_cast(V4<T>, y), 0, 1, 2, 3, 4, 5,
@@ -452,15 +456,16 @@ __device__ __forceinline__ float group4_sum(float x) {
 // swizzled 32 x D tile (2-byte types).
 template <typename T, int D> struct SwzFrags16 {
   static_assert(sizeof(T) == 2, "2-byte types only");
-  uint32_t row[D / 32];  // score A operand: row l % 16, columns 32 ks + 8 (l / 16) .. +7
-  uint32_t tr[D / 16];   // output A operand of column block db: rows 4 (l / 16) + i / 4
+  // Offsets of the first 64 columns (see SwzFrags).
+  uint32_t row[2];  // score A operand: row l % 16, columns 32 ks + 8 (l / 16) .. +7
+  uint32_t tr[4];   // output A operand of column block db: rows 4 (l / 16) + i / 4
   __device__ __forceinline__ void init(int lane) {
     const int n = lane & 15, g = lane >> 4;
 #pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) row[ks] = 2u * (uint32_t)(n * D + 8 * phys_chunk<kSwzRows>(n, 4 * ks + g));
+    for (int ks = 0; ks < 2; ++ks) row[ks] = 2u * (uint32_t)(n * D + 8 * phys_chunk<kSwzRows>(n, 4 * ks + g));
     const int r = 4 * g + (n >> 2);
 #pragma unroll
-    for (int db = 0; db < D / 16; ++db) {
+    for (int db = 0; db < 4; ++db) {
       const int d = 16 * db + 4 * (n & 3);
       tr[db] = 2u * (uint32_t)(r * D + 8 * phys_chunk<kSwzRows>(r, d >> 3) + (d & 7));
     }
@@ -468,14 +473,14 @@ template <typename T, int D> struct SwzFrags16 {
   // Keys 16 kb + l % 16 of the tile at stage + off, step ks. The swizzle
   // repeats every 16 rows, so kb is a constant offset.
   __device__ __forceinline__ V8<T> rowf(uint32_t stage, int off, int kb, int ks) const {
-    const lds_cchar* p = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[ks])) + off + kb * 16 * D * 2;
+    const lds_cchar* p = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[ks & 1])) + off + 128 * (ks >> 1) + kb * 16 * D * 2;
     return *reinterpret_cast<const __attribute__((address_space(3))) V8<T>*>(p);
   }
   // Column 16 db + l % 16, keys 4 g + {0..3} and 16 + 4 g + {0..3}: within a
   // 16-lane group, lane i addresses row 4 g + i / 4, columns 16 db + 4 (i % 4)
   // .. +3, and receives column 16 db + i of the four rows.
   __device__ __forceinline__ V8<T> trf(uint32_t stage, int off, int db) const {
-    const lds_cchar* a = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + tr[db])) + off;
+    const lds_cchar* a = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + tr[db & 3])) + off + 128 * (db >> 2);
     const i16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(a));
     const i16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(a + 16 * D * 2));
     return __builtin_shufflevector(__builtin_bit_cast(V4<T>, x), __builtin_bit_cast(V4<T>, y), 0, 1, 2, 3, 4, 5, 6,
