@@ -58,6 +58,7 @@ SOURCE_FLAGS: dict[str, list[str]] = {
     "fhog_bwd_k64.hip": _MAX_ILP,
     "fhog_bwd_pair.hip": _MAX_ILP,
     "fhog_bwd_q64.hip": _MAX_ILP,
+    "fhog_bwd_qpair.hip": _MAX_ILP,
     "fhog_bwdbwd.hip": _MAX_ILP,
     "fhog_bwdbwd_pair.hip": _MAX_ILP,
     "fhog_fwd.hip": _MAX_ILP,

@@ -6,7 +6,8 @@
 // flash_hog/_jax_refs/jax_impl.py:142-191 (attn_bwd).
 //
 // Kernel 1 (tiled over queries) computes D for its rows, writes it, and
-// accumulates dQ while streaming K and V. Kernel 2 (tiled over keys) reads L
+// accumulates dQ while streaming K and V; fp32, head dim 256 and small grids
+// run it with two waves per 32 queries (fhog_bwd_qpair.hip). Kernel 2 (tiled over keys) reads L
 // and D and accumulates dK and dV while streaming Q and dO. Both stream their
 // tiles global -> LDS (no registers) through a 4-stage ring of XOR-swizzled
 // tiles with one barrier per tile, issue causal blocks longest first with
@@ -30,16 +31,13 @@ constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kStages = 4;  // 3 stages: 2.6 % slower at B4 N2048 H16
 
-// Waves per SIMD the register allocator is asked to allow: two for 2-byte
-// types at D = 64 and 128 (at D = 128 the dQ kernel takes 238 VGPRs), one
-// otherwise.
-template <typename T, int D> struct Occupancy {
-  static constexpr int value = (sizeof(T) == 2 && D <= 128) ? 2 : 1;
-};
+// Waves per SIMD the register allocator is asked to allow (2-byte types at
+// D = 64 and 128; at D = 128 the dQ kernel takes 228 VGPRs).
+constexpr int kOcc = 2;
 
 template <typename T, int D, bool CAUSAL>
 __global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(Occupancy<T, D>::value, Occupancy<T, D>::value)))
+__attribute__((amdgpu_waves_per_eu(kOcc, kOcc)))
 bwd_q_kernel(BwdParams<T> p, int chunk) {
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 16;
@@ -80,12 +78,7 @@ bwd_q_kernel(BwdParams<T> p, int chunk) {
       qf[ks] = *reinterpret_cast<const V8<T>*>(p.q + off);
       dof[ks] = *reinterpret_cast<const V8<T>*>(p.dout + off);
       const V8<T> of = *reinterpret_cast<const V8<T>*>(p.o + off);
-      if constexpr (sizeof(T) == 2) {
-        dpart = dot8<T>(of, dof[ks], dpart);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) dpart += (float)of[e] * (float)dof[ks][e];
-      }
+      dpart = dot8<T>(of, dof[ks], dpart);
     } else {
       qf[ks] = zero8<T>();
       dof[ks] = zero8<T>();
@@ -203,10 +196,10 @@ bwd_q_kernel(BwdParams<T> p, int chunk) {
 // values of the S and dP accumulators (-L / scale and -D).
 //
 // It serves 2-byte types at D = 64; every other type and head dim, and small
-// grids at D = 64, run bwd_pair_kernel (fhog_bwd_pair.hip).
+// grids at D = 64, run bwd_pair_kernel (fhog_bwd_pair.h).
 template <typename T, int D, bool CAUSAL>
 __global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(Occupancy<T, D>::value, Occupancy<T, D>::value)))
+__attribute__((amdgpu_waves_per_eu(kOcc, kOcc)))
 bwd_k_kernel(BwdParams<T> p, int chunk) {
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 16;
@@ -422,9 +415,10 @@ bwd_k_kernel(BwdParams<T> p, int chunk) {
 // The first backward for 2-byte types at D = 64 has several kernels for each
 // half of its work, all giving the same bits: dK/dV in bwd_k_kernel above, in
 // bwd_k64_kernel (fhog_bwd_k64.hip: 64 keys per wave at one wave per SIMD,
-// generated sweep) or in bwd_pair_kernel (fhog_bwd_pair.hip: two waves per 32
-// keys), dQ in bwd_q_kernel above or in bwd_q64_kernel (fhog_bwd_q64.hip, 64
-// queries per wave). A one-wave kernel runs one 256-row block per CU
+// generated sweep) or in bwd_pair_kernel (fhog_bwd_pair.h: two waves per 32
+// keys), dQ in bwd_q_kernel above, in bwd_q64_kernel (fhog_bwd_q64.hip, 64
+// queries per wave) or in bwd_qpair_kernel (fhog_bwd_qpair.hip: two waves per 32
+// queries). A one-wave kernel runs one 256-row block per CU
 // at a time and gains nothing when a CU is left alone, so it is taken when
 // its grid fills whole rounds of the resident workgroups (or at least six),
 // and the compiled kernel, whose second workgroup per CU runs faster alone,
@@ -438,8 +432,13 @@ bwd_k_kernel(BwdParams<T> p, int chunk) {
 // (192 workgroups) 52.4 / 46.5, B1 N4096 H12 (768) 184 / 166, B2 N4096 H16 over
 // 4 key heads (512) 523 / 446, but B2 N2048 H16 (1024) 101 / 108; non-causal
 // B1 N2048 H16 (512) 95.2 / 92.9, but B2 N2048 H12 (768) 121 / 142.
-// FLASH_HOG_BWD (dK/dV) = compiled, k64 or pair and FLASH_HOG_BWDQ (dQ) =
-// compiled or q64 force a kernel; read at every launch.
+// The dQ pair kernel gains less and is taken, at D = 64 and 128, up to one
+// workgroup per CU (first backward, us, compiled / pair: B1 N512 H12 D64 27.0 /
+// 26.1, B1 N2048 H8 D128 non-causal 118 / 109; B2 N1000 H12 D64 fp16, 384
+// workgroups, 51.2 / 55.7).
+// FLASH_HOG_BWD (dK/dV, D = 64) = compiled, k64 or pair and FLASH_HOG_BWDQ (dQ,
+// D = 64 and 128) = compiled, q64 (D = 64) or pair force a kernel; read at
+// every launch.
 inline bool one_wave_grid(int workgroups, int resident) {
   return resident > 0 && workgroups > 0 && (workgroups % resident == 0 || workgroups >= 6 * resident);
 }
@@ -457,36 +456,51 @@ inline bool pair_selected(int nk, int npairs, bool causal) {
   if (v != nullptr && (std::strcmp(v, "compiled") == 0 || std::strcmp(v, "k64") == 0)) return false;
   return (long)((nk + 63) / 64) * npairs <= (long)(causal ? 3 : 2) * resident_workgroups(1);
 }
+inline bool qpair_selected(int nq, int npairs) {
+  const char* v = std::getenv("FLASH_HOG_BWDQ");
+  if (v != nullptr && std::strcmp(v, "pair") == 0) return true;
+  if (v != nullptr && (std::strcmp(v, "compiled") == 0 || std::strcmp(v, "q64") == 0)) return false;
+  return (long)((nq + 63) / 64) * npairs <= resident_workgroups(1);
+}
 
 template <typename T, int D, bool CAUSAL>
-hipError_t launch_bwd(const BwdParams<T>& p, hipStream_t stream) {
-  const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
-  const int resident = resident_workgroups(Occupancy<T, D>::value);
-  const int nq_pairs = p.batch * p.heads, nk_pairs = p.batch * p.kv_heads;
-  hipError_t e = hipSuccess;
-  if constexpr (sizeof(T) == 2 && D == 64) {
-    if (one_wave_selected("FLASH_HOG_BWDQ", "q64", (p.nq + 255) / 256, nq_pairs, CAUSAL))
-      e = launch_bwd_q64<T, CAUSAL>(p, stream);
-    else
-      hipLaunchKernelGGL((bwd_q_kernel<T, D, CAUSAL>), dim3(nqb * nq_pairs), dim3(kThreads), 0, stream, p,
-                         grid_chunk(nq_pairs, nqb, resident));
-  } else {
-    hipLaunchKernelGGL((bwd_q_kernel<T, D, CAUSAL>), dim3(nqb * nq_pairs), dim3(kThreads), 0, stream, p,
-                       grid_chunk(nq_pairs, nqb, resident));
+hipError_t launch_bwd_dq(const BwdParams<T>& p, hipStream_t stream) {
+  if constexpr (sizeof(T) == 2 && D <= 128) {
+    const int npairs = p.batch * p.heads;
+    if (!qpair_selected(p.nq, npairs)) {
+      if constexpr (D == 64) {
+        if (one_wave_selected("FLASH_HOG_BWDQ", "q64", (p.nq + 255) / 256, npairs, CAUSAL))
+          return launch_bwd_q64<T, CAUSAL>(p, stream);
+      }
+      const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
+      hipLaunchKernelGGL((bwd_q_kernel<T, D, CAUSAL>), dim3(nqb * npairs), dim3(kThreads), 0, stream, p,
+                         grid_chunk(npairs, nqb, resident_workgroups(kOcc)));
+      return hipGetLastError();
+    }
   }
-  if (e == hipSuccess) e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  return launch_bwd_qpair<T, D, CAUSAL>(p, stream);
+}
+
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_bwd_dkdv(const BwdParams<T>& p, hipStream_t stream) {
   if constexpr (sizeof(T) == 2 && D == 64) {
-    if (!pair_selected(p.nk, nk_pairs, CAUSAL)) {
-      if (one_wave_selected("FLASH_HOG_BWD", "k64", (p.nk + 255) / 256, nk_pairs, CAUSAL))
+    const int npairs = p.batch * p.kv_heads;
+    if (!pair_selected(p.nk, npairs, CAUSAL)) {
+      if (one_wave_selected("FLASH_HOG_BWD", "k64", (p.nk + 255) / 256, npairs, CAUSAL))
         return launch_bwd_k64<T, CAUSAL>(p, stream);
       const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
-      hipLaunchKernelGGL((bwd_k_kernel<T, D, CAUSAL>), dim3(nkb * nk_pairs), dim3(kThreads), 0, stream, p,
-                         grid_chunk(nk_pairs, nkb, resident));
+      hipLaunchKernelGGL((bwd_k_kernel<T, D, CAUSAL>), dim3(nkb * npairs), dim3(kThreads), 0, stream, p,
+                         grid_chunk(npairs, nkb, resident_workgroups(kOcc)));
       return hipGetLastError();
     }
   }
   return launch_bwd_pair<T, D, CAUSAL>(p, stream);
+}
+
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_bwd(const BwdParams<T>& p, hipStream_t stream) {
+  const hipError_t e = launch_bwd_dq<T, D, CAUSAL>(p, stream);
+  return e != hipSuccess ? e : launch_bwd_dkdv<T, D, CAUSAL>(p, stream);
 }
 
 #define FHOG_INST(T, D, C) template hipError_t launch_bwd<T, D, C>(const BwdParams<T>&, hipStream_t);

@@ -81,6 +81,10 @@ hipError_t launch_bwd_k64(const BwdParams<T>& p, hipStream_t s);
 // (2-byte types, D = 64); launch_bwd selects it for grids of whole rounds.
 template <typename T, bool CAUSAL>
 hipError_t launch_bwd_q64(const BwdParams<T>& p, hipStream_t s);
+// dQ and D of the first backward with two waves per 32 queries (all types and
+// head dims; launch_bwd selects it but for 2-byte D = 64 and 128 on larger grids).
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_bwd_qpair(const BwdParams<T>& p, hipStream_t s);
 // dK and dV of the first backward with two waves per 32 keys (all types and
 // head dims; at 2-byte D = 64 launch_bwd selects it for small grids).
 template <typename T, int D, bool CAUSAL>

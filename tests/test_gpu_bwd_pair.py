@@ -1,14 +1,16 @@
-"""The first backward's dK/dV kernel with two waves per 32 keys (fhog_bwd_pair.hip).
+"""The first backward's kernels with two waves per 32 rows: dK/dV per 32 keys
+(fhog_bwd_pair.h) and dQ per 32 queries (fhog_bwd_qpair.hip).
 
-It serves fp32 and 2-byte head dims 128 and 256 always, and 2-byte D = 64 on
-small grids or with FLASH_HOG_BWD=pair. Sizes are where it can go wrong: one
-row, one tile and its neighbours, a ragged last tile on either side, key
-blocks of 64 that are half empty or see no query, grouped heads, and each of
-its three schedules on grids below, at and above the sizes where the launch
-folds the block order (257 to 512 workgroups on 256 CUs) and switches
-schedule (over 1024). Against the closed form in fp64;
-tolerances are those of tests/helpers.py (fp32 products here sum at most
-1300 terms). At D = 64 it must give bwd_k_kernel's bits.
+The first serves fp32 and 2-byte head dims 128 and 256 always, and 2-byte
+D = 64 on small grids or with FLASH_HOG_BWD=pair; the second fp32 and head dim
+256 always, and 2-byte 64 and 128 on small grids or with FLASH_HOG_BWDQ=pair.
+Sizes are where they can go wrong: one row, one tile and its neighbours, a
+ragged last tile on either side, blocks of 64 that are half empty or see
+nothing, grouped heads, and grids above the sizes where the launch folds the
+block order (257 to 512 workgroups on 256 CUs) and takes three workgroups per
+CU (over 1024). Against the closed form in fp64 at the tolerances of
+tests/helpers.py (fp32 products here sum at most 1300 terms). They must give
+the bits of bwd_k_kernel (D = 64) and bwd_q_kernel (2-byte D = 64 and 128).
 """
 
 from __future__ import annotations
@@ -68,14 +70,15 @@ def test_bwd_pair(shape, dtype, D, cuda_device, monkeypatch):
                 probs[b, h] = p
     args = (x["q"], x["k"], x["v"], o, x["do"], lse, causal, scale)
     monkeypatch.setenv("FLASH_HOG_BWD", "pair")
+    monkeypatch.setenv("FLASH_HOG_BWDQ", "pair")
     got = _hip.attention_bwd(*args)
     torch.cuda.synchronize()
-    if D == 64 and dtype is not torch.float32:
+    if D <= 128 and dtype is not torch.float32:
         monkeypatch.setenv("FLASH_HOG_BWD", "compiled")
+        monkeypatch.setenv("FLASH_HOG_BWDQ", "compiled")
         want = _hip.attention_bwd(*args)
         for a, r, label in zip(got, want, ("dq", "dk", "dv", "D")):
             assert torch.equal(a, r), label
-        return
     grp = H // Hk
     for b in sorted({0, B - 1}):
         for hk in range(Hk):
@@ -84,6 +87,9 @@ def test_bwd_pair(shape, dtype, D, cuda_device, monkeypatch):
                 p, do = probs[b, h], f(x["do"], b, h)
                 d = (f(o, b, h) * do).sum(-1, keepdim=True)
                 ds = scale * p * (do @ f(x["v"], b, hk).t().contiguous() - d)
+                for a, r, label in ((got[0][b, :, h], ds @ f(x["k"], b, hk), "dq"), (got[3][b, h], d[:, 0], "D")):
+                    err = rel_err(a, r, DEGENERATE_FLOOR)
+                    assert err < TOL[dtype], f"{label} batch {b} head {h}: {err:.2e}"
                 dk = dk + ds.t().contiguous() @ f(x["q"], b, h)
                 dv = dv + p.t().contiguous() @ do
             for a, r, label in ((got[1], dk, "dk"), (got[2], dv, "dv")):
