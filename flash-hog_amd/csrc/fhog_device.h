@@ -181,34 +181,6 @@ __device__ __forceinline__ uint32_t lds_base_u32(const void* p) {
   return __builtin_amdgcn_readfirstlane(lds_addr(p));
 }
 
-// fp32 operands read from a swizzled tile (4-byte elements, 16-byte chunks of
-// 4): frag_row_swz contracts over columns (lane (n, g) gets row n, columns
-// 16 ks + 8 g .. +7), frag_tr_swz over the 32 tile rows in the permuted order
-// of a C tile fed back as an operand (lane l gets column dbase + (l & 31), rows
-// 16 s + 8 (e / 4) + 4 g + e % 4).
-template <typename T, int D>
-__device__ __forceinline__ V8<T> frag_row_swz(const T* tile, int n, int g, int ks) {
-  static_assert(sizeof(T) == 4, "2-byte types use SwzFrags' LDS reads");
-  const T* row = tile + n * D;
-  const V4<T> a = *reinterpret_cast<const V4<T>*>(row + 4 * phys_chunk(n, 4 * ks + 2 * g));
-  const V4<T> b = *reinterpret_cast<const V4<T>*>(row + 4 * phys_chunk(n, 4 * ks + 2 * g + 1));
-  return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
-template <typename T, int D>
-__device__ __forceinline__ V8<T> frag_tr_swz(const T* tile, int dbase, int lane, int s) {
-  static_assert(sizeof(T) == 4, "2-byte types use SwzFrags' LDS reads");
-  const int g = lane >> 5;
-  const int col = dbase + (lane & 31);
-  V8<T> v;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int row = 16 * s + 8 * (e >> 2) + 4 * g + (e & 3);
-    v[e] = tile[row * D + 4 * phys_chunk(row, col >> 2) + (col & 3)];
-  }
-  return v;
-}
-
 // Wait until this wave's outstanding vector-memory operations (including
 // global_load_lds) have completed; lgkm and exp counters are left alone.
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
@@ -344,13 +316,17 @@ template <typename T, int D, int COUNT = SwzTile<T, D>::kLoads, int SWZ = kSwzPa
 // aligned groups of eight (128 bytes, 64 columns), so the offsets of the first 64
 // columns serve the others with a constant: six registers whatever D, where
 // offsets for every column block took 12 at D = 128 and 24 at D = 256.
+//
+// fp32 (eight chunks are 32 columns): a row operand is two 16-byte reads, chunks
+// c = 4 ks + 2 g and c ^ 1; a transposed one eight 4-byte reads of rows
+// 16 s + 8 (e / 4) + 4 g + e % 4, whose keys are 4 ((e % 4) / 2) + 2 g + e / 4: one
+// offset for each of the four values that e gives, the rest constant.
 template <typename T, int D> struct SwzFrags {
-  uint32_t row[4];  // row operand of steps ks = 0..3 (columns 0..63)
-  uint32_t tr[2];   // first transposed read of column blocks dt = 0, 1, step 0 (rows 4 g + i / 4)
-  int lane;
+  uint32_t row[4];  // 2-byte: row operand of steps ks = 0..3 (columns 0..63); fp32: ks = 0, 1, two chunks each
+  uint32_t tr[sizeof(T) == 2 ? 2 : 4];  // 2-byte: first transposed read of column blocks dt = 0, 1, step 0 (rows
+                                        // 4 g + i / 4); fp32: rows 4 g of step 0, one for each key that e gives
 
-  __device__ __forceinline__ void init(int lane_id) {
-    lane = lane_id;
+  __device__ __forceinline__ void init(int lane) {
     if constexpr (sizeof(T) == 2) {
       const int n = lane & 31, g = lane >> 5;
 #pragma unroll
@@ -363,6 +339,14 @@ template <typename T, int D> struct SwzFrags {
         const int d = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (i & 3);
         tr[dt] = 2u * (uint32_t)(r * D + 8 * phys_chunk(r, d >> 3) + (d & 7));
       }
+    } else {
+      const int n = lane & 31, g = lane >> 5;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        row[i] = 4u * (uint32_t)(n * D + 4 * phys_chunk(n, 4 * (i >> 1) + 2 * g + (i & 1)));
+        const int key = 2 * g + 4 * (i >> 1) + (i & 1);
+        tr[i] = 4u * (uint32_t)(4 * g * D + 4 * ((n >> 2) ^ key) + (n & 3));
+      }
     }
   }
 
@@ -372,7 +356,11 @@ template <typename T, int D> struct SwzFrags {
       const lds_cchar* p = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[ks & 3]));
       return *reinterpret_cast<const __attribute__((address_space(3))) V8<T>*>(p + off + 128 * (ks >> 2));
     } else {
-      return frag_row_swz<T, D>(tile_ptr(stage, off), lane & 31, lane >> 5, ks);
+      typedef const __attribute__((address_space(3))) V4<T>* ptr;
+      const int o = off + 128 * (ks >> 1);
+      const V4<T> a = *(ptr)(reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[2 * (ks & 1)])) + o);
+      const V4<T> b = *(ptr)(reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[2 * (ks & 1) + 1])) + o);
+      return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
     }
   }
 
@@ -397,14 +385,15 @@ template <typename T, int D> struct SwzFrags {
       return __builtin_shufflevector(__builtin_bit_cast(V4<T>, x), __builtin_bit_cast(V4<T>, y), 0, 1, 2, 3, 4, 5,
                                      6, 7);
     } else {
-      return frag_tr_swz<T, D>(tile_ptr(stage, off), 32 * dt, lane, s);
+      V8<T> v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t a = stage + tr[2 * ((e & 3) >> 1) + (e >> 2)];
+        const int o = off + 128 * dt + (16 * s + 8 * (e >> 2) + (e & 3)) * 4 * D;
+        v[e] = *(const __attribute__((address_space(3))) T*)(reinterpret_cast<const lds_cchar*>((uintptr_t)a) + o);
+      }
+      return v;
     }
-  }
-
- private:
-  __device__ __forceinline__ static const T* tile_ptr(uint32_t stage, int off) {
-    // an address-space conversion, which only a C-style cast expresses
-    return (const T*)((const lds_cchar*)(uintptr_t)stage + off);
   }
 };
 
