@@ -5,13 +5,16 @@
 // natural log, of the scaled and masked logits).
 //
 // A workgroup owns 128 queries (4 waves x 32) of one (batch, head) and streams
-// 32-key tiles of K and V global -> LDS (no registers) through a 4-stage ring
+// 32-key tiles of K and V global -> LDS (no registers) through a ring
 // of XOR-swizzled tiles, one barrier per tile; wave w loads half (w % 2) of
 // tensor w / 2. Scores are computed transposed (S^T = K Q^T) and the output
 // as O^T = V^T P^T, so every lane holds one query row in both: the online-
 // softmax rescale is a per-lane scalar multiply, skipped when no row of the
 // wave raised its running maximum. Causal blocks are issued longest first with
 // (batch, head) as the minor index (see fhog_bwdbwd.hip).
+#include <cstdlib>
+#include <cstring>
+
 #include "fhog_device.h"
 #include "fhog_params.h"
 
@@ -21,15 +24,19 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
-constexpr int kStages = 4;  // 3 stages: 0.5-1 % slower
 
-// Waves per SIMD the register allocator is asked to allow: three for 2-byte
-// types at D = 64 (119 VGPRs; 50.7 against 55.4 us at two waves, B4 N2048 H16
-// causal, and four waves are no faster), two at D = 128 (190 VGPRs, no spill;
-// 147.7 against 86.3 us at one wave, B4 N2048 H16 causal) and for fp32 at
-// D = 64 (154 VGPRs; 167 against 154 us at B2 N2048 H8), one otherwise.
+// Waves per SIMD the register allocator is asked to allow: three at D = 64
+// (2-byte: 127 VGPRs, 50.7 against 55.4 us at two waves, B4 N2048 H16 causal, and
+// four are no faster; fp32: 160 VGPRs, 297 -> 287 us at B4 N2048 H16 causal with
+// the ring of three stages that leaves room for a third workgroup), two at D = 128
+// (204 VGPRs; 147.7 against 86.3 us at one wave, B4 N2048 H16 causal), one for
+// fp32 at D = 128. (2-byte D = 256 runs fwd_pair_kernel, fhog_fwd_pair.hip.)
 template <typename T, int D> struct Occupancy {
-  static constexpr int value = sizeof(T) != 2 ? (D == 64 ? 2 : 1) : D == 64 ? 3 : D == 128 ? 2 : 1;
+  static constexpr int value = D == 64 ? 3 : sizeof(T) == 2 ? 2 : 1;
+};
+// Stages of the LDS ring (2-byte types, three: 0.5-1 % slower).
+template <typename T, int D> struct Stages {
+  static constexpr int value = sizeof(T) == 4 && D == 64 ? 3 : 4;
 };
 
 template <typename T, int D, bool CAUSAL>
@@ -41,7 +48,7 @@ fwd_kernel(FwdParams<T> p, int chunk) {
   constexpr int DT = D / 32;
   constexpr int BQ = 32 * kWaves;
   constexpr int BK = 32;
-  constexpr int NST = kStages;
+  constexpr int NST = Stages<T, D>::value;
   constexpr int kTile = G::kElems * (int)sizeof(T);
   constexpr int kStage = 2 * kTile;  // K, V
   constexpr int kPer = G::kLoads / 2;
@@ -132,8 +139,20 @@ fwd_kernel(FwdParams<T> p, int chunk) {
     if (kt < wkt) {
       const uint32_t sa = lds_kv + (uint32_t)(((uint32_t)kt % NST) * kStage);  // K at 0, V at kTile
       f32x16 S = zero16();
+      if constexpr (sizeof(T) == 2) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) S = mma<T>(fr.rowf(sa, 0, ks), qf[ks], S);
+        for (int ks = 0; ks < KS; ++ks) S = mma<T>(fr.rowf(sa, 0, ks), qf[ks], S);
+      } else {
+        // the two halves of the contraction apart, as fwd_pair_kernel's two waves
+        // form them, so that the two kernels give the same bits
+        f32x16 S1 = zero16();
+#pragma unroll
+        for (int ks = 0; ks < KS / 2; ++ks) {
+          S = mma<T>(fr.rowf(sa, 0, ks), qf[ks], S);
+          S1 = mma<T>(fr.rowf(sa, 0, KS / 2 + ks), qf[KS / 2 + ks], S1);
+        }
+        S += S1;
+      }
       // S stays unscaled: the row maximum is taken on it and scaled once
       // (c2 > 0, and rounding is monotonic, so this equals the maximum of the
       // scaled values), and the scale enters the exponent's fma below.
@@ -208,13 +227,34 @@ fwd_kernel(FwdParams<T> p, int chunk) {
 
 }  // namespace
 
+// fwd_pair_kernel (two waves per 32 queries, 64-query workgroups) serves 2-byte
+// types at D = 256, and fp32 while its grid has at most one workgroup per CU, or
+// four (D = 64) or three (D = 128) when causal; fp32's two kernels give the same
+// bits (us, fwd / pair: causal N2048 H8 D64 B2 (512 workgroups) 142 / 99, B4
+// (1024) 196 / 165, B4 H16 (2048) 287 / 312; non-causal B1 (256) 142 / 97, B2
+// (512) 144 / 157; D128 causal B3 (768) 273 / 237, B4 (1024) 300 / 309).
+// FLASH_HOG_FWD = compiled or pair forces either for fp32; read at every launch.
+inline bool fwd_pair_selected(int nq, int npairs, int head_dim, bool causal) {
+  const char* v = std::getenv("FLASH_HOG_FWD");
+  if (v != nullptr && std::strcmp(v, "pair") == 0) return true;
+  if (v != nullptr && std::strcmp(v, "compiled") == 0) return false;
+  return (long)((nq + 63) / 64) * npairs <= (long)(!causal ? 1 : head_dim == 64 ? 4 : 3) * resident_workgroups(1);
+}
+
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_fwd(const FwdParams<T>& p, hipStream_t stream) {
-  const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
-  const int npairs = p.batch * p.heads;
-  const int chunk = grid_chunk(npairs, nqb, resident_workgroups(Occupancy<T, D>::value));
-  hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL>), dim3(nqb * npairs), dim3(kThreads), 0, stream, p, chunk);
-  return hipGetLastError();
+  if constexpr (sizeof(T) == 2 && D == 256) {
+    return launch_fwd_pair<T, D, CAUSAL>(p, stream);
+  } else {
+    const int npairs = p.batch * p.heads;
+    if constexpr (sizeof(T) == 4) {
+      if (fwd_pair_selected(p.nq, npairs, D, CAUSAL)) return launch_fwd_pair<T, D, CAUSAL>(p, stream);
+    }
+    const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
+    const int chunk = grid_chunk(npairs, nqb, resident_workgroups(Occupancy<T, D>::value));
+    hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL>), dim3(nqb * npairs), dim3(kThreads), 0, stream, p, chunk);
+    return hipGetLastError();
+  }
 }
 
 #define FHOG_INST(T, D, C) template hipError_t launch_fwd<T, D, C>(const FwdParams<T>&, hipStream_t);

@@ -58,6 +58,9 @@ __device__ inline int first_contributing_query(const BwdBwdParams<T>& p, int kj,
 }
 
 template <typename T, int D, bool CAUSAL> hipError_t launch_fwd(const FwdParams<T>& p, hipStream_t s);
+// The forward with two waves per 32 queries: 2-byte types at D = 256, and fp32 on
+// small grids; launch_fwd selects it.
+template <typename T, int D, bool CAUSAL> hipError_t launch_fwd_pair(const FwdParams<T>& p, hipStream_t s);
 template <typename T, int D, bool CAUSAL> hipError_t launch_bwd(const BwdParams<T>& p, hipStream_t s);
 // stages: bit 0 = stage 1 (passes 1-3), bit 1 = stage 2 (pass 4).
 template <typename T, int D, bool CAUSAL>
