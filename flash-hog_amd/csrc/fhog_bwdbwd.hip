@@ -66,7 +66,7 @@ template <typename T, int D> struct Ring {
 };
 
 // ----------------------------------------------------------------------------
-// Stage 1: passes 1-3, tiled over queries.
+// Stage 1: passes 1-3, tiled over queries, for fp32.
 //
 // Sweep 1 (passes 1+2) computes S, ddS, dP and, per row, dD = sum ddS P,
 // r2 = sum dP P, r3 = sum dP ddS P, and accumulates P ddV into the ddO
@@ -651,6 +651,22 @@ inline bool stage1_fused_selected() {
   return v != nullptr && std::strcmp(v, "fused") == 0;
 }
 
+// Stage 1 for fp32 runs bwdbwd_q_kernel below (one wave per 32 queries) on grids
+// that fill the chip and bwdbwd_qpair_kernel (fhog_bwdbwd_qpair.hip, two waves per
+// 32 queries, half the time per block and twice the workgroups) on smaller ones;
+// both give the same bits. The line is two of the latter's workgroups per CU
+// when causal, one otherwise (stage 1, us, q / qpair: causal D = 64 N2048 H8 B2
+// (512 workgroups) 887 / 631, B3 (768) 890 / 840-885, B4 (1024) 970 / 1093;
+// non-causal B1 (256) 902 / 626, B2 (512) 910 / 1021; D = 128 causal B2 (512)
+// 1620 / 1296, B4 (1024) 1783 / 2538, non-causal B1 (256) 1647 / 1255). FLASH_HOG_STAGE1 = compiled or pair forces
+// either for fp32. Read at every launch.
+inline bool stage1_qpair_selected(int nq, int npairs, bool causal) {
+  const char* v = std::getenv("FLASH_HOG_STAGE1");
+  if (v != nullptr && std::strcmp(v, "pair") == 0) return true;
+  if (v != nullptr && std::strcmp(v, "compiled") == 0) return false;
+  return (long)((nq + 63) / 64) * npairs <= (long)(causal ? 2 : 1) * resident_workgroups(1);
+}
+
 // Stage 2 runs bwdbwd_pair_kernel (fhog_bwdbwd_pair.hip, two waves per 32 keys)
 // but for 2-byte types at D = 64 on grids that fill the chip, where
 // bwdbwd_k_kernel's one wave per 32 keys is faster; both give the same bits.
@@ -674,7 +690,6 @@ inline bool stage2_pair_selected(const char* v, int nk, int npairs, bool causal)
 
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stages) {
-  const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
   if (stages & 1) {
     hipError_t e;
     if constexpr (sizeof(T) == 2 && D == 64) {
@@ -682,7 +697,10 @@ hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stage
                                   : launch_bwdbwd_stage1_q32<T, CAUSAL>(p, stream);
     } else if constexpr (sizeof(T) == 2) {
       e = launch_bwdbwd_stage1_fused<T, D, CAUSAL>(p, stream);
+    } else if (stage1_qpair_selected(p.nq, p.batch * p.heads, CAUSAL)) {
+      e = launch_bwdbwd_stage1_qpair<D, CAUSAL>(p, stream);
     } else {
+      const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
       const int npairs = p.batch * p.heads;
       hipLaunchKernelGGL((bwdbwd_q_kernel<T, D, CAUSAL>), dim3(nqb * npairs), dim3(kThreads), 0, stream, p,
                          grid_chunk(npairs, nqb, resident_workgroups(Occupancy<T, D>::value)));

@@ -92,6 +92,10 @@ hipError_t launch_bwd_qpair(const BwdParams<T>& p, hipStream_t s);
 // head dims; at 2-byte D = 64 launch_bwd selects it for small grids).
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd_pair(const BwdParams<T>& p, hipStream_t s);
+// Stage 1 for fp32 with two waves per 32 queries; launch_bwdbwd selects it for
+// small grids.
+template <int D, bool CAUSAL>
+hipError_t launch_bwdbwd_stage1_qpair(const BwdBwdParams<float>& p, hipStream_t s);
 // Stage 2 with two waves per 32 keys (all types and head dims; at 2-byte
 // D = 64 launch_bwdbwd selects it for small grids).
 template <typename T, int D, bool CAUSAL>
