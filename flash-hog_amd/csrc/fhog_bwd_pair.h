@@ -286,12 +286,18 @@ hipError_t launch_bwd_pair(const BwdParams<T>& p, hipStream_t stream) {
   // (D = 64 B4 N2048 H16 1031 -> 1013 us, B2 N2048 H8 equal), for 2-byte D = 128
   // once the grid is long (two / three: 359 / 392 us at B2 N2048 H32 over 8 key
   // heads, 512 workgroups; 300 / 287 at B4 N2048 H16, 2048; 2040 / 1956 at B2
-  // N8192 H16, 4096).
+  // N8192 H16, 4096). 2-byte D = 64 likewise with four (117 registers; first
+  // backward, two / four: causal B1 N4096 H12, 768 workgroups, 163 / 166, B2 N2048
+  // H16, 1024, 105 / 99, B128 N512 H12 484 / 417; non-causal B2 N2048 H12, 768,
+  // 146 / 117).
   if constexpr (sizeof(T) == 4 && D == 64) {
     return launch_occ<T, D, CAUSAL, 3>(p, nkb, npairs, cus, stream);
   } else {
     if constexpr (sizeof(T) == 2 && D == 128) {
       if ((long)nkb * npairs > 4L * cus) return launch_occ<T, D, CAUSAL, 3>(p, nkb, npairs, cus, stream);
+    }
+    if constexpr (sizeof(T) == 2 && D == 64) {
+      if ((long)nkb * npairs > (CAUSAL ? 3L : 2L) * cus) return launch_occ<T, D, CAUSAL, 4>(p, nkb, npairs, cus, stream);
     }
     return launch_occ<T, D, CAUSAL, 2>(p, nkb, npairs, cus, stream);
   }

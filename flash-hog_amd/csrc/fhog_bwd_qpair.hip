@@ -28,10 +28,13 @@ namespace {
 constexpr int kPairs = 2;
 constexpr int kWaves = 2 * kPairs;
 constexpr int kThreads = 64 * kWaves;
-constexpr int kOcc = 2;  // waves per SIMD
+// At least this many waves per SIMD; the narrower instances' registers allow
+// three or four (a bound of two: 430 -> 481 us for the first backward at B128 N512
+// H12 D64 causal).
+constexpr int kOcc = 2;
 template <typename T, int D, bool CAUSAL>
 __global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(kOcc, kOcc)))
+__attribute__((amdgpu_waves_per_eu(kOcc, 8)))
 bwd_qpair_kernel(BwdParams<T> p, int chunk, int fold) {
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 16;
