@@ -38,7 +38,7 @@ constexpr int kOcc = 2;
 template <typename T, int D, bool CAUSAL>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(kOcc, kOcc)))
-bwd_q_kernel(BwdParams<T> p, int chunk) {
+bwd_q_kernel(BwdParams<T> p, int chunk, int fold) {
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 16;
   constexpr int DT = D / 32;
@@ -57,7 +57,10 @@ bwd_q_kernel(BwdParams<T> p, int chunk) {
   const int nbh = p.batch * p.heads;
   const GridSlot gs = grid_slot(blockIdx.x, nbh, nqb, chunk);
   const int bh = gs.pair;
-  const int qb = CAUSAL ? nqb - 1 - gs.rank : gs.rank;  // causal: the longest query rows first
+  // causal: the longest query rows first, up to rank `fold`; the ranks from
+  // there on run backwards (fold_rank; first backward of D = 128 B1 N4096 H16 over
+  // 4 key heads 589 -> 574 us)
+  const int qb = CAUSAL ? nqb - 1 - folded(gs.rank, nqb, fold) : gs.rank;
   const int b = bh / p.heads, h = bh % p.heads;
   const int hk = h / (p.heads / p.kv_heads);
   const long rs = (long)p.heads * D;      // query-side row stride
@@ -488,7 +491,8 @@ hipError_t launch_bwd_dq(const BwdParams<T>& p, hipStream_t stream) {
       }
       const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
       hipLaunchKernelGGL((bwd_q_kernel<T, D, CAUSAL>), dim3(nqb * npairs), dim3(kThreads), 0, stream, p,
-                         grid_chunk(npairs, nqb, resident_workgroups(kOcc)));
+                         grid_chunk(npairs, nqb, resident_workgroups(kOcc)),
+                         fold_rank(CAUSAL, nqb, npairs, resident_workgroups(1)));
       return hipGetLastError();
     }
   }

@@ -78,7 +78,7 @@ bwdbwd_pair_kernel(BwdBwdParams<T> p, int chunk, int fold) {
   const GridSlot gs = grid_slot(blockIdx.x, nbh, nkb, chunk);
   // causal: the longest key columns come first, up to rank `fold`; the ranks
   // from there on run backwards (fold_rank)
-  const int kb = gs.rank < fold ? gs.rank : nkb - 1 - (gs.rank - fold);
+  const int kb = folded(gs.rank, nkb, fold);
   const int bh = gs.pair;
   const int b = bh / p.kv_heads, hk = bh % p.kv_heads;
   const int grp = p.heads / p.kv_heads;  // query heads per key/value head

@@ -76,7 +76,7 @@ bwdbwd_qpair_kernel(BwdBwdParams<float> p, int chunk, int fold) {
   const GridSlot gs = grid_slot(blockIdx.x, nbh, nqb, chunk);
   // causal: the longest query rows first, up to rank `fold`; the ranks from
   // there on run backwards (fold_rank)
-  const int rank = gs.rank < fold ? gs.rank : nqb - 1 - (gs.rank - fold);
+  const int rank = folded(gs.rank, nqb, fold);
   const int qb = CAUSAL ? nqb - 1 - rank : rank;
   const int bh = gs.pair;
   const int b = bh / p.heads, h = bh % p.heads;

@@ -315,27 +315,29 @@ template <typename T, int D, int COUNT = SwzTile<T, D>::kLoads, int SWZ = kSwzPa
 // the loop when registers are scarce. The swizzle permutes chunks within
 // aligned groups of eight (128 bytes, 64 columns), so the offsets of the first 64
 // columns serve the others with a constant: six registers whatever D, where
-// offsets for every column block took 12 at D = 128 and 24 at D = 256.
+// offsets for every column block take 12 at D = 128 and 24 at D = 256 (COLS: how
+// many columns have offsets of their own).
 //
 // fp32 (eight chunks are 32 columns): a row operand is two 16-byte reads, chunks
 // c = 4 ks + 2 g and c ^ 1; a transposed one eight 4-byte reads of rows
 // 16 s + 8 (e / 4) + 4 g + e % 4, whose keys are 4 ((e % 4) / 2) + 2 g + e / 4: one
 // offset for each of the four values that e gives, the rest constant.
-template <typename T, int D> struct SwzFrags {
-  uint32_t row[4];  // 2-byte: row operand of steps ks = 0..3 (columns 0..63); fp32: ks = 0, 1, two chunks each
-  uint32_t tr[sizeof(T) == 2 ? 2 : 4];  // 2-byte: first transposed read of column blocks dt = 0, 1, step 0 (rows
-                                        // 4 g + i / 4); fp32: rows 4 g of step 0, one for each key that e gives
+template <typename T, int D, int COLS = 64> struct SwzFrags {
+  static constexpr int kRow = sizeof(T) == 2 ? COLS / 16 : 4, kTr = sizeof(T) == 2 ? COLS / 32 : 4;
+  uint32_t row[kRow];  // 2-byte: row operand of the first steps ks; fp32: ks = 0, 1, two chunks each
+  uint32_t tr[kTr];    // 2-byte: first transposed read of the first column blocks dt, step 0 (rows 4 g + i / 4);
+                       // fp32: rows 4 g of step 0, one for each key that e gives
 
   __device__ __forceinline__ void init(int lane) {
     if constexpr (sizeof(T) == 2) {
       const int n = lane & 31, g = lane >> 5;
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
+      for (int ks = 0; ks < kRow; ++ks)
         row[ks] = 2u * (uint32_t)(n * D + 8 * phys_chunk(n, 2 * ks + g));
       const int i = lane & 15;
       const int r = 4 * g + (i >> 2);
 #pragma unroll
-      for (int dt = 0; dt < 2; ++dt) {
+      for (int dt = 0; dt < kTr; ++dt) {
         const int d = 32 * dt + 16 * ((lane >> 4) & 1) + 4 * (i & 3);
         tr[dt] = 2u * (uint32_t)(r * D + 8 * phys_chunk(r, d >> 3) + (d & 7));
       }
@@ -353,8 +355,8 @@ template <typename T, int D> struct SwzFrags {
   // Operand contracting over columns: lane (n, g) gets row n, columns 16 ks + 8 g .. +7.
   __device__ __forceinline__ V8<T> rowf(uint32_t stage, int off, int ks) const {
     if constexpr (sizeof(T) == 2) {
-      const lds_cchar* p = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[ks & 3]));
-      return *reinterpret_cast<const __attribute__((address_space(3))) V8<T>*>(p + off + 128 * (ks >> 2));
+      const lds_cchar* p = reinterpret_cast<const lds_cchar*>((uintptr_t)(stage + row[ks % kRow]));
+      return *reinterpret_cast<const __attribute__((address_space(3))) V8<T>*>(p + off + 2 * COLS * (ks / kRow));
     } else {
       typedef const __attribute__((address_space(3))) V4<T>* ptr;
       const int o = off + 128 * (ks >> 1);
@@ -376,8 +378,8 @@ template <typename T, int D> struct SwzFrags {
   // be a multiple of 32, which every ring stage and tile offset here is.
   __device__ __forceinline__ V8<T> trf(uint32_t stage, int off, int dt, int s) const {
     if constexpr (sizeof(T) == 2) {
-      const uint32_t a0 = stage + tr[dt & 1];
-      const int o = off + 128 * (dt >> 1) + s * 32 * D;
+      const uint32_t a0 = stage + tr[dt % kTr];
+      const int o = off + 2 * COLS * (dt / kTr) + s * 32 * D;
       const lds_cchar* a = reinterpret_cast<const lds_cchar*>((uintptr_t)a0) + o;
       const lds_cchar* b = reinterpret_cast<const lds_cchar*>((uintptr_t)(a0 ^ 16u)) + o + 16 * D;
       const i16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)(a));
@@ -549,6 +551,7 @@ inline int fold_rank(bool causal, int nb, int npairs, int cus) {
   const long grid = (long)nb * npairs;
   return causal && cus > 0 && grid > cus && grid <= 2L * cus ? (cus + npairs - 1) / npairs : nb;
 }
+__device__ __forceinline__ int folded(int rank, int nb, int fold) { return rank < fold ? rank : nb - 1 - (rank - fold); }
 
 // The `pairs` argument of block_pair for a grid of nb causal blocks per
 // (batch, head) pair: mirror pairs when the unpaired grid outnumbers the
