@@ -53,6 +53,7 @@ HIPCC_FLAGS = [
 _MAX_ILP = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 SOURCE_FLAGS: dict[str, list[str]] = {
     "fhog_bwdbwd_fused.hip": _MAX_ILP,
+    "fhog_bwdbwd_fused_pair.hip": _MAX_ILP,
     "fhog_bwdbwd_q32.hip": _MAX_ILP,
     "fhog_bwdbwd_qpair.hip": _MAX_ILP,
     "fhog_bwdbwd_k32.hip": _MAX_ILP,

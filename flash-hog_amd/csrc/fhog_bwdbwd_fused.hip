@@ -1,7 +1,7 @@
 // Stage 1 of the Flash-HOG double backward (passes 1-3) in one sweep over the
-// keys, for 2-byte types at D = 128 and 256, and at D = 64 when
-// FLASH_HOG_STAGE1=fused selects it over fhog_bwdbwd_q32.hip (fhog_bwdbwd.hip
-// holds the two-sweep stage 1 used for fp32, and stage 2). The math follows
+// keys, for 2-byte types at D = 256 and, for short causal sequences, at D = 64
+// (longer ones: fhog_bwdbwd_q32.hip; D = 128: fhog_bwdbwd_fused_pair.hip; fp32:
+// two sweeps, fhog_bwdbwd.hip and fhog_bwdbwd_qpair.hip). The math follows
 // flash_hog/_jax_refs/jax_impl.py:273-336 and the pass split of
 // flash_hog/jax/_pallas_gpu_kernel.py:149-278; outputs and row statistics are
 // those of fhog_bwdbwd.hip's stage 1.
@@ -48,10 +48,8 @@
 // beside the score tiles in the 256 registers of a wave that shares its SIMD
 // with another, and two co-resident waves are what overlaps one wave's matrix
 // work with the other's vector work. So a wave owns 16 queries and uses the
-// 16x16x32 matrix instruction (v_mfma_f32_16x16x32_{bf16,f16}). At D = 128 this
-// still fits two waves per SIMD when each tile's scores are formed and then
-// finished (no pipelining): 2.78 ms at B2 N8192 H16 against 3.90 ms for the
-// two-sweep stage 1 at one wave per SIMD. Layouts:
+// 16x16x32 matrix instruction (v_mfma_f32_16x16x32_{bf16,f16}). At D = 256 that
+// state still takes a SIMD's 512 registers. Layouts:
 //   A (16 x 32): lane holds A[m = l % 16][k = 8 (l / 16) + e],   e = 0..7
 //   B (32 x 16): lane holds B[k = 8 (l / 16) + e][n = l % 16]
 //   C (16 x 16): lane holds C[m = 4 (l / 16) + i][n = l % 16],   i = 0..3
@@ -84,19 +82,17 @@ struct Scores {
 
 template <typename T, int D, bool CAUSAL, bool PRE>
 __global__ void __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1, D <= 128 ? 2 : 1)))
-bwdbwd_q_fused_kernel(BwdBwdParams<T> p, int chunk) {
+__attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1)))
+bwdbwd_q_fused_kernel(BwdBwdParams<T> p, int chunk, int fold) {
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 32;       // 32-deep steps over the head dim (score products)
   constexpr int DB = D / 16;       // 16-wide output column blocks
   constexpr int BQ = kQ * kWaves;  // queries per workgroup
   constexpr int BK = 32;           // keys per streamed tile
   // D = 64: a software-pipelined loop (the scores of tile t + 1 beside the
-  // element-wise step of tile t) over a 4-stage ring (64 KiB); D = 128: the
-  // accumulators and operands take twice the registers, so each tile's
-  // scores are formed and finished in turn, over a 2-stage ring (64 KiB).
-  // D = 256: the same at one wave per SIMD (512 registers), over a 2-stage
-  // ring of 128 KiB (one workgroup per CU).
+  // element-wise step of tile t) over a 4-stage ring (64 KiB); D = 256: each
+  // tile's scores are formed and finished in turn, at one wave per SIMD (512
+  // registers), over a 2-stage ring of 128 KiB (one workgroup per CU).
   constexpr bool PIPE = D == 64;
   constexpr int NST = PIPE ? 4 : 2;  // tiles t (finishing), t + 1 (scores), two in flight
   constexpr int kTile = G::kElems * (int)sizeof(T);
@@ -110,7 +106,9 @@ bwdbwd_q_fused_kernel(BwdBwdParams<T> p, int chunk) {
   const int nbh = p.batch * p.heads;
   const GridSlot gs = grid_slot(blockIdx.x, nbh, nqb, chunk);
   const int bh = gs.pair;
-  const int qb = CAUSAL ? nqb - 1 - gs.rank : gs.rank;  // causal: the longest query rows first
+  // causal: the longest query rows first, up to rank `fold`; the ranks from
+  // there on run backwards (fold_rank)
+  const int qb = CAUSAL ? nqb - 1 - folded(gs.rank, nqb, fold) : gs.rank;
   const int b = bh / p.heads, h = bh % p.heads;
   const int hk = h / (p.heads / p.kv_heads);
   const long rs = (long)p.heads * D;      // query-side row stride
@@ -388,14 +386,15 @@ template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwdbwd_stage1_fused(const BwdBwdParams<T>& p, hipStream_t stream) {
   const int nqb = (p.nq + kQ * kWaves - 1) / (kQ * kWaves);
   const int npairs = p.batch * p.heads;
-  const int chunk = grid_chunk(npairs, nqb, resident_workgroups(D <= 128 ? 2 : 1));
+  const int chunk = grid_chunk(npairs, nqb, resident_workgroups(D == 64 ? 2 : 1));
+  const int fold = fold_rank(CAUSAL && D == 64, nqb, npairs, resident_workgroups(1));
   const dim3 grid(nqb * npairs);
   int e2;
   if (std::is_same_v<T, __bf16> && std::frexp(p.scale, &e2) == 0.5f)  // scale = 2^(e2 - 1)
     hipLaunchKernelGGL((bwdbwd_q_fused_kernel<T, D, CAUSAL, std::is_same_v<T, __bf16>>), grid, dim3(kThreads), 0,
-                       stream, p, chunk);
+                       stream, p, chunk, fold);
   else
-    hipLaunchKernelGGL((bwdbwd_q_fused_kernel<T, D, CAUSAL, false>), grid, dim3(kThreads), 0, stream, p, chunk);
+    hipLaunchKernelGGL((bwdbwd_q_fused_kernel<T, D, CAUSAL, false>), grid, dim3(kThreads), 0, stream, p, chunk, fold);
   return hipGetLastError();
 }
 
@@ -405,10 +404,6 @@ FHOG_INST(__bf16, 64, true)
 FHOG_INST(__bf16, 64, false)
 FHOG_INST(_Float16, 64, true)
 FHOG_INST(_Float16, 64, false)
-FHOG_INST(__bf16, 128, true)
-FHOG_INST(__bf16, 128, false)
-FHOG_INST(_Float16, 128, true)
-FHOG_INST(_Float16, 128, false)
 FHOG_INST(__bf16, 256, true)
 FHOG_INST(__bf16, 256, false)
 FHOG_INST(_Float16, 256, true)

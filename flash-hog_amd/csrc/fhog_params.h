@@ -65,9 +65,13 @@ template <typename T, int D, bool CAUSAL> hipError_t launch_bwd(const BwdParams<
 // stages: bit 0 = stage 1 (passes 1-3), bit 1 = stage 2 (pass 4).
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t s, int stages = 3);
-// Stage 1 in one sweep (2-byte types, D = 64 and 128); launch_bwdbwd selects it.
+// Stage 1 in one sweep, 16 queries per wave (2-byte types, D = 64 and 256);
+// launch_bwdbwd selects it.
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwdbwd_stage1_fused(const BwdBwdParams<T>& p, hipStream_t s);
+// Stage 1 in one sweep, two waves per 32 queries (2-byte types, D = 128).
+template <typename T, bool CAUSAL>
+hipError_t launch_bwdbwd_stage1_fused_pair(const BwdBwdParams<T>& p, hipStream_t s);
 // Stage 1 with 32 queries per wave at one wave per SIMD (2-byte types, D = 64);
 // launch_bwdbwd selects it.
 template <typename T, bool CAUSAL>
