@@ -640,15 +640,19 @@ bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk) {
 
 // Stage 1 for 2-byte types at D = 64 runs the kernel with 32 queries per
 // wave at one wave per SIMD, a hand-scheduled sweep and a persistent grid
-// (fhog_bwdbwd_q32.hip) unless FLASH_HOG_STAGE1=fused selects the fused
-// kernel (16 queries per wave, two waves per SIMD; one at D = 256, which
-// it serves). Both give the same results to rounding; the q32 kernel is 3-6 % faster
-// on every D = 64 configuration measured (179 against 185 us at B4 N2048 H16
-// causal bf16, 137 against 146 us at B8 N1000 H12 fp16). Read at every launch,
-// so a process can switch between them.
-inline bool stage1_fused_selected() {
+// (fhog_bwdbwd_q32.hip) but for causal sequences of up to 512, which run the fused
+// kernel (16 queries per wave, two waves per SIMD): its 64-query blocks take half
+// as long and waste less of the diagonal. Both give the same results to
+// rounding, so the choice looks at the sequence only, never at how many there are
+// (stage 1, us, q32 / fused: causal N256 H12 B1 21.5 / 11.9, B256 310 / 297; N512
+// B1 28.4 / 18.8, B16 64.7 / 52.6, B64 209 / 209, B128 418 / 425; N1024 B32 316 /
+// 330; non-causal N512 B16 fp16 74.6 / 85.7; B4 N2048 H16 causal 171 / 185).
+// FLASH_HOG_STAGE1 = q32 or fused forces either; read at every launch.
+inline bool stage1_fused_selected(int nq, int nk, bool causal) {
   const char* v = std::getenv("FLASH_HOG_STAGE1");
-  return v != nullptr && std::strcmp(v, "fused") == 0;
+  if (v != nullptr && std::strcmp(v, "fused") == 0) return true;
+  if (v != nullptr && std::strcmp(v, "q32") == 0) return false;
+  return causal && nq <= 512 && nk <= 512;
 }
 
 // Stage 1 for fp32 runs bwdbwd_q_kernel below (one wave per 32 queries) on grids
@@ -693,8 +697,8 @@ hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stage
   if (stages & 1) {
     hipError_t e;
     if constexpr (sizeof(T) == 2 && D == 64) {
-      e = stage1_fused_selected() ? launch_bwdbwd_stage1_fused<T, D, CAUSAL>(p, stream)
-                                  : launch_bwdbwd_stage1_q32<T, CAUSAL>(p, stream);
+      e = stage1_fused_selected(p.nq, p.nk, CAUSAL) ? launch_bwdbwd_stage1_fused<T, D, CAUSAL>(p, stream)
+                                                    : launch_bwdbwd_stage1_q32<T, CAUSAL>(p, stream);
     } else if constexpr (sizeof(T) == 2 && D == 128) {
       e = launch_bwdbwd_stage1_fused_pair<T, CAUSAL>(p, stream);
     } else if constexpr (sizeof(T) == 2) {
