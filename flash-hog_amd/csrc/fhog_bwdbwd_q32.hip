@@ -58,20 +58,27 @@ __device__ __forceinline__ const void* uni(const void* x) {
 
 // A workgroup's share of the grid. The grid is persistent (at most one
 // workgroup per CU, the most that fit at one wave per SIMD) and walks a list
-// of items: with a causal mask item r of a (batch, head) pair is the query
-// block of rank r (nqb - 1 - r, the longest rows first) followed by the block
-// of rank nqb - 1 - r, so every item but a middle one holds the same number
-// of key tiles; without a mask an item is one block. Workgroup w takes items
-// w', w' + G, w' + 2 G, ... where w' numbers the workgroups XCD by XCD (the
-// hardware hands workgroup w to XCD w mod 8), so that the blocks a (batch,
-// head) pair has in flight share one L2.
+// of items. Without a mask an item is one query block. With a causal mask there
+// are two lists (`deal`):
+// - Folded: item r of a (batch, head) pair is the query block of rank r (nqb - 1
+//   - r, the longest rows first) followed by the block of rank nqb - 1 - r, so
+//   every item but a middle one holds the same number of key tiles.
+// - Dealt: the blocks one by one, longest first over all (batch, head) pairs,
+//   every other round of workgroups in reverse, so that whoever had a long block
+//   gets a short one next. A grid that folded items would leave partly idle in
+//   its last (or only) round is balanced to about a block's length.
+// Workgroup w takes folded items and unmasked blocks w', w' + G, w' + 2 G, ...
+// where w' numbers the workgroups XCD by XCD (the hardware hands workgroup w to
+// XCD w mod 8), so that the blocks a (batch, head) pair has in flight share one
+// L2; dealt ones are reversed in groups of eight workgroups, so that an XCD keeps
+// to the same pairs.
 struct Q32Walk {
-  int item, half;
+  int item, half;  // half: second block of a folded item, or the round of a dealt one
 };
 
 template <typename T, bool CAUSAL, bool PRE>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
-bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems) {
+bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems, int deal) {
   constexpr int D = 64;
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 16;       // 16-deep steps over the head dim
@@ -94,7 +101,8 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems) {
   const int npr = CAUSAL ? (nqb + 1) / 2 : nqb;  // items per (batch, head) pair
   const int ngrid = (int)gridDim.x;
   const int w = (int)blockIdx.x;
-  Q32Walk walk{ngrid % 8 == 0 ? (w % 8) * (ngrid / 8) + w / 8 : w, 0};
+  const int npairs = p.batch * p.heads;
+  Q32Walk walk{!(CAUSAL && deal) && ngrid % 8 == 0 ? (w % 8) * (ngrid / 8) + w / 8 : w, 0};
   if (walk.item >= nitems) return;
   const long rs = (long)p.heads * D;      // query-side row stride
   const long rsk = (long)p.kv_heads * D;  // key-side row stride
@@ -123,8 +131,9 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems) {
   };
   auto block_of = [&](Q32Walk it) {
     Blk k;
-    const int bh = it.item / npr, r = it.item % npr;
-    const int rank = CAUSAL && it.half ? nqb - 1 - r : r;
+    const bool dealt = CAUSAL && deal;
+    const int bh = dealt ? it.item % npairs : it.item / npr, r = dealt ? it.item / npairs : it.item % npr;
+    const int rank = CAUSAL && !deal && it.half ? nqb - 1 - r : r;
     const int qb = CAUSAL ? nqb - 1 - rank : rank;  // causal: rank 0 is the last block
     const int b = bh / p.heads, h = bh % p.heads;
     const int hk = h / (p.heads / p.kv_heads);
@@ -155,6 +164,11 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems) {
   };
   // The item after `it` in this workgroup's list.
   auto next_of = [&](Q32Walk it) {
+    if (CAUSAL && deal) {
+      const int round = it.half + 1;
+      const int rev = ngrid % 8 == 0 ? (ngrid / 8 - 1 - w / 8) * 8 + w % 8 : ngrid - 1 - w;
+      return Q32Walk{round * ngrid + (round & 1 ? rev : w), round};
+    }
     if (CAUSAL && it.half == 0 && 2 * (it.item % npr) + 1 != nqb) return Q32Walk{it.item, 1};
     return Q32Walk{it.item + ngrid, 0};
   };
@@ -406,18 +420,43 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems) {
 
 }  // namespace
 
+// Whether a causal grid deals its blocks one by one instead of folding them
+// (bwdbwd_q32_kernel; both give the same bits): when every block can have a CU of
+// its own, or when the folded items' rounds take over 8 % longer than the longest
+// block or an even share of all blocks (their keys vary linearly, from first to
+// last). Stage 1, us, folded / dealt: one round of blocks, B1 N512 H12 28.6 / 20.5,
+// B1 N1024 H12 41.8 / 33.7, B1 N2048 H12 67.5 / 62.0; estimated gain 12 %, B4 N1024
+// H12 46.0 / 44.6; 11 %, B24 N1024 H12 258 / 248; 33 %, B1 N8192 H12 650 / 518; 36 %,
+// B8 N1500 H12 fp16 218 / 176; 50 %, B3 N2048 H12 155 / 115; but 7 %, B40 N1024 H12
+// 414 / 422; 6 %, B2 N2048 H12 77.0 / 78.4; 3 %, B1 N4096 H12 141 / 149 (fewer CUs
+// run faster); none, B32 N1024 H12 324 / 332, B4 N2048 H16 182 / 183.
+template <typename T> inline bool q32_deal(const BwdBwdParams<T>& p, int nqb, int npairs, int resident) {
+  const long blocks = (long)npairs * nqb;
+  if (blocks <= resident) return true;
+  auto keys = [&](int qb) {
+    const long e = (long)(qb + 1) * (32 * kWaves) + p.coff;
+    return (double)(e < 0 ? 0 : e < p.nk ? e : p.nk);
+  };
+  const double first = keys(0), last = keys(nqb - 1);
+  const long rounds = ((long)npairs * ((nqb + 1) / 2) + resident - 1) / (resident > 0 ? resident : 1);
+  const double share = 0.5 * (first + last) * (double)blocks / resident;
+  return resident > 0 && (double)rounds * (first + last) > 1.08 * (last > share ? last : share);
+}
+
 template <typename T, bool CAUSAL>
 hipError_t launch_bwdbwd_stage1_q32(const BwdBwdParams<T>& p, hipStream_t stream) {
   const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
-  const int nitems = p.batch * p.heads * (CAUSAL ? (nqb + 1) / 2 : nqb);
+  const int npairs = p.batch * p.heads;
   const int resident = resident_workgroups(1);
+  const int deal = CAUSAL && q32_deal(p, nqb, npairs, resident);
+  const int nitems = npairs * (CAUSAL && !deal ? (nqb + 1) / 2 : nqb);
   const dim3 grid(resident > 0 && resident < nitems ? resident : nitems);
   int e2;
   if (std::is_same_v<T, __bf16> && std::frexp(p.scale, &e2) == 0.5f)  // scale = 2^(e2 - 1)
     hipLaunchKernelGGL((bwdbwd_q32_kernel<T, CAUSAL, std::is_same_v<T, __bf16>>), grid, dim3(kThreads), 0, stream, p,
-                       nitems);
+                       nitems, deal);
   else
-    hipLaunchKernelGGL((bwdbwd_q32_kernel<T, CAUSAL, false>), grid, dim3(kThreads), 0, stream, p, nitems);
+    hipLaunchKernelGGL((bwdbwd_q32_kernel<T, CAUSAL, false>), grid, dim3(kThreads), 0, stream, p, nitems, deal);
   return hipGetLastError();
 }
 
