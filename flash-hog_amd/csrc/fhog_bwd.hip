@@ -464,8 +464,8 @@ inline bool one_wave_selected(const char* var, const char* name, int n, int npai
   if (v != nullptr && std::strcmp(v, "compiled") == 0) return false;
   const int nb = (int)(((long)n + 255) / 256);
   const int resident = resident_workgroups(1);
-  const int pairs = block_pairing(causal, nb, npairs, resident, 1);
-  return one_wave_cover(n, causal, percent) && one_wave_grid((pairs ? (nb + 1) / 2 : nb) * npairs, resident);
+  const bool mirrored = causal && (long)nb * npairs > resident;
+  return one_wave_cover(n, causal, percent) && one_wave_grid((mirrored ? (nb + 1) / 2 : nb) * npairs, resident);
 }
 inline bool pair_selected(int nk, int npairs, bool causal) {
   const char* v = std::getenv("FLASH_HOG_BWD");

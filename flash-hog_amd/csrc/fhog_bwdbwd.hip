@@ -343,7 +343,7 @@ bwdbwd_q_kernel(BwdBwdParams<T> p, int chunk) {
 template <typename T, int D, bool CAUSAL, bool PRE>
 __global__ void __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(Occupancy<T, D>::value, Occupancy<T, D>::value)))
-bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk) {
+bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk, int fold) {
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 16;
   constexpr int DT = D / 32;
@@ -360,11 +360,12 @@ bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk) {
   const int n = lane & 31, g = lane >> 5;
   const int nbh = p.batch * p.kv_heads;
   const int nkb = (p.nk + BKB - 1) / BKB;
-  // Key block `rank` of pair bh (causal: the longest key columns come first),
-  // and with pairs > 0 also a second one (block_pair).
+  // Key block `rank` of pair bh (causal: the longest key columns come first, up to
+  // rank `fold`; the ranks from there on run backwards, fold_rank), and with
+  // pairs > 0 also a second one (block_pair).
   const GridSlot slot = grid_slot(blockIdx.x, nbh, pairs ? (nkb + 1) / 2 : nkb, chunk);
   const int bh = slot.pair;
-  const BlockPair bp = block_pair(slot.rank, nkb, pairs);
+  const BlockPair bp = block_pair(folded(slot.rank, nkb, fold), nkb, pairs);
   for (int blk = 0; blk < bp.count; ++blk) {
     const int kb = blk == 0 ? bp.first : bp.second;
     if (blk > 0) __syncthreads();  // every wave is done with the previous block's ring
@@ -723,19 +724,19 @@ hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stage
       if (stage2_pair_selected(variant, p.nk, p.batch * p.kv_heads, CAUSAL))
         return launch_bwdbwd_stage2_pair<T, D, CAUSAL>(p, stream);
       const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
-      // Pair causal key blocks when the grid outnumbers the resident workgroups.
       const int npairs = p.batch * p.kv_heads;
       const int resident = resident_workgroups(Occupancy<T, D>::value);
       const int pairs = block_pairing(CAUSAL, nkb, npairs, resident, Occupancy<T, D>::value);
       const int nranks = pairs ? (nkb + 1) / 2 : nkb;
       const int chunk = grid_chunk(npairs, nranks, resident);
+      const int fold = pairs ? nkb : fold_rank(CAUSAL, nkb, npairs, resident_workgroups(1));
       const dim3 grid(nranks * npairs);
       int e2;
       if (std::is_same_v<T, __bf16> && std::frexp(p.scale, &e2) == 0.5f)  // scale = 2^(e2 - 1)
         hipLaunchKernelGGL((bwdbwd_k_kernel<T, D, CAUSAL, std::is_same_v<T, __bf16>>), grid, dim3(kThreads), 0, stream,
-                           p, pairs, chunk);
+                           p, pairs, chunk, fold);
       else
-        hipLaunchKernelGGL((bwdbwd_k_kernel<T, D, CAUSAL, false>), grid, dim3(kThreads), 0, stream, p, pairs, chunk);
+        hipLaunchKernelGGL((bwdbwd_k_kernel<T, D, CAUSAL, false>), grid, dim3(kThreads), 0, stream, p, pairs, chunk, fold);
       return hipGetLastError();
     } else {
       return launch_bwdbwd_stage2_pair<T, D, CAUSAL>(p, stream);

@@ -555,11 +555,16 @@ __device__ __forceinline__ int folded(int rank, int nb, int fold) { return rank 
 
 // The `pairs` argument of block_pair for a grid of nb causal blocks per
 // (batch, head) pair: mirror pairs when the unpaired grid outnumbers the
-// resident workgroups, skewed ones when the paired grid is exactly one round
-// at two workgroups per CU.
+// resident workgroups and the paired one fills whole rounds of them, skewed ones
+// when it is exactly one round at two workgroups per CU. Otherwise the unpaired
+// blocks, longest first, balance better (stage 2, us, paired / unpaired: paired
+// grids of 0.56 rounds, B3 N2048 H12, 125 / 96; 0.75, B1 N8192 H12, 442 / 387;
+// 1.5, B16 N1024 H12, 132 / 122; 2.25, B24 N1024 H12, 216 / 194; but 1, B4 N2048
+// H16, 138 / 148; 3, B32 N1024 H12, 262 / 263; 6, B256 N256 H12, 270 / 277).
 inline int block_pairing(bool causal, int nb, int npairs, int resident, int waves) {
-  int pairs = causal && resident > 0 && (long)nb * npairs > resident;
-  if (pairs && nb % 4 == 0 && (long)((nb + 1) / 2) * npairs == resident && waves == 2) pairs = 2;
+  const long paired = (long)((nb + 1) / 2) * npairs;
+  int pairs = causal && resident > 0 && (long)nb * npairs > resident && paired % resident == 0;
+  if (pairs && nb % 4 == 0 && paired == resident && waves == 2) pairs = 2;
   return pairs;
 }
 
