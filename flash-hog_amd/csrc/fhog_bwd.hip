@@ -425,13 +425,16 @@ bwd_k_kernel(BwdParams<T> p, int chunk) {
 //
 // The one-wave kernels (k64, q64) are the fastest per tile, but run one 256-row
 // block per CU at a time and gain nothing when a CU is left alone. They are taken
-// when their grid fills whole rounds of the resident workgroups (or at least
-// six; at B8 N2048 H12 causal, 1.5 rounds, q64 took 258 against 241) and their
-// blocks cover little more than 128-row ones, in padding and, causal, above the
-// diagonal: up to 6 % more for dQ, 10 % for dK/dV (both one-wave / both compiled:
-// 6 % more, B8 N2048 H16 causal 280 / 297; 7 %, B20 N1700 H12 437 / 423; 11 %,
-// B64 N1000 H12 587 / 552; 20 %, B64 N600 H16 fp16 non-causal 559 / 501; 27 %, B24
-// N1300 H12 391 / 317; dK/dV alone 8 %, B16 N1536 H16 357 / 363).
+// when their blocks cover little more than 128-row ones, in padding and, causal,
+// above the diagonal: up to 6 % more for dQ, 10 % for dK/dV (both one-wave / both
+// compiled: 6 % more, B8 N2048 H16 causal 280 / 297; 7 %, B20 N1700 H12 437 / 423;
+// 11 %, B64 N1000 H12 587 / 552; 20 %, B64 N600 H16 fp16 non-causal 559 / 501; 27 %,
+// B24 N1300 H12 391 / 317; dK/dV alone 8 %, B16 N1536 H16 357 / 363); and when their
+// grid fills whole rounds of the resident workgroups, or at least six (at B8 N2048
+// H12 causal, 1.5 rounds, q64 took 258 against 241). A causal dK/dV needs no whole
+// rounds: its key blocks, longest first, even out (first backward, compiled / k64:
+// 1.1 rounds, B3 N2048 H12, 108 / 105; 1.5, B2 N4096 H12, 216 / 208, B1 N8192 H12, 405 /
+// 387; 1.75, B7 N4096 H16 over 4 key heads, 958 / 869; 4.1, B11 N2048 H12, 326 / 320).
 //
 // The pair kernels do more LDS work per tile but take half the time per tile of
 // a wave, and their 64-row blocks spread a small grid over twice as many CUs and
@@ -458,14 +461,16 @@ inline bool one_wave_cover(int n, bool causal, int percent) {
   const long b1 = ((long)n + 127) / 128, b2 = ((long)n + 255) / 256 * 2;
   return 100 * b2 * (causal ? b2 + 2 : 1) <= percent * b1 * (causal ? b1 + 1 : 1);
 }
-inline bool one_wave_selected(const char* var, const char* name, int n, int npairs, bool causal, int percent) {
+inline bool one_wave_selected(const char* var, const char* name, int n, int npairs, bool causal, int percent,
+                              bool any_grid) {
   const char* v = std::getenv(var);
   if (v != nullptr && std::strcmp(v, name) == 0) return true;
   if (v != nullptr && std::strcmp(v, "compiled") == 0) return false;
   const int nb = (int)(((long)n + 255) / 256);
   const int resident = resident_workgroups(1);
   const bool mirrored = causal && (long)nb * npairs > resident;
-  return one_wave_cover(n, causal, percent) && one_wave_grid((mirrored ? (nb + 1) / 2 : nb) * npairs, resident);
+  return one_wave_cover(n, causal, percent) &&
+         (any_grid || one_wave_grid((mirrored ? (nb + 1) / 2 : nb) * npairs, resident));
 }
 inline bool pair_selected(int nk, int npairs, bool causal) {
   const char* v = std::getenv("FLASH_HOG_BWD");
@@ -486,7 +491,7 @@ hipError_t launch_bwd_dq(const BwdParams<T>& p, hipStream_t stream) {
     const int npairs = p.batch * p.heads;
     if (!qpair_selected(p.nq, npairs, D, CAUSAL)) {
       if constexpr (D == 64) {
-        if (one_wave_selected("FLASH_HOG_BWDQ", "q64", p.nq, npairs, CAUSAL, 106))
+        if (one_wave_selected("FLASH_HOG_BWDQ", "q64", p.nq, npairs, CAUSAL, 106, false))
           return launch_bwd_q64<T, CAUSAL>(p, stream);
       }
       const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
@@ -504,7 +509,7 @@ hipError_t launch_bwd_dkdv(const BwdParams<T>& p, hipStream_t stream) {
   if constexpr (sizeof(T) == 2 && D == 64) {
     const int npairs = p.batch * p.kv_heads;
     if (!pair_selected(p.nk, npairs, CAUSAL)) {
-      if (one_wave_selected("FLASH_HOG_BWD", "k64", p.nk, npairs, CAUSAL, 110))
+      if (one_wave_selected("FLASH_HOG_BWD", "k64", p.nk, npairs, CAUSAL, 110, CAUSAL))
         return launch_bwd_k64<T, CAUSAL>(p, stream);
       const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
       hipLaunchKernelGGL((bwd_k_kernel<T, D, CAUSAL>), dim3(nkb * npairs), dim3(kThreads), 0, stream, p,
