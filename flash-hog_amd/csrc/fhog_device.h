@@ -554,18 +554,27 @@ inline int fold_rank(bool causal, int nb, int npairs, int cus) {
 __device__ __forceinline__ int folded(int rank, int nb, int fold) { return rank < fold ? rank : nb - 1 - (rank - fold); }
 
 // The `pairs` argument of block_pair for a grid of nb causal blocks per
-// (batch, head) pair: mirror pairs when the unpaired grid outnumbers the
-// resident workgroups and the paired one fills whole rounds of them, skewed ones
-// when it is exactly one round at two workgroups per CU. Otherwise the unpaired
-// blocks, longest first, balance better (stage 2, us, paired / unpaired: paired
-// grids of 0.56 rounds, B3 N2048 H12, 125 / 96; 0.75, B1 N8192 H12, 442 / 387;
-// 1.5, B16 N1024 H12, 132 / 122; 2.25, B24 N1024 H12, 216 / 194; but 1, B4 N2048
-// H16, 138 / 148; 3, B32 N1024 H12, 262 / 263; 6, B256 N256 H12, 270 / 277).
+// (batch, head) pair. Mirror pairs halve the number of workgroups and are taken
+// only where the paired grid fills whole rounds of the resident ones; elsewhere
+// the unpaired blocks, longest first, balance better (stage 2, us, paired /
+// unpaired: paired grids of 0.56 rounds, B3 N2048 H12, 125 / 96; 0.75, B1 N8192 H12,
+// 442 / 387; 1.5, B16 N1024 H12, 132 / 122; 2.25, B24 N1024 H12, 216 / 194). At two
+// workgroups per CU that is
+// - one round, skewed if nb allows (B4 N2048 H16 138 / 148, B1 N16384 H8 944 / 1021);
+// - more rounds of fewer than 8 blocks per pair (nb = 2, 6 rounds, B256 N256 H12
+//   270 / 277; 4, 2 rounds, B64 N512 H8 124 / 128; 5, 3 rounds, B8 N640 H64 173 / 175;
+//   but 8, 2 rounds, B16 N1024 H16 180 / 174; 16, 2 rounds, B8 N2048 H16 302 / 290; 256,
+//   2 rounds, B1 N32768 H8 3795 / 3720);
+// - one paired workgroup per CU, from 32 blocks per pair (64, B1 N8192 H8 309 / 320; 32,
+//   B4 N4096 H16 over 4 key heads 623 / 634; but 16, B4 N2048 H8 92.6 / 90.1).
+// At one workgroup per CU pairs are as good in any number of whole rounds.
 inline int block_pairing(bool causal, int nb, int npairs, int resident, int waves) {
-  const long paired = (long)((nb + 1) / 2) * npairs;
-  int pairs = causal && resident > 0 && (long)nb * npairs > resident && paired % resident == 0;
-  if (pairs && nb % 4 == 0 && paired == resident && waves == 2) pairs = 2;
-  return pairs;
+  const long paired = (long)((nb + 1) / 2) * npairs, single = (long)nb * npairs;
+  if (!causal || resident <= 0) return 0;
+  if (waves == 2 && nb >= 32 && single == resident && 2 * paired == resident) return 1;
+  if (single <= resident || paired % resident != 0) return 0;
+  if (waves == 2 && paired == resident && nb % 4 == 0) return 2;
+  return waves != 2 || paired == resident || nb < 8;
 }
 
 }  // namespace fhog

@@ -9,7 +9,8 @@ batches below give, with 128-row blocks on 256 CUs, three blocks per head in
 1.5 rounds, four in 1.25 rounds of folded items, four in exactly one and two of
 them, and nine blocks in 4.5 rounds; in stage 2, at two workgroups per CU, three
 and four blocks mirrored in one round (an odd count has a middle block that is its
-own mirror).
+own mirror), eight unmirrored although they would fill two, and 32 mirrored in
+half a round.
 """
 
 from __future__ import annotations
@@ -28,6 +29,8 @@ GRIDS = [
     ("four_blocks_whole_round", 32, 512, 512, 4, 1),
     ("three_blocks_mirrored", 64, 330, 330, 4, 1),
     ("four_blocks_two_rounds", 64, 512, 512, 4, 1),
+    ("eight_blocks_two_rounds", 64, 1000, 1000, 4, 1),
+    ("many_blocks_one_per_cu", 4, 4000, 4000, 4, 1),
     ("nine_blocks_bottom_right", 8, 1100, 1170, 16, 2),
     ("rows_without_keys", 24, 700, 500, 6, 2),
 ]
