@@ -26,8 +26,8 @@
 // stage i mod 8, tile i + 6 is loaded at step i into the stage tile i - 2
 // left. Grouped-query heads are visited query tile by query tile, the heads
 // of the group in turn, as in bwd_k_kernel. Causal key blocks are taken in
-// mirror pairs (block r, then block nkb - 1 - r) when the grid outnumbers
-// the CUs.
+// mirror pairs (block r, then block nkb - 1 - r) when those fill whole rounds
+// of the CUs, and singly, longest first, otherwise (block_pairing).
 #include <cmath>
 #include <cstdint>
 

@@ -21,8 +21,8 @@
 // A workgroup owns 256 queries of one (batch, head) pair and streams 32-key
 // tiles of K (wave 0) and V (wave 1) of the head's key/value head through an
 // 8-stage LDS ring of 8 KiB stages. Causal query blocks are taken in mirror
-// pairs (the longest block, then the shortest) when the grid outnumbers the
-// CUs.
+// pairs (the longest block, then the shortest) when those fill whole rounds of
+// the CUs, and singly, longest first, otherwise (block_pairing).
 #include <cmath>
 #include <cstdint>
 

@@ -2,7 +2,7 @@
 // keys) for 2-byte types at D = 64: 32 queries per wave on the 32x32x16
 // matrix instruction, one wave per SIMD, software-pipelined three tiles deep.
 // The math and outputs are those of fhog_bwdbwd_fused.hip (which serves
-// D = 128 and 256): with u = dP - D, x = P ddS, X = P (dPa + ddS u),
+// D = 256 and short causal sequences): with u = dP - D, x = P ddS, X = P (dPa + ddS u),
 //   dQ2 = scale (sum_j P u ddK + sum_j X K - dD sum_j P u K - c sum_j P K),
 //   ddO = sum_j P ddV + sum_j x V - dD' O,     c = D dD + B,
 //   c = sum_j X - dD sum_j P u,  B = c - D dD,
@@ -25,8 +25,8 @@
 // matrix instruction at one wave per SIMD: 85 % of the pipe.)
 //
 // The default stage 1 for 2-byte types at D = 64: 177-180 us at B4 N2048 H16
-// causal bf16 against 184-189 us for the fused kernel, 3-6 % faster on every
-// D = 64 configuration measured.
+// causal bf16 against 184-189 us for the fused kernel. Causal sequences of
+// up to 512 run that one (launch_bwdbwd).
 //
 // Layouts (32x32x16, see fhog_device.h): score tiles are transposed,
 // S^T = K Q^T, so lane n of a wave holds query q0 + n and register r key
