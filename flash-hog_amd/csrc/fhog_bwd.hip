@@ -415,84 +415,36 @@ bwd_k_kernel(BwdParams<T> p, int chunk) {
 
 }  // namespace
 
-// The first backward for 2-byte types at D = 64 has several kernels for each
-// half of its work, all giving the same bits: dK/dV in bwd_k_kernel above, in
-// bwd_k64_kernel (fhog_bwd_k64.hip: 64 keys per wave at one wave per SIMD,
-// generated sweep) or in bwd_pair_kernel (fhog_bwd_pair.h: two waves per 32
-// keys), dQ in bwd_q_kernel above, in bwd_q64_kernel (fhog_bwd_q64.hip, 64
-// queries per wave) or in bwd_qpair_kernel (fhog_bwd_qpair.hip: two waves per 32
-// queries). First backward, us, at D = 64 bf16 unless named:
-//
-// The one-wave kernels (k64, q64) are the fastest per tile, but run one 256-row
-// block per CU at a time and gain nothing when a CU is left alone. They are taken
-// when their blocks cover little more than 128-row ones, in padding and, causal,
-// above the diagonal: up to 6 % more for dQ, 10 % for dK/dV (both one-wave / both
-// compiled: 6 % more, B8 N2048 H16 causal 280 / 297; 7 %, B20 N1700 H12 437 / 423;
-// 11 %, B64 N1000 H12 587 / 552; 20 %, B64 N600 H16 fp16 non-causal 559 / 501; 27 %,
-// B24 N1300 H12 391 / 317; dK/dV alone 8 %, B16 N1536 H16 357 / 363); and when their
-// grid fills whole rounds of the resident workgroups, or at least six (at B8 N2048
-// H12 causal, 1.5 rounds, q64 took 258 against 241). A causal dK/dV needs no whole
-// rounds: its key blocks, longest first, even out (first backward, compiled / k64:
-// 1.1 rounds, B3 N2048 H12, 108 / 105; 1.5, B2 N4096 H12, 216 / 208, B1 N8192 H12, 405 /
-// 387; 1.75, B7 N4096 H16 over 4 key heads, 958 / 869; 4.1, B11 N2048 H12, 326 / 320).
-//
-// The pair kernels do more LDS work per tile but take half the time per tile of
-// a wave, and their 64-row blocks spread a small grid over twice as many CUs and
-// waste less of a short causal sequence's diagonal. dK/dV takes its pair kernel
-// up to three workgroups per CU, and for causal sequences of up to 1024 keys
-// (others / pair: causal B1 N1024 H12 (192 workgroups) 52.4 / 45.0, B1 N4096 H12
-// (768) 184 / 163, B2 N4096 H16 over 4 key heads (512) 523 / 446, B128 N512 H12
-// 448 / 417, B24 N1024 H12 219 / 213, B32 N1024 H16 399 / 403, B4 N2048 H16 136 /
-// 151; non-causal B1 N2048 H16 (512) 95.2 / 92.9, B2 N2048 H12 (768) 120 / 117, B8
-// N1000 H12 fp16 (1536) 122.8 / 124.0). dQ gains less and takes its pair kernel,
-// at D = 64 and 128, up to one workgroup per CU (B1 N512 H12 27.0 / 26.1, B1
-// N2048 H8 D128 non-causal 118 / 109; B2 N1000 H12 fp16, 384 workgroups, 51.2 /
-// 55.7), and at D = 64 for causal sequences of up to 512 queries (B32 N512 H12
-// 106 / 99, B128 N256 H12 171 / 166; B32 N1024 H12 287 / 301).
-// FLASH_HOG_BWD (dK/dV, D = 64) = compiled, k64 or pair and FLASH_HOG_BWDQ (dQ,
-// D = 64 and 128) = compiled, q64 (D = 64) or pair force a kernel; read at
-// every launch.
-inline bool one_wave_grid(int workgroups, int resident) {
-  return resident > 0 && workgroups > 0 && (workgroups % resident == 0 || workgroups >= 6 * resident);
-}
-// Whether 256-row blocks of n rows cover at most `percent` of what 128-row ones
-// do (rows of the blocks times, when causal, the mean of what they see).
-inline bool one_wave_cover(int n, bool causal, int percent) {
-  const long b1 = ((long)n + 127) / 128, b2 = ((long)n + 255) / 256 * 2;
-  return 100 * b2 * (causal ? b2 + 2 : 1) <= percent * b1 * (causal ? b1 + 1 : 1);
-}
-inline bool one_wave_selected(const char* var, const char* name, int n, int npairs, bool causal, int percent,
-                              bool any_grid) {
-  const char* v = std::getenv(var);
-  if (v != nullptr && std::strcmp(v, name) == 0) return true;
-  if (v != nullptr && std::strcmp(v, "compiled") == 0) return false;
-  const int nb = (int)(((long)n + 255) / 256);
-  const int resident = resident_workgroups(1);
-  const bool mirrored = causal && (long)nb * npairs > resident;
-  return one_wave_cover(n, causal, percent) &&
-         (any_grid || one_wave_grid((mirrored ? (nb + 1) / 2 : nb) * npairs, resident));
-}
-inline bool pair_selected(int nk, int npairs, bool causal) {
+// The kernels of each half are chosen by the rules of fhog_grid.h. FLASH_HOG_BWD
+// (dK/dV, D = 64) = compiled, k64 or pair and FLASH_HOG_BWDQ (dQ, D = 64 and 128)
+// = compiled, q64 (D = 64) or pair force a kernel; read at every launch.
+enum class Dkdv { compiled, k64, pair };
+inline Dkdv dkdv_selected(Mask m, int npairs) {
   const char* v = std::getenv("FLASH_HOG_BWD");
-  if (v != nullptr && std::strcmp(v, "pair") == 0) return true;
-  if (v != nullptr && (std::strcmp(v, "compiled") == 0 || std::strcmp(v, "k64") == 0)) return false;
-  return (causal && nk <= 1024) || (long)((nk + 63) / 64) * npairs <= 3L * resident_workgroups(1);
+  if (v != nullptr && std::strcmp(v, "pair") == 0) return Dkdv::pair;
+  if (v != nullptr && std::strcmp(v, "k64") == 0) return Dkdv::k64;
+  if (v != nullptr && std::strcmp(v, "compiled") == 0) return Dkdv::compiled;
+  const int cus = resident_workgroups(1);
+  return bwd_pair_rule(m, npairs, cus) ? Dkdv::pair : bwd_k64_rule(m, npairs, cus) ? Dkdv::k64 : Dkdv::compiled;
 }
-inline bool qpair_selected(int nq, int npairs, int head_dim, bool causal) {
+enum class Dq { compiled, q64, pair };
+inline Dq dq_selected(Mask m, int npairs, int head_dim) {
   const char* v = std::getenv("FLASH_HOG_BWDQ");
-  if (v != nullptr && std::strcmp(v, "pair") == 0) return true;
-  if (v != nullptr && (std::strcmp(v, "compiled") == 0 || std::strcmp(v, "q64") == 0)) return false;
-  return (causal && head_dim == 64 && nq <= 512) || (long)((nq + 63) / 64) * npairs <= resident_workgroups(1);
+  if (v != nullptr && std::strcmp(v, "pair") == 0) return Dq::pair;
+  if (v != nullptr && std::strcmp(v, "q64") == 0) return Dq::q64;
+  if (v != nullptr && std::strcmp(v, "compiled") == 0) return Dq::compiled;
+  const int cus = resident_workgroups(1);
+  return bwd_qpair_rule(m, npairs, head_dim, cus) ? Dq::pair : bwd_q64_rule(m, npairs, cus) ? Dq::q64 : Dq::compiled;
 }
 
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd_dq(const BwdParams<T>& p, hipStream_t stream) {
   if constexpr (sizeof(T) == 2 && D <= 128) {
     const int npairs = p.batch * p.heads;
-    if (!qpair_selected(p.nq, npairs, D, CAUSAL)) {
+    const Dq sel = dq_selected(mask_of(CAUSAL, p), npairs, D);
+    if (sel != Dq::pair) {
       if constexpr (D == 64) {
-        if (one_wave_selected("FLASH_HOG_BWDQ", "q64", p.nq, npairs, CAUSAL, 106, false))
-          return launch_bwd_q64<T, CAUSAL>(p, stream);
+        if (sel == Dq::q64) return launch_bwd_q64<T, CAUSAL>(p, stream);
       }
       const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
       hipLaunchKernelGGL((bwd_q_kernel<T, D, CAUSAL>), dim3(nqb * npairs), dim3(kThreads), 0, stream, p,
@@ -508,9 +460,9 @@ template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd_dkdv(const BwdParams<T>& p, hipStream_t stream) {
   if constexpr (sizeof(T) == 2 && D == 64) {
     const int npairs = p.batch * p.kv_heads;
-    if (!pair_selected(p.nk, npairs, CAUSAL)) {
-      if (one_wave_selected("FLASH_HOG_BWD", "k64", p.nk, npairs, CAUSAL, 110, CAUSAL))
-        return launch_bwd_k64<T, CAUSAL>(p, stream);
+    const Dkdv sel = dkdv_selected(mask_of(CAUSAL, p), npairs);
+    if (sel == Dkdv::k64) return launch_bwd_k64<T, CAUSAL>(p, stream);
+    if (sel == Dkdv::compiled) {
       const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
       hipLaunchKernelGGL((bwd_k_kernel<T, D, CAUSAL>), dim3(nkb * npairs), dim3(kThreads), 0, stream, p,
                          grid_chunk(npairs, nkb, resident_workgroups(kOcc)));

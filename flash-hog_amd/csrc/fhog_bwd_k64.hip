@@ -326,7 +326,7 @@ hipError_t launch_bwd_k64(const BwdParams<T>& p, hipStream_t stream) {
   const int nkb = (p.nk + 64 * kWaves - 1) / (64 * kWaves);
   const int npairs = p.batch * p.kv_heads;
   const int resident = resident_workgroups(1);
-  const int pairs = block_pairing(CAUSAL, nkb, npairs, resident, 1);
+  const int pairs = block_pairing(mask_of(CAUSAL, p), nkb, npairs, resident, 1);
   const int nranks = pairs ? (nkb + 1) / 2 : nkb;
   const int chunk = grid_chunk(npairs, nranks, resident);
   hipLaunchKernelGGL((bwd_k64_kernel<T, CAUSAL>), dim3(nranks * npairs), dim3(kThreads), 0, stream, p, pairs,

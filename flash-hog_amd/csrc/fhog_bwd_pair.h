@@ -282,22 +282,15 @@ hipError_t launch_bwd_pair(const BwdParams<T>& p, hipStream_t stream) {
   const int nkb = (p.nk + 32 * kPairs - 1) / (32 * kPairs);
   const int npairs = p.batch * p.kv_heads;
   const int cus = resident_workgroups(1);
-  // Three workgroups per CU at 256-byte rows (168 registers): for fp32 always
-  // (D = 64 B4 N2048 H16 1031 -> 1013 us, B2 N2048 H8 equal), for 2-byte D = 128
-  // once the grid is long (two / three: 359 / 392 us at B2 N2048 H32 over 8 key
-  // heads, 512 workgroups; 300 / 287 at B4 N2048 H16, 2048; 2040 / 1956 at B2
-  // N8192 H16, 4096). 2-byte D = 64 likewise with four (117 registers; first
-  // backward, two / four: causal B1 N4096 H12, 768 workgroups, 163 / 166, B2 N2048
-  // H16, 1024, 105 / 99, B128 N512 H12 484 / 417; non-causal B2 N2048 H12, 768,
-  // 146 / 117).
+  [[maybe_unused]] const int waves = bwd_pair_waves(mask_of(CAUSAL, p), npairs, D, (int)sizeof(T), cus);
   if constexpr (sizeof(T) == 4 && D == 64) {
     return launch_occ<T, D, CAUSAL, 3>(p, nkb, npairs, cus, stream);
   } else {
     if constexpr (sizeof(T) == 2 && D == 128) {
-      if ((long)nkb * npairs > 4L * cus) return launch_occ<T, D, CAUSAL, 3>(p, nkb, npairs, cus, stream);
+      if (waves == 3) return launch_occ<T, D, CAUSAL, 3>(p, nkb, npairs, cus, stream);
     }
     if constexpr (sizeof(T) == 2 && D == 64) {
-      if ((long)nkb * npairs > (CAUSAL ? 3L : 2L) * cus) return launch_occ<T, D, CAUSAL, 4>(p, nkb, npairs, cus, stream);
+      if (waves == 4) return launch_occ<T, D, CAUSAL, 4>(p, nkb, npairs, cus, stream);
     }
     return launch_occ<T, D, CAUSAL, 2>(p, nkb, npairs, cus, stream);
   }

@@ -308,7 +308,7 @@ hipError_t launch_bwd_q64(const BwdParams<T>& p, hipStream_t stream) {
   const int nqb = (p.nq + 64 * kWaves - 1) / (64 * kWaves);
   const int npairs = p.batch * p.heads;
   const int resident = resident_workgroups(1);
-  const int pairs = block_pairing(CAUSAL, nqb, npairs, resident, 1);
+  const int pairs = block_pairing(mask_of(CAUSAL, p), nqb, npairs, resident, 1);
   const int nranks = pairs ? (nqb + 1) / 2 : nqb;
   const int chunk = grid_chunk(npairs, nranks, resident);
   hipLaunchKernelGGL((bwd_q64_kernel<T, CAUSAL>), dim3(nranks * npairs), dim3(kThreads), 0, stream, p, pairs,

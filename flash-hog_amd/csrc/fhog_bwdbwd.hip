@@ -639,58 +639,29 @@ bwdbwd_k_kernel(BwdBwdParams<T> p, int pairs, int chunk, int fold) {
 
 }  // namespace
 
-// Stage 1 for 2-byte types at D = 64 runs the kernel with 32 queries per
-// wave at one wave per SIMD, a hand-scheduled sweep and a persistent grid
-// (fhog_bwdbwd_q32.hip) but for causal sequences of up to 512, which run the fused
-// kernel (16 queries per wave, two waves per SIMD): its 64-query blocks take half
-// as long and waste less of the diagonal. Both give the same results to
-// rounding, so the choice looks at the sequence only, never at how many there are
-// (stage 1, us, q32 / fused: causal N256 H12 B1 21.5 / 11.9, B256 310 / 297; N512
-// B1 28.4 / 18.8, B16 64.7 / 52.6, B64 209 / 209, B128 418 / 425; N1024 B32 316 /
-// 330; non-causal N512 B16 fp16 74.6 / 85.7; B4 N2048 H16 causal 171 / 185).
-// FLASH_HOG_STAGE1 = q32 or fused forces either; read at every launch.
-inline bool stage1_fused_selected(int nq, int nk, bool causal) {
-  const char* v = std::getenv("FLASH_HOG_STAGE1");
-  if (v != nullptr && std::strcmp(v, "fused") == 0) return true;
-  if (v != nullptr && std::strcmp(v, "q32") == 0) return false;
-  return causal && nq <= 512 && nk <= 512;
-}
-
-// Stage 1 for fp32 runs bwdbwd_q_kernel below (one wave per 32 queries) on grids
-// that fill the chip and bwdbwd_qpair_kernel (fhog_bwdbwd_qpair.hip, two waves per
-// 32 queries, half the time per block and twice the workgroups) on smaller ones;
-// both give the same bits. The line is two of the latter's workgroups per CU
-// when causal, one otherwise (stage 1, us, q / qpair: causal D = 64 N2048 H8 B2
-// (512 workgroups) 887 / 631, B3 (768) 890 / 840-885, B4 (1024) 970 / 1093;
-// non-causal B1 (256) 902 / 626, B2 (512) 910 / 1021; D = 128 causal B2 (512)
-// 1620 / 1296, B4 (1024) 1783 / 2538, non-causal B1 (256) 1647 / 1255). FLASH_HOG_STAGE1 = compiled or pair forces
-// either for fp32. Read at every launch.
-inline bool stage1_qpair_selected(int nq, int npairs, bool causal) {
-  const char* v = std::getenv("FLASH_HOG_STAGE1");
-  if (v != nullptr && std::strcmp(v, "pair") == 0) return true;
-  if (v != nullptr && std::strcmp(v, "compiled") == 0) return false;
-  return (long)((nq + 63) / 64) * npairs <= (long)(causal ? 2 : 1) * resident_workgroups(1);
-}
-
-// Stage 2 runs bwdbwd_pair_kernel (fhog_bwdbwd_pair.hip, two waves per 32 keys)
-// but for 2-byte types at D = 64 on grids that fill the chip, where
-// bwdbwd_k_kernel's one wave per 32 keys is faster; both give the same bits.
-// The pair kernel's grid has twice the workgroups of half the work each, and
-// is taken while it has at most three of them per CU when causal, one
-// otherwise (stage 2, us, k / pair: causal B1 N512 H12 24.8 / 20.2, B1 N2048
-// H12 (384 workgroups) 78.4 / 69.7, B2 N2048 H12 (768) 85.2 / 74.8, B2 N4096
-// H16 over 4 key heads (512) 575 / 511, but B2 N2048 H16 (1024) 93.3 / 95.8 and
-// B1 N8192 H12 (1536) 452 / 497; non-causal B1 N300 over one key head 51.9 /
-// 44.2, but B1 N2048 H12 (384) 79.6 / 82.4, B2 N1000 H12 fp16 43.9 / 48.0).
-// FLASH_HOG_STAGE2 = compiled (bwdbwd_k_kernel) or pair forces either, and k32
-// selects, for bf16, the kernel with a generated sweep at one wave per SIMD
-// (fhog_bwdbwd_k32.hip), which agrees to rounding and is about 10 % slower at B4
+// The kernels of each stage are chosen by the rules of fhog_grid.h. FLASH_HOG_STAGE1
+// = q32 or fused (2-byte types at D = 64), compiled or pair (fp32) and
+// FLASH_HOG_STAGE2 = compiled or pair (2-byte types at D = 64) force a kernel; k32
+// selects, for bf16 at D = 64, the stage 2 with a generated sweep at one wave per
+// SIMD (fhog_bwdbwd_k32.hip), which agrees to rounding and is about 10 % slower at B4
 // N2048 H16. Read at every launch.
-inline bool stage2_selected(const char* v, const char* name) { return v != nullptr && std::strcmp(v, name) == 0; }
-inline bool stage2_pair_selected(const char* v, int nk, int npairs, bool causal) {
-  if (stage2_selected(v, "pair")) return true;
-  if (stage2_selected(v, "compiled")) return false;
-  return (long)((nk + 63) / 64) * npairs <= (long)(causal ? 3 : 1) * resident_workgroups(1);
+inline bool named(const char* v, const char* name) { return v != nullptr && std::strcmp(v, name) == 0; }
+inline bool stage1_fused_selected(Mask m) {
+  const char* v = std::getenv("FLASH_HOG_STAGE1");
+  if (named(v, "fused")) return true;
+  if (named(v, "q32")) return false;
+  return stage1_fused_rule(m);
+}
+inline bool stage1_qpair_selected(Mask m, int npairs) {
+  const char* v = std::getenv("FLASH_HOG_STAGE1");
+  if (named(v, "pair")) return true;
+  if (named(v, "compiled")) return false;
+  return stage1_qpair_rule(m, npairs, resident_workgroups(1));
+}
+inline bool stage2_pair_selected(const char* v, Mask m, int npairs) {
+  if (named(v, "pair")) return true;
+  if (named(v, "compiled")) return false;
+  return stage2_pair_rule(m, npairs, resident_workgroups(1));
 }
 
 template <typename T, int D, bool CAUSAL>
@@ -698,13 +669,13 @@ hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stage
   if (stages & 1) {
     hipError_t e;
     if constexpr (sizeof(T) == 2 && D == 64) {
-      e = stage1_fused_selected(p.nq, p.nk, CAUSAL) ? launch_bwdbwd_stage1_fused<T, D, CAUSAL>(p, stream)
+      e = stage1_fused_selected(mask_of(CAUSAL, p)) ? launch_bwdbwd_stage1_fused<T, D, CAUSAL>(p, stream)
                                                     : launch_bwdbwd_stage1_q32<T, CAUSAL>(p, stream);
     } else if constexpr (sizeof(T) == 2 && D == 128) {
       e = launch_bwdbwd_stage1_fused_pair<T, CAUSAL>(p, stream);
     } else if constexpr (sizeof(T) == 2) {
       e = launch_bwdbwd_stage1_fused<T, D, CAUSAL>(p, stream);
-    } else if (stage1_qpair_selected(p.nq, p.batch * p.heads, CAUSAL)) {
+    } else if (stage1_qpair_selected(mask_of(CAUSAL, p), p.batch * p.heads)) {
       e = launch_bwdbwd_stage1_qpair<D, CAUSAL>(p, stream);
     } else {
       const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
@@ -719,14 +690,14 @@ hipError_t launch_bwdbwd(const BwdBwdParams<T>& p, hipStream_t stream, int stage
     if constexpr (sizeof(T) == 2 && D == 64) {
       const char* variant = std::getenv("FLASH_HOG_STAGE2");
       if constexpr (std::is_same_v<T, __bf16>) {
-        if (stage2_selected(variant, "k32")) return launch_bwdbwd_stage2_k32<CAUSAL>(p, stream);
+        if (named(variant, "k32")) return launch_bwdbwd_stage2_k32<CAUSAL>(p, stream);
       }
-      if (stage2_pair_selected(variant, p.nk, p.batch * p.kv_heads, CAUSAL))
+      if (stage2_pair_selected(variant, mask_of(CAUSAL, p), p.batch * p.kv_heads))
         return launch_bwdbwd_stage2_pair<T, D, CAUSAL>(p, stream);
       const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
       const int npairs = p.batch * p.kv_heads;
       const int resident = resident_workgroups(Occupancy<T, D>::value);
-      const int pairs = block_pairing(CAUSAL, nkb, npairs, resident, Occupancy<T, D>::value);
+      const int pairs = block_pairing(mask_of(CAUSAL, p), nkb, npairs, resident, Occupancy<T, D>::value);
       const int nranks = pairs ? (nkb + 1) / 2 : nkb;
       const int chunk = grid_chunk(npairs, nranks, resident);
       const int fold = pairs ? nkb : fold_rank(CAUSAL, nkb, npairs, resident_workgroups(1));

@@ -297,7 +297,7 @@ hipError_t launch_bwdbwd_stage2_k32(const BwdBwdParams<__bf16>& p, hipStream_t s
   const int nkb = (p.nk + 32 * kWaves - 1) / (32 * kWaves);
   const int npairs = p.batch * p.kv_heads;
   const int resident = resident_workgroups(1);
-  const int pairs = block_pairing(CAUSAL, nkb, npairs, resident, 1);
+  const int pairs = block_pairing(mask_of(CAUSAL, p), nkb, npairs, resident, 1);
   const int nranks = pairs ? (nkb + 1) / 2 : nkb;
   const int chunk = grid_chunk(npairs, nranks, resident);
   const dim3 grid(nranks * npairs);

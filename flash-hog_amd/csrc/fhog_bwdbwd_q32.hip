@@ -420,35 +420,12 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems, int deal) {
 
 }  // namespace
 
-// Whether a causal grid deals its blocks one by one instead of folding them
-// (bwdbwd_q32_kernel; both give the same bits): when every block can have a CU of
-// its own, or when the folded items' rounds take over 8 % longer than the longest
-// block or an even share of all blocks (their keys vary linearly, from first to
-// last). Stage 1, us, folded / dealt: one round of blocks, B1 N512 H12 28.6 / 20.5,
-// B1 N1024 H12 41.8 / 33.7, B1 N2048 H12 67.5 / 62.0; estimated gain 12 %, B4 N1024
-// H12 46.0 / 44.6; 11 %, B24 N1024 H12 258 / 248; 33 %, B1 N8192 H12 650 / 518; 36 %,
-// B8 N1500 H12 fp16 218 / 176; 50 %, B3 N2048 H12 155 / 115; but 7 %, B40 N1024 H12
-// 414 / 422; 6 %, B2 N2048 H12 77.0 / 78.4; 3 %, B1 N4096 H12 141 / 149 (fewer CUs
-// run faster); none, B32 N1024 H12 324 / 332, B4 N2048 H16 182 / 183.
-template <typename T> inline bool q32_deal(const BwdBwdParams<T>& p, int nqb, int npairs, int resident) {
-  const long blocks = (long)npairs * nqb;
-  if (blocks <= resident) return true;
-  auto keys = [&](int qb) {
-    const long e = (long)(qb + 1) * (32 * kWaves) + p.coff;
-    return (double)(e < 0 ? 0 : e < p.nk ? e : p.nk);
-  };
-  const double first = keys(0), last = keys(nqb - 1);
-  const long rounds = ((long)npairs * ((nqb + 1) / 2) + resident - 1) / (resident > 0 ? resident : 1);
-  const double share = 0.5 * (first + last) * (double)blocks / resident;
-  return resident > 0 && (double)rounds * (first + last) > 1.08 * (last > share ? last : share);
-}
-
 template <typename T, bool CAUSAL>
 hipError_t launch_bwdbwd_stage1_q32(const BwdBwdParams<T>& p, hipStream_t stream) {
   const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
   const int npairs = p.batch * p.heads;
   const int resident = resident_workgroups(1);
-  const int deal = CAUSAL && q32_deal(p, nqb, npairs, resident);
+  const int deal = q32_deal_rule(mask_of(CAUSAL, p), npairs, resident);
   const int nitems = npairs * (CAUSAL && !deal ? (nqb + 1) / 2 : nqb);
   const dim3 grid(resident > 0 && resident < nitems ? resident : nitems);
   int e2;

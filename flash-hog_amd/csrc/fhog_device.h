@@ -21,6 +21,8 @@
 #include <type_traits>
 #include <stdint.h>
 
+#include "fhog_grid.h"
+
 namespace fhog {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -531,50 +533,7 @@ inline int resident_workgroups(int waves) {
   return cus * waves;
 }
 
-// The chunk for grid_slot. A grid of at most 8 rounds of resident
-// workgroups keeps the rank-major order, whose last round holds the blocks
-// with the least work; a longer grid takes about one round per chunk (at
-// least 8 pairs, a multiple of 8), so that the streamed tiles of the pairs
-// in flight stay in L2 instead of being fetched again by every block.
-inline int grid_chunk(int npairs, int nranks, int resident) {
-  if (resident <= 0 || (long)npairs * nranks <= 8L * resident) return npairs;
-  const int c = resident / nranks / 8 * 8;
-  return c < 8 ? 8 : (c < npairs ? c : npairs);
-}
-
-// First rank that runs backwards (block nb - 1 - (rank - fold)) in a grid of nb
-// causal blocks, longest first, per (batch, head) pair. A grid of one to two
-// workgroups per CU runs as one round in which workgroups i and i + (number of
-// CUs) share a CU: the second of them take their ranks backwards, so that the
-// shortest blocks sit beside the longest. nb: none does.
-inline int fold_rank(bool causal, int nb, int npairs, int cus) {
-  const long grid = (long)nb * npairs;
-  return causal && cus > 0 && grid > cus && grid <= 2L * cus ? (cus + npairs - 1) / npairs : nb;
-}
+// Block of a rank, the ranks from `fold` (fold_rank) on running backwards.
 __device__ __forceinline__ int folded(int rank, int nb, int fold) { return rank < fold ? rank : nb - 1 - (rank - fold); }
-
-// The `pairs` argument of block_pair for a grid of nb causal blocks per
-// (batch, head) pair. Mirror pairs halve the number of workgroups and are taken
-// only where the paired grid fills whole rounds of the resident ones; elsewhere
-// the unpaired blocks, longest first, balance better (stage 2, us, paired /
-// unpaired: paired grids of 0.56 rounds, B3 N2048 H12, 125 / 96; 0.75, B1 N8192 H12,
-// 442 / 387; 1.5, B16 N1024 H12, 132 / 122; 2.25, B24 N1024 H12, 216 / 194). At two
-// workgroups per CU that is
-// - one round, skewed if nb allows (B4 N2048 H16 138 / 148, B1 N16384 H8 944 / 1021);
-// - more rounds of fewer than 8 blocks per pair (nb = 2, 6 rounds, B256 N256 H12
-//   270 / 277; 4, 2 rounds, B64 N512 H8 124 / 128; 5, 3 rounds, B8 N640 H64 173 / 175;
-//   but 8, 2 rounds, B16 N1024 H16 180 / 174; 16, 2 rounds, B8 N2048 H16 302 / 290; 256,
-//   2 rounds, B1 N32768 H8 3795 / 3720);
-// - one paired workgroup per CU, from 32 blocks per pair (64, B1 N8192 H8 309 / 320; 32,
-//   B4 N4096 H16 over 4 key heads 623 / 634; but 16, B4 N2048 H8 92.6 / 90.1).
-// At one workgroup per CU pairs are as good in any number of whole rounds.
-inline int block_pairing(bool causal, int nb, int npairs, int resident, int waves) {
-  const long paired = (long)((nb + 1) / 2) * npairs, single = (long)nb * npairs;
-  if (!causal || resident <= 0) return 0;
-  if (waves == 2 && nb >= 32 && single == resident && 2 * paired == resident) return 1;
-  if (single <= resident || paired % resident != 0) return 0;
-  if (waves == 2 && paired == resident && nb % 4 == 0) return 2;
-  return waves != 2 || paired == resident || nb < 8;
-}
 
 }  // namespace fhog

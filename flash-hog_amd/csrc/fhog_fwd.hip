@@ -228,18 +228,13 @@ fwd_kernel(FwdParams<T> p, int chunk) {
 
 }  // namespace
 
-// fwd_pair_kernel (two waves per 32 queries, 64-query workgroups) serves 2-byte
-// types at D = 256, and fp32 while its grid has at most one workgroup per CU, or
-// four (D = 64) or three (D = 128) when causal; fp32's two kernels give the same
-// bits (us, fwd / pair: causal N2048 H8 D64 B2 (512 workgroups) 142 / 99, B4
-// (1024) 196 / 165, B4 H16 (2048) 287 / 312; non-causal B1 (256) 142 / 97, B2
-// (512) 144 / 157; D128 causal B3 (768) 273 / 237, B4 (1024) 300 / 309).
-// FLASH_HOG_FWD = compiled or pair forces either for fp32; read at every launch.
-inline bool fwd_pair_selected(int nq, int npairs, int head_dim, bool causal) {
+// FLASH_HOG_FWD = compiled or pair forces either kernel for fp32 (otherwise
+// fwd_pair_rule); read at every launch.
+inline bool fwd_pair_selected(Mask m, int npairs, int head_dim) {
   const char* v = std::getenv("FLASH_HOG_FWD");
   if (v != nullptr && std::strcmp(v, "pair") == 0) return true;
   if (v != nullptr && std::strcmp(v, "compiled") == 0) return false;
-  return (long)((nq + 63) / 64) * npairs <= (long)(!causal ? 1 : head_dim == 64 ? 4 : 3) * resident_workgroups(1);
+  return fwd_pair_rule(m, npairs, head_dim, resident_workgroups(1));
 }
 
 template <typename T, int D, bool CAUSAL>
@@ -249,7 +244,7 @@ hipError_t launch_fwd(const FwdParams<T>& p, hipStream_t stream) {
   } else {
     const int npairs = p.batch * p.heads;
     if constexpr (sizeof(T) == 4) {
-      if (fwd_pair_selected(p.nq, npairs, D, CAUSAL)) return launch_fwd_pair<T, D, CAUSAL>(p, stream);
+      if (fwd_pair_selected(mask_of(CAUSAL, p), npairs, D)) return launch_fwd_pair<T, D, CAUSAL>(p, stream);
     }
     const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
     const int chunk = grid_chunk(npairs, nqb, resident_workgroups(Occupancy<T, D>::value));

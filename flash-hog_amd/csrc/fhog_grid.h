@@ -1,0 +1,212 @@
+// Launch rules: which kernel a call takes and in which order a grid takes its
+// blocks, from the sizes, the mask and the number of compute units alone. Plain
+// C++ without HIP, so that the rules can be compiled and checked on the host.
+// Figures in the comments are from one MI355X (256 CUs).
+#pragma once
+
+namespace fhog {
+
+// Query i sees key j iff j <= i + coff (causal), or always. coff is 0 (top-left)
+// or nk - nq (bottom-right).
+struct Mask {
+  bool causal;
+  int nq, nk, coff;
+};
+
+// The chunk for grid_slot. A grid of at most 8 rounds of resident
+// workgroups keeps the rank-major order, whose last round holds the blocks
+// with the least work; a longer grid takes about one round per chunk (at
+// least 8 pairs, a multiple of 8), so that the streamed tiles of the pairs
+// in flight stay in L2 instead of being fetched again by every block.
+inline int grid_chunk(int npairs, int nranks, int resident) {
+  if (resident <= 0 || (long)npairs * nranks <= 8L * resident) return npairs;
+  const int c = resident / nranks / 8 * 8;
+  return c < 8 ? 8 : (c < npairs ? c : npairs);
+}
+
+// First rank that runs backwards (block nb - 1 - (rank - fold)) in a grid of nb
+// causal blocks, longest first, per (batch, head) pair. A grid of one to two
+// workgroups per CU runs as one round in which workgroups i and i + (number of
+// CUs) share a CU: the second of them take their ranks backwards, so that the
+// shortest blocks sit beside the longest. nb: none does.
+inline int fold_rank(bool causal, int nb, int npairs, int cus) {
+  const long grid = (long)nb * npairs;
+  return causal && cus > 0 && grid > cus && grid <= 2L * cus ? (cus + npairs - 1) / npairs : nb;
+}
+
+// The `pairs` argument of block_pair for a grid of nb causal blocks per
+// (batch, head) pair. Mirror pairs halve the number of workgroups and are taken
+// only where the paired grid fills whole rounds of the resident ones; elsewhere
+// the unpaired blocks, longest first, balance better (stage 2, us, paired /
+// unpaired: paired grids of 0.56 rounds, B3 N2048 H12, 125 / 96; 0.75, B1 N8192 H12,
+// 442 / 387; 1.5, B16 N1024 H12, 132 / 122; 2.25, B24 N1024 H12, 216 / 194). At two
+// workgroups per CU that is
+// - one round, skewed if nb allows (B4 N2048 H16 138 / 148, B1 N16384 H8 944 / 1021);
+// - more rounds of fewer than 8 blocks per pair (nb = 2, 6 rounds, B256 N256 H12
+//   270 / 277; 4, 2 rounds, B64 N512 H8 124 / 128; 5, 3 rounds, B8 N640 H64 173 / 175;
+//   but 8, 2 rounds, B16 N1024 H16 180 / 174; 16, 2 rounds, B8 N2048 H16 302 / 290; 256,
+//   2 rounds, B1 N32768 H8 3795 / 3720);
+// - one paired workgroup per CU, from 32 blocks per pair (64, B1 N8192 H8 309 / 320; 32,
+//   B4 N4096 H16 over 4 key heads 623 / 634; but 16, B4 N2048 H8 92.6 / 90.1).
+// At one workgroup per CU pairs are as good in any number of whole rounds.
+inline int block_pairing(Mask m, int nb, int npairs, int resident, int waves) {
+  const long paired = (long)((nb + 1) / 2) * npairs, single = (long)nb * npairs;
+  if (!m.causal || resident <= 0) return 0;
+  if (waves == 2 && nb >= 32 && single == resident && 2 * paired == resident) return 1;
+  if (single <= resident || paired % resident != 0) return 0;
+  if (waves == 2 && paired == resident && nb % 4 == 0) return 2;
+  return waves != 2 || paired == resident || nb < 8;
+}
+
+// The forward: fwd_pair_kernel (two waves per 32 queries, 64-query workgroups) serves
+// 2-byte types at D = 256, and fp32 while its grid has at most one workgroup per
+// CU, or four (D = 64) or three (D = 128) when causal; fp32's two kernels give the same
+// bits (us, fwd / pair: causal N2048 H8 D64 B2 (512 workgroups) 142 / 99, B4
+// (1024) 196 / 165, B4 H16 (2048) 287 / 312; non-causal B1 (256) 142 / 97, B2
+// (512) 144 / 157; D128 causal B3 (768) 273 / 237, B4 (1024) 300 / 309).
+inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
+  return (long)((m.nq + 63) / 64) * npairs <= (long)(!m.causal ? 1 : head_dim == 64 ? 4 : 3) * cus;
+}
+
+// The first backward for 2-byte types at D = 64 has several kernels for each
+// half of its work, all giving the same bits: dK/dV in bwd_k_kernel
+// (fhog_bwd.hip), in bwd_k64_kernel (fhog_bwd_k64.hip: 64 keys per wave at one wave
+// per SIMD, generated sweep) or in bwd_pair_kernel (fhog_bwd_pair.h: two waves per
+// 32 keys), dQ in bwd_q_kernel (fhog_bwd.hip), in bwd_q64_kernel (fhog_bwd_q64.hip,
+// 64 queries per wave) or in bwd_qpair_kernel (fhog_bwd_qpair.hip: two waves per 32
+// queries). First backward, us, at D = 64 bf16 unless named:
+//
+// The one-wave kernels (k64, q64) are the fastest per tile, but run one 256-row
+// block per CU at a time and gain nothing when a CU is left alone. They are taken
+// when their blocks cover little more than 128-row ones, in padding and, causal,
+// above the diagonal: up to 6 % more for dQ, 10 % for dK/dV (both one-wave / both
+// compiled: 6 % more, B8 N2048 H16 causal 280 / 297; 7 %, B20 N1700 H12 437 / 423;
+// 11 %, B64 N1000 H12 587 / 552; 20 %, B64 N600 H16 fp16 non-causal 559 / 501; 27 %,
+// B24 N1300 H12 391 / 317; dK/dV alone 8 %, B16 N1536 H16 357 / 363); and when their
+// grid fills whole rounds of the resident workgroups, or at least six (at B8 N2048
+// H12 causal, 1.5 rounds, q64 took 258 against 241). A causal dK/dV needs no whole
+// rounds: its key blocks, longest first, even out (first backward, compiled / k64:
+// 1.1 rounds, B3 N2048 H12, 108 / 105; 1.5, B2 N4096 H12, 216 / 208, B1 N8192 H12, 405 /
+// 387; 1.75, B7 N4096 H16 over 4 key heads, 958 / 869; 4.1, B11 N2048 H12, 326 / 320).
+//
+// The pair kernels do more LDS work per tile but take half the time per tile of
+// a wave, and their 64-row blocks spread a small grid over twice as many CUs and
+// waste less of a short causal sequence's diagonal. dK/dV takes its pair kernel
+// up to three workgroups per CU, and for causal sequences of up to 1024 keys
+// (others / pair: causal B1 N1024 H12 (192 workgroups) 52.4 / 45.0, B1 N4096 H12
+// (768) 184 / 163, B2 N4096 H16 over 4 key heads (512) 523 / 446, B128 N512 H12
+// 448 / 417, B24 N1024 H12 219 / 213, B32 N1024 H16 399 / 403, B4 N2048 H16 136 /
+// 151; non-causal B1 N2048 H16 (512) 95.2 / 92.9, B2 N2048 H12 (768) 120 / 117, B8
+// N1000 H12 fp16 (1536) 122.8 / 124.0). dQ gains less and takes its pair kernel,
+// at D = 64 and 128, up to one workgroup per CU (B1 N512 H12 27.0 / 26.1, B1
+// N2048 H8 D128 non-causal 118 / 109; B2 N1000 H12 fp16, 384 workgroups, 51.2 /
+// 55.7), and at D = 64 for causal sequences of up to 512 queries (B32 N512 H12
+// 106 / 99, B128 N256 H12 171 / 166; B32 N1024 H12 287 / 301).
+inline bool one_wave_grid(int workgroups, int resident) {
+  return resident > 0 && workgroups > 0 && (workgroups % resident == 0 || workgroups >= 6 * resident);
+}
+// Whether 256-row blocks of n rows cover at most `percent` of what 128-row ones
+// do (rows of the blocks times, when causal, the mean of what they see).
+inline bool one_wave_cover(int n, bool causal, int percent) {
+  const long b1 = ((long)n + 127) / 128, b2 = ((long)n + 255) / 256 * 2;
+  return 100 * b2 * (causal ? b2 + 2 : 1) <= percent * b1 * (causal ? b1 + 1 : 1);
+}
+// Whether the whole rounds of q64 or k64 are there (n: the blocked side).
+inline bool one_wave_rounds(Mask m, int n, int npairs, int cus) {
+  const int nb = (int)(((long)n + 255) / 256);
+  const bool mirrored = m.causal && (long)nb * npairs > cus;
+  return one_wave_grid((mirrored ? (nb + 1) / 2 : nb) * npairs, cus);
+}
+inline bool bwd_q64_rule(Mask m, int npairs, int cus) {
+  return one_wave_cover(m.nq, m.causal, 106) && one_wave_rounds(m, m.nq, npairs, cus);
+}
+inline bool bwd_k64_rule(Mask m, int npairs, int cus) {
+  return one_wave_cover(m.nk, m.causal, 110) && (m.causal || one_wave_rounds(m, m.nk, npairs, cus));
+}
+inline bool bwd_pair_rule(Mask m, int npairs, int cus) {
+  return (m.causal && m.nk <= 1024) || (long)((m.nk + 63) / 64) * npairs <= 3L * cus;
+}
+inline bool bwd_qpair_rule(Mask m, int npairs, int head_dim, int cus) {
+  return (m.causal && head_dim == 64 && m.nq <= 512) || (long)((m.nq + 63) / 64) * npairs <= cus;
+}
+
+// Waves per SIMD of bwd_pair_kernel. Three workgroups per CU at 256-byte rows (168
+// registers): for fp32 always (D = 64 B4 N2048 H16 1031 -> 1013 us, B2 N2048 H8
+// equal), for 2-byte D = 128 once the grid is long (two / three: 359 / 392 us at B2 N2048 H32 over 8 key
+// heads, 512 workgroups; 300 / 287 at B4 N2048 H16, 2048; 2040 / 1956 at B2
+// N8192 H16, 4096). 2-byte D = 64 likewise with four (117 registers; first
+// backward, two / four: causal B1 N4096 H12, 768 workgroups, 163 / 166, B2 N2048
+// H16, 1024, 105 / 99, B128 N512 H12 484 / 417; non-causal B2 N2048 H12, 768,
+// 146 / 117).
+inline int bwd_pair_waves(Mask m, int npairs, int head_dim, int bytes, int cus) {
+  const long grid = (long)((m.nk + 63) / 64) * npairs;
+  if (bytes == 4 && head_dim == 64) return 3;
+  if (bytes == 2 && head_dim == 128 && grid > 4L * cus) return 3;
+  if (bytes == 2 && head_dim == 64 && grid > (m.causal ? 3L : 2L) * cus) return 4;
+  return 2;
+}
+
+// Stage 1 for 2-byte types at D = 64 runs the kernel with 32 queries per
+// wave at one wave per SIMD, a hand-scheduled sweep and a persistent grid
+// (fhog_bwdbwd_q32.hip) but for causal sequences of up to 512, which run the fused
+// kernel (16 queries per wave, two waves per SIMD): its 64-query blocks take half
+// as long and waste less of the diagonal. Both give the same results to
+// rounding, so the choice looks at the sequence only, never at how many there are
+// (stage 1, us, q32 / fused: causal N256 H12 B1 21.5 / 11.9, B256 310 / 297; N512
+// B1 28.4 / 18.8, B16 64.7 / 52.6, B64 209 / 209, B128 418 / 425; N1024 B32 316 /
+// 330; non-causal N512 B16 fp16 74.6 / 85.7; B4 N2048 H16 causal 171 / 185).
+inline bool stage1_fused_rule(Mask m) { return m.causal && m.nq <= 512 && m.nk <= 512; }
+
+// Stage 1 for fp32 runs bwdbwd_q_kernel (fhog_bwdbwd.hip, one wave per 32 queries) on grids
+// that fill the chip and bwdbwd_qpair_kernel (fhog_bwdbwd_qpair.hip, two waves per
+// 32 queries, half the time per block and twice the workgroups) on smaller ones;
+// both give the same bits. The line is two of the latter's workgroups per CU
+// when causal, one otherwise (stage 1, us, q / qpair: causal D = 64 N2048 H8 B2
+// (512 workgroups) 887 / 631, B3 (768) 890 / 840-885, B4 (1024) 970 / 1093;
+// non-causal B1 (256) 902 / 626, B2 (512) 910 / 1021; D = 128 causal B2 (512)
+// 1620 / 1296, B4 (1024) 1783 / 2538, non-causal B1 (256) 1647 / 1255).
+inline bool stage1_qpair_rule(Mask m, int npairs, int cus) {
+  return (long)((m.nq + 63) / 64) * npairs <= (long)(m.causal ? 2 : 1) * cus;
+}
+
+// Stage 2 runs bwdbwd_pair_kernel (fhog_bwdbwd_pair.hip, two waves per 32 keys)
+// but for 2-byte types at D = 64 on grids that fill the chip, where
+// bwdbwd_k_kernel's one wave per 32 keys is faster; both give the same bits.
+// The pair kernel's grid has twice the workgroups of half the work each, and
+// is taken while it has at most three of them per CU when causal, one
+// otherwise (stage 2, us, k / pair: causal B1 N512 H12 24.8 / 20.2, B1 N2048
+// H12 (384 workgroups) 78.4 / 69.7, B2 N2048 H12 (768) 85.2 / 74.8, B2 N4096
+// H16 over 4 key heads (512) 575 / 511, but B2 N2048 H16 (1024) 93.3 / 95.8 and
+// B1 N8192 H12 (1536) 452 / 497; non-causal B1 N300 over one key head 51.9 /
+// 44.2, but B1 N2048 H12 (384) 79.6 / 82.4, B2 N1000 H12 fp16 43.9 / 48.0).
+inline bool stage2_pair_rule(Mask m, int npairs, int cus) {
+  return (long)((m.nk + 63) / 64) * npairs <= (long)(m.causal ? 3 : 1) * cus;
+}
+
+// Whether a causal grid deals its blocks one by one instead of folding them
+// (bwdbwd_q32_kernel; both give the same bits): when every block can have a CU of
+// its own, or when the folded items' rounds take over 8 % longer than the longest
+// block or an even share of all blocks (their keys vary linearly, from first to
+// last). Stage 1, us, folded / dealt: one round of blocks, B1 N512 H12 28.6 / 20.5,
+// B1 N1024 H12 41.8 / 33.7, B1 N2048 H12 67.5 / 62.0; estimated gain 12 %, B4 N1024
+// H12 46.0 / 44.6; 11 %, B24 N1024 H12 258 / 248; 33 %, B1 N8192 H12 650 / 518; 36 %,
+// B8 N1500 H12 fp16 218 / 176; 50 %, B3 N2048 H12 155 / 115; but 7 %, B40 N1024 H12
+// 414 / 422; 6 %, B2 N2048 H12 77.0 / 78.4; 3 %, B1 N4096 H12 141 / 149 (fewer CUs
+// run faster); none, B32 N1024 H12 324 / 332, B4 N2048 H16 182 / 183.
+inline bool q32_deal_rule(Mask m, int npairs, int cus) {
+  constexpr int kRows = 128;
+  const int nqb = (int)(((long)m.nq + kRows - 1) / kRows);
+  const long blocks = (long)npairs * nqb;
+  if (!m.causal) return false;
+  if (blocks <= cus) return true;
+  auto keys = [&](int qb) {
+    const long e = (long)(qb + 1) * kRows + m.coff;
+    return (double)(e < 0 ? 0 : e < m.nk ? e : m.nk);
+  };
+  const double first = keys(0), last = keys(nqb - 1);
+  const long rounds = ((long)npairs * ((nqb + 1) / 2) + cus - 1) / (cus > 0 ? cus : 1);
+  const double share = 0.5 * (first + last) * (double)blocks / cus;
+  return cus > 0 && (double)rounds * (first + last) > 1.08 * (last > share ? last : share);
+}
+
+}  // namespace fhog

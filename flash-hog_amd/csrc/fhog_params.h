@@ -16,6 +16,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "fhog_grid.h"
+
 namespace fhog {
 
 template <typename T> struct FwdParams {
@@ -56,6 +58,9 @@ __device__ inline int first_contributing_query(const BwdBwdParams<T>& p, int kj,
   if (p.nk == 1) return p.nq;
   return causal ? kj - p.coff + (kj == 0) : 0;
 }
+
+// What the launch rules look at.
+template <typename P> inline Mask mask_of(bool causal, const P& p) { return Mask{causal, p.nq, p.nk, p.coff}; }
 
 template <typename T, int D, bool CAUSAL> hipError_t launch_fwd(const FwdParams<T>& p, hipStream_t s);
 // The forward with two waves per 32 queries: 2-byte types at D = 256, and fp32 on

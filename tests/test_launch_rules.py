@@ -1,0 +1,120 @@
+"""The launch rules of csrc/fhog_grid.h, compiled for the host.
+
+The rules are plain C++: a few C wrappers around them are built with the host
+compiler and called here with the sizes of 256 CUs, so that a rule can be checked
+without a GPU. Each row names a call and the kernel or block order that was
+measured the faster one there; the times stand beside the rules.
+"""
+
+from __future__ import annotations
+
+import ctypes
+import pathlib
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = pathlib.Path(__file__).resolve().parent.parent / "flash-hog_amd" / "csrc"
+CUS = 256
+
+WRAPPERS = r"""
+#include "fhog_grid.h"
+using fhog::Mask;
+static Mask mask(int causal, int nq, int nk) { return Mask{causal != 0, nq, nk, causal == 2 ? nk - nq : 0}; }
+extern "C" {
+int fwd_pair(int c, int nq, int nk, int np, int d, int cus) { return fhog::fwd_pair_rule(mask(c, nq, nk), np, d, cus); }
+int bwd_pair(int c, int nq, int nk, int np, int cus) { return fhog::bwd_pair_rule(mask(c, nq, nk), np, cus); }
+int bwd_k64(int c, int nq, int nk, int np, int cus) { return fhog::bwd_k64_rule(mask(c, nq, nk), np, cus); }
+int bwd_qpair(int c, int nq, int nk, int np, int d, int cus) { return fhog::bwd_qpair_rule(mask(c, nq, nk), np, d, cus); }
+int bwd_q64(int c, int nq, int nk, int np, int cus) { return fhog::bwd_q64_rule(mask(c, nq, nk), np, cus); }
+int bwd_waves(int c, int nq, int nk, int np, int d, int bytes, int cus) {
+  return fhog::bwd_pair_waves(mask(c, nq, nk), np, d, bytes, cus);
+}
+int stage1_fused(int c, int nq, int nk) { return fhog::stage1_fused_rule(mask(c, nq, nk)); }
+int stage1_qpair(int c, int nq, int nk, int np, int cus) { return fhog::stage1_qpair_rule(mask(c, nq, nk), np, cus); }
+int stage2_pair(int c, int nq, int nk, int np, int cus) { return fhog::stage2_pair_rule(mask(c, nq, nk), np, cus); }
+int q32_deal(int c, int nq, int nk, int np, int cus) { return fhog::q32_deal_rule(mask(c, nq, nk), np, cus); }
+int pairing(int c, int nq, int nk, int nb, int np, int resident, int waves) {
+  return fhog::block_pairing(mask(c, nq, nk), nb, np, resident, waves);
+}
+int fold(int c, int nb, int np, int cus) { return fhog::fold_rank(c != 0, nb, np, cus); }
+int chunk(int np, int nranks, int resident) { return fhog::grid_chunk(np, nranks, resident); }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("c++") or shutil.which("clang++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cpp").write_text(WRAPPERS)
+    cmd = [cxx, "-std=c++20", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}", str(d / "rules.cpp"), "-o",
+           str(d / "rules.so")]
+    subprocess.run(cmd, check=True)
+    return ctypes.CDLL(str(d / "rules.so"))
+
+
+def dkdv(r, causal, nq, nk, npairs):
+    if r.bwd_pair(causal, nq, nk, npairs, CUS):
+        return "pair"
+    return "k64" if r.bwd_k64(causal, nq, nk, npairs, CUS) else "compiled"
+
+
+def dq(r, causal, nq, nk, npairs, head_dim=64):
+    if r.bwd_qpair(causal, nq, nk, npairs, head_dim, CUS):
+        return "pair"
+    return "q64" if r.bwd_q64(causal, nq, nk, npairs, CUS) else "compiled"
+
+
+def stage2_order(r, causal, nq, nk, npairs):
+    """`pairs` of bwdbwd_k_kernel: 128-key blocks, two workgroups per CU."""
+    return r.pairing(causal, nq, nk, (nk + 127) // 128, npairs, 2 * CUS, 2)
+
+
+def one_wave_order(r, causal, nq, nk, n, npairs):
+    """`pairs` of the kernels with 256-row blocks, one workgroup per CU."""
+    return r.pairing(causal, nq, nk, (n + 255) // 256, npairs, CUS, 1)
+
+
+# batch, length, heads (square, top-left causal): dK/dV, dQ, stage 2, its block order
+SQUARES = [
+    (1, 1024, 12, "pair", "pair", "pair", None),
+    (1, 4096, 12, "pair", "compiled", "pair", None),
+    (2, 2048, 12, "pair", "compiled", "pair", None),
+    (2, 2048, 16, "k64", "q64", "k", 0),
+    (4, 2048, 16, "k64", "q64", "k", 2),
+    (1, 16384, 8, "k64", "q64", "k", 2),
+    (8, 2048, 16, "k64", "q64", "k", 0),
+    (1, 32768, 8, "k64", "q64", "k", 0),
+    (1, 8192, 8, "k64", "q64", "k", 1),
+    (4, 2048, 8, "k64", "q64", "k", 0),
+    (3, 2048, 12, "k64", "compiled", "k", 0),
+]
+
+
+@pytest.mark.parametrize("row", SQUARES, ids=lambda r: "b%d_n%d_h%d" % r[:3])
+def test_squares(rules, row):
+    batch, n, heads, want_kv, want_q, want_2, order = row
+    np_ = batch * heads
+    assert dkdv(rules, 1, n, n, np_) == want_kv
+    assert dq(rules, 1, n, n, np_) == want_q
+    assert ("pair" if rules.stage2_pair(1, n, n, np_, CUS) else "k") == want_2
+    if order is not None:
+        assert stage2_order(rules, 1, n, n, np_) == order
+
+
+def test_folded_ranks_are_a_permutation(rules):
+    for nb in range(1, 70):
+        for npairs in (1, 3, 8, 12, 37, 64, 300):
+            f = rules.fold(1, nb, npairs, CUS)
+            assert sorted(r if r < f else nb - 1 - (r - f) for r in range(nb)) == list(range(nb))
+
+
+def test_chunks_cover_every_pair(rules):
+    for npairs in (1, 7, 64, 500, 5000):
+        for nranks in (1, 2, 9, 64, 700):
+            for resident in (0, CUS, 2 * CUS):
+                assert 1 <= rules.chunk(npairs, nranks, resident) <= max(npairs, 8)
