@@ -59,7 +59,7 @@ __device__ __forceinline__ const void* uni(const void* x) {
 // A workgroup's share of the grid. The grid is persistent (at most one
 // workgroup per CU, the most that fit at one wave per SIMD) and walks a list
 // of items. Without a mask an item is one query block. With a causal mask there
-// are two lists (`deal`):
+// are two lists, each with an instance of its own (DEAL):
 // - Folded: item r of a (batch, head) pair is the query block of rank r (nqb - 1
 //   - r, the longest rows first) followed by the block of rank nqb - 1 - r, so
 //   every item but a middle one holds the same number of key tiles.
@@ -76,9 +76,10 @@ struct Q32Walk {
   int item, half;  // half: second block of a folded item, or the round of a dealt one
 };
 
-template <typename T, bool CAUSAL, bool PRE>
+template <typename T, bool CAUSAL, bool PRE, bool DEAL>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
-bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems, int deal) {
+bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems) {
+  static_assert(CAUSAL || !DEAL, "without a mask there is one list");
   constexpr int D = 64;
   typedef SwzTile<T, D> G;
   constexpr int KS = D / 16;       // 16-deep steps over the head dim
@@ -102,7 +103,7 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems, int deal) {
   const int ngrid = (int)gridDim.x;
   const int w = (int)blockIdx.x;
   const int npairs = p.batch * p.heads;
-  Q32Walk walk{!(CAUSAL && deal) && ngrid % 8 == 0 ? (w % 8) * (ngrid / 8) + w / 8 : w, 0};
+  Q32Walk walk{!DEAL && ngrid % 8 == 0 ? (w % 8) * (ngrid / 8) + w / 8 : w, 0};
   if (walk.item >= nitems) return;
   const long rs = (long)p.heads * D;      // query-side row stride
   const long rsk = (long)p.kv_heads * D;  // key-side row stride
@@ -131,9 +132,8 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems, int deal) {
   };
   auto block_of = [&](Q32Walk it) {
     Blk k;
-    const bool dealt = CAUSAL && deal;
-    const int bh = dealt ? it.item % npairs : it.item / npr, r = dealt ? it.item / npairs : it.item % npr;
-    const int rank = CAUSAL && !deal && it.half ? nqb - 1 - r : r;
+    const int bh = DEAL ? it.item % npairs : it.item / npr, r = DEAL ? it.item / npairs : it.item % npr;
+    const int rank = CAUSAL && !DEAL && it.half ? nqb - 1 - r : r;
     const int qb = CAUSAL ? nqb - 1 - rank : rank;  // causal: rank 0 is the last block
     const int b = bh / p.heads, h = bh % p.heads;
     const int hk = h / (p.heads / p.kv_heads);
@@ -164,7 +164,7 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems, int deal) {
   };
   // The item after `it` in this workgroup's list.
   auto next_of = [&](Q32Walk it) {
-    if (CAUSAL && deal) {
+    if constexpr (DEAL) {
       const int round = it.half + 1;
       const int rev = ngrid % 8 == 0 ? (ngrid / 8 - 1 - w / 8) * 8 + w % 8 : ngrid - 1 - w;
       return Q32Walk{round * ngrid + (round & 1 ? rev : w), round};
@@ -420,21 +420,28 @@ bwdbwd_q32_kernel(BwdBwdParams<T> p, int nitems, int deal) {
 
 }  // namespace
 
+template <typename T, bool CAUSAL, bool DEAL>
+hipError_t launch_list(const BwdBwdParams<T>& p, int nitems, int resident, hipStream_t stream) {
+  const dim3 grid(resident > 0 && resident < nitems ? resident : nitems);
+  int e2;
+  constexpr bool kPre = std::is_same_v<T, __bf16>;
+  if (kPre && std::frexp(p.scale, &e2) == 0.5f)  // scale = 2^(e2 - 1)
+    hipLaunchKernelGGL((bwdbwd_q32_kernel<T, CAUSAL, kPre, DEAL>), grid, dim3(kThreads), 0, stream, p, nitems);
+  else
+    hipLaunchKernelGGL((bwdbwd_q32_kernel<T, CAUSAL, false, DEAL>), grid, dim3(kThreads), 0, stream, p, nitems);
+  return hipGetLastError();
+}
+
 template <typename T, bool CAUSAL>
 hipError_t launch_bwdbwd_stage1_q32(const BwdBwdParams<T>& p, hipStream_t stream) {
   const int nqb = (p.nq + 32 * kWaves - 1) / (32 * kWaves);
   const int npairs = p.batch * p.heads;
   const int resident = resident_workgroups(1);
-  const int deal = q32_deal_rule(mask_of(CAUSAL, p), npairs, resident);
-  const int nitems = npairs * (CAUSAL && !deal ? (nqb + 1) / 2 : nqb);
-  const dim3 grid(resident > 0 && resident < nitems ? resident : nitems);
-  int e2;
-  if (std::is_same_v<T, __bf16> && std::frexp(p.scale, &e2) == 0.5f)  // scale = 2^(e2 - 1)
-    hipLaunchKernelGGL((bwdbwd_q32_kernel<T, CAUSAL, std::is_same_v<T, __bf16>>), grid, dim3(kThreads), 0, stream, p,
-                       nitems, deal);
-  else
-    hipLaunchKernelGGL((bwdbwd_q32_kernel<T, CAUSAL, false>), grid, dim3(kThreads), 0, stream, p, nitems, deal);
-  return hipGetLastError();
+  if constexpr (CAUSAL) {
+    if (q32_deal_rule(mask_of(CAUSAL, p), npairs, resident))
+      return launch_list<T, CAUSAL, true>(p, npairs * nqb, resident, stream);
+  }
+  return launch_list<T, CAUSAL, false>(p, npairs * (CAUSAL ? (nqb + 1) / 2 : nqb), resident, stream);
 }
 
 #define FHOG_INST(T, C) template hipError_t launch_bwdbwd_stage1_q32<T, C>(const BwdBwdParams<T>&, hipStream_t);
