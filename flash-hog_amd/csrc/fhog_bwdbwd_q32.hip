@@ -25,8 +25,8 @@
 // matrix instruction at one wave per SIMD: 85 % of the pipe.)
 //
 // The default stage 1 for 2-byte types at D = 64: 177-180 us at B4 N2048 H16
-// causal bf16 against 184-189 us for the fused kernel. Causal sequences of
-// up to 512 run that one (launch_bwdbwd).
+// causal bf16 against 184-189 us for the fused kernel. Short causal
+// problems run that one (stage1_fused_rule).
 //
 // Layouts (32x32x16, see fhog_device.h): score tiles are transposed,
 // S^T = K Q^T, so lane n of a wave holds query q0 + n and register r key

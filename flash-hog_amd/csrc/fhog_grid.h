@@ -13,6 +13,35 @@ struct Mask {
   int nq, nk, coff;
 };
 
+// The sum over blocks of `rows` rows of what a block sees on the other side:
+// key-tiled, the queries from its first key's diagonal on; query-tiled, the keys up
+// to its last row's diagonal. Times `rows` that is the pairs the blocks cover, masked
+// ones included.
+inline long blocks_see(Mask m, int rows, bool key_tiled) {
+  const long n = key_tiled ? m.nk : m.nq, other = key_tiled ? m.nq : m.nk, nb = (n + rows - 1) / rows;
+  if (!m.causal) return nb * other;
+  // block i (from the last key, or from the first query) sees clamp(a + i rows, 0, other)
+  const long a = key_tiled ? other + m.coff - (nb - 1) * rows : rows + (long)m.coff;
+  auto blocks_below = [&](long x) {  // how many blocks have a + i rows < x
+    const long c = x > a ? (x - a + rows - 1) / rows : 0;
+    return c < nb ? c : nb;
+  };
+  const long lo = blocks_below(1), hi = blocks_below(other);
+  const long mid = hi > lo ? hi - lo : 0;
+  return mid * a + rows * (mid * (lo + hi - 1) / 2) + (nb - (hi > lo ? hi : lo)) * other;
+}
+
+// How much of a causal problem is a rectangle that the diagonal does not touch: the
+// queries past the last key (top-left, nq > nk) or the keys before the first
+// diagonal (bottom-right, nk > nq). Blocks differ in length only in the rest, so the
+// larger this part, the more a causal grid behaves like one without a mask. True
+// where it is at most 1 / parts of the shorter side.
+inline bool near_square(Mask m, int parts) {
+  const long coff = m.coff, over = m.nq - m.nk + coff;
+  const long rect = over > coff ? over : coff, side = m.nq < m.nk ? m.nq : m.nk;
+  return m.causal && parts * rect <= side;
+}
+
 // The chunk for grid_slot. A grid of at most 8 rounds of resident
 // workgroups keeps the rank-major order, whose last round holds the blocks
 // with the least work; a longer grid takes about one round per chunk (at
@@ -146,16 +175,24 @@ inline int bwd_pair_waves(Mask m, int npairs, int head_dim, int bytes, int cus) 
   return 2;
 }
 
-// Stage 1 for 2-byte types at D = 64 runs the kernel with 32 queries per
-// wave at one wave per SIMD, a hand-scheduled sweep and a persistent grid
-// (fhog_bwdbwd_q32.hip) but for causal sequences of up to 512, which run the fused
-// kernel (16 queries per wave, two waves per SIMD): its 64-query blocks take half
-// as long and waste less of the diagonal. Both give the same results to
-// rounding, so the choice looks at the sequence only, never at how many there are
-// (stage 1, us, q32 / fused: causal N256 H12 B1 21.5 / 11.9, B256 310 / 297; N512
-// B1 28.4 / 18.8, B16 64.7 / 52.6, B64 209 / 209, B128 418 / 425; N1024 B32 316 /
-// 330; non-causal N512 B16 fp16 74.6 / 85.7; B4 N2048 H16 causal 171 / 185).
-inline bool stage1_fused_rule(Mask m) { return m.causal && m.nq <= 512 && m.nk <= 512; }
+// Stage 1 for 2-byte types at D = 64 runs the kernel with 32 queries per wave at one
+// wave per SIMD, a hand-scheduled sweep, a persistent grid and 128-query blocks
+// (fhog_bwdbwd_q32.hip) but for short causal problems, where the fused kernel's
+// 64-query blocks (16 queries per wave, two waves per SIMD) take half as long and
+// cover less of what the mask or the last row cuts off. Both give the same results
+// to rounding, so the choice looks at the lengths only, never at how many sequences
+// there are: up to 512 on both sides, where 128-query blocks cover 12 % more than
+// 64-query ones, or 15 % where the diagonal is not most of the problem.
+// Stage 1, us, q32 / fused, H12 bf16: 36 % more (N448) B128 410 / 355; 28 % (400
+// queries, 500 keys bottom-right, H8) B16 45.6 / 40.4; 20 % (N256) B256 322 / 314; 14 %
+// (N384) B64 148 / 147; but 11 % (N512) B128 427 / 433, B32 103 / 105, though B16 55.6 /
+// 53.8 and B1 20.3 / 18.7. Rectangles: 14 % (256 queries, 128 keys) B128 125 / 132; 8 %
+// (256 queries, 512 keys bottom-right) B64 140 / 146; 7 % (512 queries, 128 keys) B128
+// 239 / 258. Non-causal N512 B16 fp16 74.6 / 85.7; B4 N2048 H16 causal 177 / 190.
+inline bool stage1_fused_rule(Mask m) {
+  if (!m.causal || m.nq > 512 || m.nk > 512) return false;
+  return 100 * 2 * blocks_see(m, 128, false) >= (near_square(m, 16) ? 112 : 115) * blocks_see(m, 64, false);
+}
 
 // Stage 1 for fp32 runs bwdbwd_q_kernel (fhog_bwdbwd.hip, one wave per 32 queries) on grids
 // that fill the chip and bwdbwd_qpair_kernel (fhog_bwdbwd_qpair.hip, two waves per

@@ -1,6 +1,6 @@
 """The 32-query stage 1 at D = 64 (fhog_bwdbwd_q32.hip) on every small case.
 
-Causal sequences of up to 512 run the fused kernel by default (launch_bwdbwd), so
+Short causal problems run the fused kernel by default (stage1_fused_rule), so
 the small causal cases of the parity, scale, single-key and random-sweep suites
 would not reach the 32-query kernel; here they run again with
 FLASH_HOG_STAGE1=q32, at the same tolerances.

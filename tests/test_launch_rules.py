@@ -38,6 +38,8 @@ int q32_deal(int c, int nq, int nk, int np, int cus) { return fhog::q32_deal_rul
 int pairing(int c, int nq, int nk, int nb, int np, int resident, int waves) {
   return fhog::block_pairing(mask(c, nq, nk), nb, np, resident, waves);
 }
+long sees(int c, int nq, int nk, int rows, int keys) { return fhog::blocks_see(mask(c, nq, nk), rows, keys != 0); }
+int near_square(int c, int nq, int nk, int parts) { return fhog::near_square(mask(c, nq, nk), parts); }
 int fold(int c, int nb, int np, int cus) { return fhog::fold_rank(c != 0, nb, np, cus); }
 int chunk(int np, int nranks, int resident) { return fhog::grid_chunk(np, nranks, resident); }
 }
@@ -54,7 +56,9 @@ def rules(tmp_path_factory):
     cmd = [cxx, "-std=c++20", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}", str(d / "rules.cpp"), "-o",
            str(d / "rules.so")]
     subprocess.run(cmd, check=True)
-    return ctypes.CDLL(str(d / "rules.so"))
+    lib = ctypes.CDLL(str(d / "rules.so"))
+    lib.sees.restype = ctypes.c_long
+    return lib
 
 
 def dkdv(r, causal, nq, nk, npairs):
@@ -118,3 +122,47 @@ def test_chunks_cover_every_pair(rules):
         for nranks in (1, 2, 9, 64, 700):
             for resident in (0, CUS, 2 * CUS):
                 assert 1 <= rules.chunk(npairs, nranks, resident) <= max(npairs, 8)
+
+
+def test_blocks_see(rules):
+    """blocks_see against a count block by block."""
+    lengths = (1, 31, 64, 65, 127, 128, 200, 256, 384, 500, 512, 1000)
+    for nq in lengths:
+        for nk in lengths:
+            for causal in (0, 1, 2):
+                coff = nk - nq if causal == 2 else 0
+                for rows in (64, 128, 256):
+                    if causal:
+                        by_query = [min(nk, max(0, q0 + rows + coff)) for q0 in range(0, nq, rows)]
+                        by_key = [nq - min(nq, max(0, k0 - coff)) for k0 in range(0, nk, rows)]
+                    else:
+                        by_query, by_key = [nk] * -(-nq // rows), [nq] * -(-nk // rows)
+                    assert rules.sees(causal, nq, nk, rows, 0) == sum(by_query), (causal, nq, nk, rows)
+                    assert rules.sees(causal, nq, nk, rows, 1) == sum(by_key), (causal, nq, nk, rows)
+
+
+def test_near_square(rules):
+    for parts in (3, 4, 16):
+        assert rules.near_square(1, 700, 700, parts) and rules.near_square(2, 700, 700, parts)
+        assert rules.near_square(1, 300, 5000, parts)  # top-left: keys past the last query are seen by none
+        assert rules.near_square(2, 5000, 300, parts)  # bottom-right: the first queries see nothing
+        assert rules.near_square(1, 480 + 480 // parts, 480, parts)
+        assert not rules.near_square(1, 481 + 480 // parts, 480, parts)
+        assert not rules.near_square(2, 480, 481 + 480 // parts, parts)
+        assert not rules.near_square(0, 700, 700, parts)
+
+
+# n_q, n_k, causal, whether stage 1 at D = 64 takes the fused kernel
+STAGE1 = [
+    (256, 256, 1, True), (384, 384, 1, True), (448, 448, 1, True), (1, 1, 1, True), (448, 512, 2, True),
+    (400, 500, 2, True), (32, 512, 2, True), (200, 512, 1, True), (512, 200, 2, True),
+    (512, 512, 1, False), (500, 500, 1, False), (513, 513, 1, False), (256, 512, 2, False), (128, 512, 2, False),
+    (512, 128, 1, False), (512, 256, 1, False), (512, 448, 1, False), (256, 128, 1, False), (384, 512, 2, False),
+    (256, 256, 0, False), (64, 600, 2, False),
+]
+
+
+@pytest.mark.parametrize("row", STAGE1, ids=str)
+def test_stage1_fused(rules, row):
+    nq, nk, causal, want = row
+    assert bool(rules.stage1_fused(causal, nq, nk)) == want
