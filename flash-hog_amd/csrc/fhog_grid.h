@@ -129,8 +129,10 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 // N1000 H12 fp16 (1536) 122.8 / 124.0). dQ gains less and takes its pair kernel,
 // at D = 64 and 128, up to one workgroup per CU (B1 N512 H12 27.0 / 26.1, B1
 // N2048 H8 D128 non-causal 118 / 109; B2 N1000 H12 fp16, 384 workgroups, 51.2 /
-// 55.7), and at D = 64 for causal sequences of up to 512 queries (B32 N512 H12
-// 106 / 99, B128 N256 H12 171 / 166; B32 N1024 H12 287 / 301).
+// 55.7). Short causal sequences gain nothing on fuller grids (compiled / pair: B128 N256
+// H12 168 / 166, B128 N384 H12 292 / 296, B32 N512 H12 101 / 99, B128 N512 H12 408 / 423, over
+// 4 key heads 442 / 467), and a chunk of queries against more keys loses (512 queries
+// of 1024 keys bottom-right B64 H12 409 / 448, of 4096 B32 877 / 1036).
 inline bool one_wave_grid(int workgroups, int resident) {
   return resident > 0 && workgroups > 0 && (workgroups % resident == 0 || workgroups >= 6 * resident);
 }
@@ -155,9 +157,7 @@ inline bool bwd_k64_rule(Mask m, int npairs, int cus) {
 inline bool bwd_pair_rule(Mask m, int npairs, int cus) {
   return (m.causal && m.nk <= 1024) || (long)((m.nk + 63) / 64) * npairs <= 3L * cus;
 }
-inline bool bwd_qpair_rule(Mask m, int npairs, int head_dim, int cus) {
-  return (m.causal && head_dim == 64 && m.nq <= 512) || (long)((m.nq + 63) / 64) * npairs <= cus;
-}
+inline bool bwd_qpair_rule(Mask m, int npairs, int cus) { return (long)((m.nq + 63) / 64) * npairs <= cus; }
 
 // Waves per SIMD of bwd_pair_kernel. Three workgroups per CU at 256-byte rows (168
 // registers): for fp32 always (D = 64 B4 N2048 H16 1031 -> 1013 us, B2 N2048 H8

@@ -26,7 +26,7 @@ extern "C" {
 int fwd_pair(int c, int nq, int nk, int np, int d, int cus) { return fhog::fwd_pair_rule(mask(c, nq, nk), np, d, cus); }
 int bwd_pair(int c, int nq, int nk, int np, int cus) { return fhog::bwd_pair_rule(mask(c, nq, nk), np, cus); }
 int bwd_k64(int c, int nq, int nk, int np, int cus) { return fhog::bwd_k64_rule(mask(c, nq, nk), np, cus); }
-int bwd_qpair(int c, int nq, int nk, int np, int d, int cus) { return fhog::bwd_qpair_rule(mask(c, nq, nk), np, d, cus); }
+int bwd_qpair(int c, int nq, int nk, int np, int cus) { return fhog::bwd_qpair_rule(mask(c, nq, nk), np, cus); }
 int bwd_q64(int c, int nq, int nk, int np, int cus) { return fhog::bwd_q64_rule(mask(c, nq, nk), np, cus); }
 int bwd_waves(int c, int nq, int nk, int np, int d, int bytes, int cus) {
   return fhog::bwd_pair_waves(mask(c, nq, nk), np, d, bytes, cus);
@@ -67,8 +67,8 @@ def dkdv(r, causal, nq, nk, npairs):
     return "k64" if r.bwd_k64(causal, nq, nk, npairs, CUS) else "compiled"
 
 
-def dq(r, causal, nq, nk, npairs, head_dim=64):
-    if r.bwd_qpair(causal, nq, nk, npairs, head_dim, CUS):
+def dq(r, causal, nq, nk, npairs):
+    if r.bwd_qpair(causal, nq, nk, npairs, CUS):
         return "pair"
     return "q64" if r.bwd_q64(causal, nq, nk, npairs, CUS) else "compiled"
 
@@ -166,3 +166,17 @@ STAGE1 = [
 def test_stage1_fused(rules, row):
     nq, nk, causal, want = row
     assert bool(rules.stage1_fused(causal, nq, nk)) == want
+
+
+# batch, n_q, n_k, heads, causal: the dQ kernel
+DQ = [
+    (64, 512, 1024, 12, 2, "compiled"), (32, 512, 4096, 12, 2, "compiled"),
+    (64, 512, 640, 12, 2, "compiled"), (64, 256, 512, 12, 2, "compiled"), (128, 512, 512, 12, 1, "compiled"),
+    (1, 512, 512, 12, 1, "pair"), (2, 512, 4096, 12, 2, "pair"),
+]
+
+
+@pytest.mark.parametrize("row", DQ, ids=str)
+def test_dq(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert dq(rules, causal, nq, nk, batch * heads) == want
