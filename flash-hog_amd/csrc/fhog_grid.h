@@ -108,10 +108,14 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 // The one-wave kernels (k64, q64) are the fastest per tile, but run one 256-row
 // block per CU at a time and gain nothing when a CU is left alone. They are taken
 // when their blocks cover little more than 128-row ones, in padding and, causal,
-// above the diagonal: up to 6 % more for dQ, 10 % for dK/dV (both one-wave / both
-// compiled: 6 % more, B8 N2048 H16 causal 280 / 297; 7 %, B20 N1700 H12 437 / 423;
-// 11 %, B64 N1000 H12 587 / 552; 20 %, B64 N600 H16 fp16 non-causal 559 / 501; 27 %,
-// B24 N1300 H12 391 / 317; dK/dV alone 8 %, B16 N1536 H16 357 / 363); and when their
+// past the diagonal: up to 6 % more for dQ, 10 % for dK/dV (first backward, us, causal
+// bf16, one-wave / compiled for dQ: 6 % more, B8 N2048 H16 280 / 297 with both halves;
+// 8 %, B8 N4736 H12 977 / 977; 11 %, B8 N3200 H12 506 / 503; 16 %, B32 N2117 H16 fp16 1446 /
+// 1386; 23 %, B24 N1300 H12 348 / 319; 24 %, B32 N1408 H16 681 / 633; for dK/dV: 4 %, B8
+// N3200 H12 472 / 492; 6 %, B32 N2117 H16 fp16 1324 / 1369; 7 %, B20 N1700 H12 413 / 421;
+// 9 %, B32 N1408 H16 624 / 629, B24 N1300 H12 320 / 316; 11 %, B64 N1030 H12 616 / 609;
+// rectangles: 8 %, 1280 queries of 1024 keys B32 H12 364 / 377; 4 %, 2048 of 1024 626 /
+// 690); and when their
 // grid fills whole rounds of the resident workgroups, or at least six (at B8 N2048
 // H12 causal, 1.5 rounds, q64 took 258 against 241). A causal dK/dV needs no whole
 // rounds: its key blocks, longest first, even out (first backward, compiled / k64:
@@ -136,11 +140,9 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 inline bool one_wave_grid(int workgroups, int resident) {
   return resident > 0 && workgroups > 0 && (workgroups % resident == 0 || workgroups >= 6 * resident);
 }
-// Whether 256-row blocks of n rows cover at most `percent` of what 128-row ones
-// do (rows of the blocks times, when causal, the mean of what they see).
-inline bool one_wave_cover(int n, bool causal, int percent) {
-  const long b1 = ((long)n + 127) / 128, b2 = ((long)n + 255) / 256 * 2;
-  return 100 * b2 * (causal ? b2 + 2 : 1) <= percent * b1 * (causal ? b1 + 1 : 1);
+// Whether 256-row blocks cover at most `percent` of what 128-row ones do.
+inline bool one_wave_cover(Mask m, bool key_tiled, int percent) {
+  return 100 * 2 * blocks_see(m, 256, key_tiled) <= percent * blocks_see(m, 128, key_tiled);
 }
 // Whether the whole rounds of q64 or k64 are there (n: the blocked side).
 inline bool one_wave_rounds(Mask m, int n, int npairs, int cus) {
@@ -149,10 +151,10 @@ inline bool one_wave_rounds(Mask m, int n, int npairs, int cus) {
   return one_wave_grid((mirrored ? (nb + 1) / 2 : nb) * npairs, cus);
 }
 inline bool bwd_q64_rule(Mask m, int npairs, int cus) {
-  return one_wave_cover(m.nq, m.causal, 106) && one_wave_rounds(m, m.nq, npairs, cus);
+  return one_wave_cover(m, false, 106) && one_wave_rounds(m, m.nq, npairs, cus);
 }
 inline bool bwd_k64_rule(Mask m, int npairs, int cus) {
-  return one_wave_cover(m.nk, m.causal, 110) && (m.causal || one_wave_rounds(m, m.nk, npairs, cus));
+  return one_wave_cover(m, true, 110) && (m.causal || one_wave_rounds(m, m.nk, npairs, cus));
 }
 inline bool bwd_pair_rule(Mask m, int npairs, int cus) {
   return (m.causal && m.nk <= 1024) || (long)((m.nk + 63) / 64) * npairs <= 3L * cus;

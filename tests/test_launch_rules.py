@@ -171,6 +171,7 @@ def test_stage1_fused(rules, row):
 # batch, n_q, n_k, heads, causal: the dQ kernel
 DQ = [
     (64, 512, 1024, 12, 2, "compiled"), (32, 512, 4096, 12, 2, "compiled"),
+    (8, 512, 8192, 16, 2, "q64"),
     (64, 512, 640, 12, 2, "compiled"), (64, 256, 512, 12, 2, "compiled"), (128, 512, 512, 12, 1, "compiled"),
     (1, 512, 512, 12, 1, "pair"), (2, 512, 4096, 12, 2, "pair"),
 ]
@@ -180,3 +181,18 @@ DQ = [
 def test_dq(rules, row):
     batch, nq, nk, heads, causal, want = row
     assert dq(rules, causal, nq, nk, batch * heads) == want
+
+
+# batch, n_q, n_k, heads, causal: whether dK/dV's 256-row kernel may run
+K64 = [
+    (32, 2117, 2117, 16, 1, True), (8, 3200, 3200, 12, 1, True), (4, 4096, 1024, 12, 1, True),
+    (32, 2048, 1024, 12, 1, True), (32, 1280, 1024, 12, 1, True), (2, 8192, 4096, 12, 1, True),
+    (64, 1030, 1030, 12, 1, False), (64, 1000, 1000, 12, 1, False), (64, 512, 256, 16, 1, False),
+    (64, 600, 600, 16, 0, False), (8, 2048, 2048, 10, 0, False), (8, 2048, 2048, 16, 0, True),
+]
+
+
+@pytest.mark.parametrize("row", K64, ids=str)
+def test_k64(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert bool(rules.bwd_k64(causal, nq, nk, batch * heads, CUS)) == want
