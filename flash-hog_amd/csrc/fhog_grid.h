@@ -125,12 +125,16 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 // The pair kernels do more LDS work per tile but take half the time per tile of
 // a wave, and their 64-row blocks spread a small grid over twice as many CUs and
 // waste less of a short causal sequence's diagonal. dK/dV takes its pair kernel
-// up to three workgroups per CU, and for causal sequences of up to 1024 keys
+// up to three workgroups per CU, and on fuller grids for causal problems of up to
+// 1024 keys whose diagonal shows: where 128-key blocks cover 6 % more than 64-key ones
 // (others / pair: causal B1 N1024 H12 (192 workgroups) 52.4 / 45.0, B1 N4096 H12
 // (768) 184 / 163, B2 N4096 H16 over 4 key heads (512) 523 / 446, B128 N512 H12
 // 448 / 417, B24 N1024 H12 219 / 213, B32 N1024 H16 399 / 403, B4 N2048 H16 136 /
-// 151; non-causal B1 N2048 H16 (512) 95.2 / 92.9, B2 N2048 H12 (768) 120 / 117, B8
-// N1000 H12 fp16 (1536) 122.8 / 124.0). dQ gains less and takes its pair kernel,
+// 151; rectangles: 7 % more, 400 queries of 600 keys bottom-right B64 H12 fp16 250 / 244,
+// 128 of 512 B64 113 / 107; 6 %, 768 queries of 512 keys B64 305 / 313; 5 %, 768 of 1024
+// bottom-right B32 250 / 254; 4 %, 1280 of 1024 364 / 385, 1024 of 512 B32 H16 269 / 284; 2 %,
+// 8192 of 1024 B8 H16 923 / 1100; non-causal B1 N2048 H16 (512) 95.2 / 92.9, B2 N2048
+// H12 (768) 120 / 117, B8 N1000 H12 fp16 (1536) 122.8 / 124.0). dQ gains less and takes its pair kernel,
 // at D = 64 and 128, up to one workgroup per CU (B1 N512 H12 27.0 / 26.1, B1
 // N2048 H8 D128 non-causal 118 / 109; B2 N1000 H12 fp16, 384 workgroups, 51.2 /
 // 55.7). Short causal sequences gain nothing on fuller grids (compiled / pair: B128 N256
@@ -157,7 +161,9 @@ inline bool bwd_k64_rule(Mask m, int npairs, int cus) {
   return one_wave_cover(m, true, 110) && (m.causal || one_wave_rounds(m, m.nk, npairs, cus));
 }
 inline bool bwd_pair_rule(Mask m, int npairs, int cus) {
-  return (m.causal && m.nk <= 1024) || (long)((m.nk + 63) / 64) * npairs <= 3L * cus;
+  if ((long)((m.nk + 63) / 64) * npairs <= 3L * cus) return true;
+  if (!m.causal || m.nk > 1024) return false;
+  return 1000 * 2 * blocks_see(m, 128, true) >= (near_square(m, 16) ? 1058 : 1065) * blocks_see(m, 64, true);
 }
 inline bool bwd_qpair_rule(Mask m, int npairs, int cus) { return (long)((m.nq + 63) / 64) * npairs <= cus; }
 

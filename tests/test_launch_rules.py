@@ -196,3 +196,25 @@ K64 = [
 def test_k64(rules, row):
     batch, nq, nk, heads, causal, want = row
     assert bool(rules.bwd_k64(causal, nq, nk, batch * heads, CUS)) == want
+
+
+# batch, n_q, n_k, heads, causal: the dK/dV kernel
+DKDV = [
+    (8, 8192, 1024, 16, 1, "k64"), (16, 4096, 512, 16, 1, "k64"),
+    (32, 1280, 1024, 12, 1, "k64"), (32, 1024, 512, 16, 1, "k64"), (32, 768, 1024, 12, 2, "k64"),
+    (64, 768, 512, 12, 1, "compiled"), (64, 400, 600, 12, 2, "pair"), (64, 256, 512, 12, 2, "pair"),
+    (32, 2048, 512, 12, 2, "pair"), (128, 512, 512, 12, 1, "pair"), (32, 1024, 1024, 16, 1, "pair"),
+    (64, 1000, 1000, 12, 1, "pair"), (32, 1100, 1100, 16, 1, "compiled"),
+]
+
+
+@pytest.mark.parametrize("row", DKDV, ids=str)
+def test_dkdv(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert dkdv(rules, causal, nq, nk, batch * heads) == want
+
+
+def test_dkdv_short_squares(rules):
+    """Square causal problems of up to 1024 tokens run the pair kernel on any grid."""
+    for n in range(1, 1025):
+        assert rules.bwd_pair(1, n, n, 4000, CUS) and rules.bwd_pair(2, n, n, 4000, CUS), n
