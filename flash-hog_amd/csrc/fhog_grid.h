@@ -174,12 +174,13 @@ inline bool bwd_qpair_rule(Mask m, int npairs, int cus) { return (long)((m.nq + 
 // N8192 H16, 4096). 2-byte D = 64 likewise with four (117 registers; first
 // backward, two / four: causal B1 N4096 H12, 768 workgroups, 163 / 166, B2 N2048
 // H16, 1024, 105 / 99, B128 N512 H12 484 / 417; non-causal B2 N2048 H12, 768,
-// 146 / 117).
+// 146 / 117; 768 workgroups of rectangles: 2560 queries of 2048 keys B2 H12 113 / 105,
+// 2304 of 2048 98.0 / 97.1, 4096 of 2048 219 / 181, 1024 of 2048 bottom-right 79.5 / 70.0).
 inline int bwd_pair_waves(Mask m, int npairs, int head_dim, int bytes, int cus) {
   const long grid = (long)((m.nk + 63) / 64) * npairs;
   if (bytes == 4 && head_dim == 64) return 3;
   if (bytes == 2 && head_dim == 128 && grid > 4L * cus) return 3;
-  if (bytes == 2 && head_dim == 64 && grid > (m.causal ? 3L : 2L) * cus) return 4;
+  if (bytes == 2 && head_dim == 64 && grid > (near_square(m, 16) ? 3L : 2L) * cus) return 4;
   return 2;
 }
 

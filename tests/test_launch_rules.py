@@ -218,3 +218,17 @@ def test_dkdv_short_squares(rules):
     """Square causal problems of up to 1024 tokens run the pair kernel on any grid."""
     for n in range(1, 1025):
         assert rules.bwd_pair(1, n, n, 4000, CUS) and rules.bwd_pair(2, n, n, 4000, CUS), n
+
+
+# batch, n_q, n_k, heads, causal: waves per SIMD of dK/dV's pair kernel, 2-byte D = 64
+DKDV_WAVES = [
+    (1, 4096, 4096, 12, 1, 2), (2, 2048, 2048, 12, 2, 2), (2, 2048, 2048, 16, 1, 4), (2, 2176, 2048, 12, 1, 2),
+    (2, 2560, 2048, 12, 1, 4), (2, 4096, 2048, 12, 1, 4), (2, 1024, 2048, 12, 2, 4), (2, 4096, 2048, 8, 1, 2),
+    (2, 2048, 2048, 12, 0, 4), (1, 2048, 2048, 16, 0, 2),
+]
+
+
+@pytest.mark.parametrize("row", DKDV_WAVES, ids=str)
+def test_dkdv_waves(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert rules.bwd_waves(causal, nq, nk, batch * heads, 64, 2, CUS) == want
