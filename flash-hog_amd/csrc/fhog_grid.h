@@ -125,8 +125,10 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 // The pair kernels do more LDS work per tile but take half the time per tile of
 // a wave, and their 64-row blocks spread a small grid over twice as many CUs and
 // waste less of a short causal sequence's diagonal. dK/dV takes its pair kernel
-// up to three workgroups per CU, and on fuller grids for causal problems of up to
-// 1024 keys whose diagonal shows: where 128-key blocks cover 6 % more than 64-key ones
+// up to three workgroups per CU, two for long rectangles (768 workgroups, k64 / pair:
+// 3072 queries of 2048 keys B2 H12 126 / 124, 8192 of 2048 349 / 380, 4096 of 256 B12 H16 260
+// / 284, 1024 of 4096 bottom-right B1 106 / 111), and on fuller grids for causal problems
+// of up to 1024 keys whose diagonal shows: where 128-key blocks cover 6 % more than 64-key ones
 // (others / pair: causal B1 N1024 H12 (192 workgroups) 52.4 / 45.0, B1 N4096 H12
 // (768) 184 / 163, B2 N4096 H16 over 4 key heads (512) 523 / 446, B128 N512 H12
 // 448 / 417, B24 N1024 H12 219 / 213, B32 N1024 H16 399 / 403, B4 N2048 H16 136 /
@@ -161,7 +163,7 @@ inline bool bwd_k64_rule(Mask m, int npairs, int cus) {
   return one_wave_cover(m, true, 110) && (m.causal || one_wave_rounds(m, m.nk, npairs, cus));
 }
 inline bool bwd_pair_rule(Mask m, int npairs, int cus) {
-  if ((long)((m.nk + 63) / 64) * npairs <= 3L * cus) return true;
+  if ((long)((m.nk + 63) / 64) * npairs <= (m.causal && !near_square(m, 2) ? 2L : 3L) * cus) return true;
   if (!m.causal || m.nk > 1024) return false;
   return 1000 * 2 * blocks_see(m, 128, true) >= (near_square(m, 16) ? 1058 : 1065) * blocks_see(m, 64, true);
 }

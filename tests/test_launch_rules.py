@@ -205,6 +205,8 @@ DKDV = [
     (64, 768, 512, 12, 1, "compiled"), (64, 400, 600, 12, 2, "pair"), (64, 256, 512, 12, 2, "pair"),
     (32, 2048, 512, 12, 2, "pair"), (128, 512, 512, 12, 1, "pair"), (32, 1024, 1024, 16, 1, "pair"),
     (64, 1000, 1000, 12, 1, "pair"), (32, 1100, 1100, 16, 1, "compiled"),
+    (2, 8192, 2048, 12, 1, "k64"), (4, 4096, 1024, 12, 1, "k64"), (1, 1024, 4096, 12, 2, "k64"),
+    (2, 3072, 2048, 12, 1, "pair"), (2, 8192, 2048, 8, 1, "pair"),
 ]
 
 
