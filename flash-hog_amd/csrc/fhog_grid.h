@@ -221,14 +221,20 @@ inline bool stage1_qpair_rule(Mask m, int npairs, int cus) {
 // but for 2-byte types at D = 64 on grids that fill the chip, where
 // bwdbwd_k_kernel's one wave per 32 keys is faster; both give the same bits.
 // The pair kernel's grid has twice the workgroups of half the work each, and
-// is taken while it has at most three of them per CU when causal, one
-// otherwise (stage 2, us, k / pair: causal B1 N512 H12 24.8 / 20.2, B1 N2048
-// H12 (384 workgroups) 78.4 / 69.7, B2 N2048 H12 (768) 85.2 / 74.8, B2 N4096
-// H16 over 4 key heads (512) 575 / 511, but B2 N2048 H16 (1024) 93.3 / 95.8 and
-// B1 N8192 H12 (1536) 452 / 497; non-causal B1 N300 over one key head 51.9 /
-// 44.2, but B1 N2048 H12 (384) 79.6 / 82.4, B2 N1000 H12 fp16 43.9 / 48.0).
+// is taken while it has at most three of them per CU when causal and near a square,
+// two on other causal rectangles, whose blocks are nearly equal, and one without a
+// mask (stage 2, us, k / pair: causal B1 N512 H12 24.8 / 20.2, B1 N2048 H12 (384
+// workgroups) 78.4 / 69.7, B2 N2048 H12 (768) 85.2 / 74.8, B2 N4096 H16 over 4 key heads
+// (512) 575 / 511, but B2 N2048 H16 (1024) 93.3 / 95.8 and B1 N8192 H12 (1536) 452 / 497;
+// rectangles with 768: 2304 queries of 2048 keys 95.8 / 86.0, 2560 107 / 102, 1536 of 2048
+// bottom-right 67.1 / 66.5, but 3072 of 2048 129 / 137, 4096 175 / 208, 6144 280 / 352, 1024 of
+// 2048 bottom-right 54.0 / 62.9, 1024 of 8192 64.7 / 75.2; with 640: 4096 of 2048 164 / 185;
+// with 512: 4096 of 2048 152 / 141, 8192 295 / 286, 1024 of 2048 bottom-right 43.9 / 43.6, of
+// 4096 43.4 / 44.3; with 384: 8192 of 2048 295 / 277; non-causal B1 N300 over one key head
+// 51.9 / 44.2, N2048 H8 (256) 78.3 / 66.7, but H12 (384) 79.6 / 82.4, B2 N1000 H12 fp16 43.9 /
+// 48.0).
 inline bool stage2_pair_rule(Mask m, int npairs, int cus) {
-  return (long)((m.nk + 63) / 64) * npairs <= (long)(m.causal ? 3 : 1) * cus;
+  return (long)((m.nk + 63) / 64) * npairs <= (!m.causal ? 1L : near_square(m, 4) ? 3L : 2L) * cus;
 }
 
 // Whether a causal grid deals its blocks one by one instead of folding them

@@ -234,3 +234,19 @@ DKDV_WAVES = [
 def test_dkdv_waves(rules, row):
     batch, nq, nk, heads, causal, want = row
     assert rules.bwd_waves(causal, nq, nk, batch * heads, 64, 2, CUS) == want
+
+
+# batch, n_q, n_k, heads, causal: whether stage 2 at D = 64 takes its pair kernel
+STAGE2 = [
+    (2, 2048, 2048, 12, 1, True), (2, 2560, 2048, 12, 1, True), (2, 1792, 2048, 12, 2, True),
+    (2, 4096, 2048, 8, 1, True), (1, 8192, 2048, 12, 1, True),
+    (2, 3072, 2048, 12, 1, False), (2, 8192, 2048, 12, 1, False), (2, 1024, 2048, 12, 2, False),
+    (1, 1024, 8192, 6, 2, False), (2, 4096, 2048, 10, 1, False), (2, 2048, 2048, 16, 1, False),
+    (1, 2048, 2048, 8, 0, True), (1, 2048, 2048, 12, 0, False),
+]
+
+
+@pytest.mark.parametrize("row", STAGE2, ids=str)
+def test_stage2_pair(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert bool(rules.stage2_pair(causal, nq, nk, batch * heads, CUS)) == want
