@@ -75,13 +75,16 @@ inline int fold_rank(bool causal, int nb, int npairs, int cus) {
 //   270 / 277; 4, 2 rounds, B64 N512 H8 124 / 128; 5, 3 rounds, B8 N640 H64 173 / 175;
 //   but 8, 2 rounds, B16 N1024 H16 180 / 174; 16, 2 rounds, B8 N2048 H16 302 / 290; 256,
 //   2 rounds, B1 N32768 H8 3795 / 3720);
-// - one paired workgroup per CU, from 32 blocks per pair (64, B1 N8192 H8 309 / 320; 32,
-//   B4 N4096 H16 over 4 key heads 623 / 634; but 16, B4 N2048 H8 92.6 / 90.1).
+// - one paired workgroup per CU, from 32 blocks per pair in a square (64, B1 N8192 H8
+//   309 / 320, B2 N8192 H16 over 4 key heads 1230 / 1260; 32, B4 N4096 H16 over 4 key heads
+//   623 / 634; but 16, B4 N2048 H8 92.6 / 90.1). A square's pairs leave the CUs no shorter
+//   block to fill with; equal blocks run better two to a CU (B2 H8, 4352 queries of 4096
+//   keys 182 / 180, 5120 236 / 221, 8192 452 / 383, 2048 of 4096 bottom-right 159 / 124).
 // At one workgroup per CU pairs are as good in any number of whole rounds.
 inline int block_pairing(Mask m, int nb, int npairs, int resident, int waves) {
   const long paired = (long)((nb + 1) / 2) * npairs, single = (long)nb * npairs;
   if (!m.causal || resident <= 0) return 0;
-  if (waves == 2 && nb >= 32 && single == resident && 2 * paired == resident) return 1;
+  if (waves == 2 && nb >= 32 && single == resident && 2 * paired == resident) return near_square(m, 32);
   if (single <= resident || paired % resident != 0) return 0;
   if (waves == 2 && paired == resident && nb % 4 == 0) return 2;
   return waves != 2 || paired == resident || nb < 8;

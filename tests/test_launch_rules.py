@@ -250,3 +250,17 @@ STAGE2 = [
 def test_stage2_pair(rules, row):
     batch, nq, nk, heads, causal, want = row
     assert bool(rules.stage2_pair(causal, nq, nk, batch * heads, CUS)) == want
+
+
+# batch, n_q, n_k, heads, causal: `pairs` of stage 2's one-wave kernel
+STAGE2_ORDER = [
+    (1, 8192, 8192, 8, 1, 1), (2, 4096, 4096, 8, 1, 1), (1, 8192, 8192, 8, 2, 1), (1, 6144, 8192, 8, 1, 1),
+    (2, 16384, 4096, 8, 1, 0), (2, 5120, 4096, 8, 1, 0), (2, 2048, 4096, 8, 2, 0), (4, 512, 4096, 4, 2, 0),
+    (1, 9216, 8192, 8, 1, 0), (2, 4096, 4096, 9, 1, 0), (4, 2048, 2048, 8, 1, 0), (1, 8192, 8192, 8, 0, 0),
+]
+
+
+@pytest.mark.parametrize("row", STAGE2_ORDER, ids=str)
+def test_stage2_order(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert stage2_order(rules, causal, nq, nk, batch * heads) == want
