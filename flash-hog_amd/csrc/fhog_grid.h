@@ -68,26 +68,39 @@ inline int fold_rank(bool causal, int nb, int npairs, int cus) {
 // only where the paired grid fills whole rounds of the resident ones; elsewhere
 // the unpaired blocks, longest first, balance better (stage 2, us, paired /
 // unpaired: paired grids of 0.56 rounds, B3 N2048 H12, 125 / 96; 0.75, B1 N8192 H12,
-// 442 / 387; 1.5, B16 N1024 H12, 132 / 122; 2.25, B24 N1024 H12, 216 / 194). At two
-// workgroups per CU that is
+// 442 / 387; 0.88, B4 N2048 H14, 145 / 144; 1.06, B2 N4096 H17, 411 / 314; 1.5, B16 N1024
+// H12, 132 / 122; 2.25, B24 N1024 H12, 216 / 194). At two workgroups per CU that is
 // - one round, skewed if nb allows (B4 N2048 H16 138 / 148, B1 N16384 H8 944 / 1021);
-// - more rounds of fewer than 8 blocks per pair (nb = 2, 6 rounds, B256 N256 H12
-//   270 / 277; 4, 2 rounds, B64 N512 H8 124 / 128; 5, 3 rounds, B8 N640 H64 173 / 175;
-//   but 8, 2 rounds, B16 N1024 H16 180 / 174; 16, 2 rounds, B8 N2048 H16 302 / 290; 256,
-//   2 rounds, B1 N32768 H8 3795 / 3720);
+// - more rounds of few blocks per pair. What decides is which of the two orders is
+//   chunked (grid_chunk, over 8 rounds), so that a pair's blocks run close together.
+//   Neither (up to 8 rounds of single blocks): fewer than 8 (nb = 2, B128 N256 H16 204 /
+//   216; 4, B64 N512 H8 122 / 125; 5, B8 N640 H64 173 / 175; but 2, B64 N256 H16 98 / 95; 8,
+//   B16 N1024 H16 180 / 174; 16, B8 N2048 H16 302 / 290). The single blocks only: fewer than 4
+//   (2, B192 N256 H16 292 / 300; 3, B96 N384 H16 249 / 254; but 4, B128 N512 H12 364 / 352, B96
+//   N512 H16 383 / 369; 6, B64 N768 H16 465 / 442; 16, B32 N2048 H16 1304 / 1190; 256, B1
+//   N32768 H8 3795 / 3720). Both: fewer than 16 (2, B384 N256 H16 565 / 580; 3, B192 N384 H16
+//   461 / 487; 4, B160 N512 H16 585 / 595; 8, B96 N1024 H16 1051 / 1067; 12, B64 N1536 H16
+//   1427 / 1447; but 14, B64 N1792 H16 1865 / 1845; 16, B64 N2048 H16 2398 / 2373);
 // - one paired workgroup per CU, from 32 blocks per pair in a square (64, B1 N8192 H8
 //   309 / 320, B2 N8192 H16 over 4 key heads 1230 / 1260; 32, B4 N4096 H16 over 4 key heads
-//   623 / 634; but 16, B4 N2048 H8 92.6 / 90.1). A square's pairs leave the CUs no shorter
-//   block to fill with; equal blocks run better two to a CU (B2 H8, 4352 queries of 4096
-//   keys 182 / 180, 5120 236 / 221, 8192 452 / 383, 2048 of 4096 bottom-right 159 / 124).
-// At one workgroup per CU pairs are as good in any number of whole rounds.
+//   623 / 634; but 16, B4 N2048 H8 92.6 / 90.1). Equal blocks run better two to a CU (B2 H8,
+//   4352 queries of 4096 keys 182 / 180, 5120 236 / 221, 8192 452 / 383, 2048 of 4096
+//   bottom-right 159 / 124). The gain does not end at equality below (64, B1 N8192 H7 316 /
+//   332, H6 304 / 315), where the single blocks are kept all the same.
+// At one workgroup per CU pairs are taken in any number of whole rounds; there the two
+// orders are within 2 % (first backward, us, paired / unpaired: B16 N1536 H16 353 / 359,
+// B24 N2048 H16 873 / 861, B32 N1536 H16 716 / 730, B32 N2048 H16 1197 / 1184, B48 N2048 H16
+// 1692 / 1719).
 inline int block_pairing(Mask m, int nb, int npairs, int resident, int waves) {
   const long paired = (long)((nb + 1) / 2) * npairs, single = (long)nb * npairs;
   if (!m.causal || resident <= 0) return 0;
   if (waves == 2 && nb >= 32 && single == resident && 2 * paired == resident) return near_square(m, 32);
-  if (single <= resident || paired % resident != 0) return 0;
-  if (waves == 2 && paired == resident && nb % 4 == 0) return 2;
-  return waves != 2 || paired == resident || nb < 8;
+  if (single <= resident) return 0;
+  if (paired % resident != 0) return 0;
+  if (waves != 2) return 1;
+  if (paired == resident) return nb % 4 == 0 ? 2 : 1;
+  const bool chunked = single > 8L * resident, chunked_pairs = paired > 8L * resident;
+  return nb < (chunked_pairs ? 16 : chunked ? 4 : 8);
 }
 
 // The forward: fwd_pair_kernel (two waves per 32 queries, 64-query workgroups) serves
