@@ -105,14 +105,35 @@ inline int block_pairing(Mask m, int nb, int npairs, int resident, int waves) {
   return nb < (chunked_pairs ? 16 : chunked ? 4 : 8);
 }
 
+// What the busiest CU holds when a query-tiled grid of two workgroups per CU is
+// folded (fold_rank: the longest block beside the shortest), in percent of the longest
+// block: 100 in a square, up to 200 the longer the rectangle.
+inline int folded_percent(Mask m) {
+  if (!m.causal) return 200;
+  if (m.coff > 0) return (int)(100 * (m.nk + (long)m.coff) / m.nk);  // bottom-right, nk > nq: nk and coff
+  if (m.coff < 0 || m.nq <= m.nk) return 100;
+  return m.nq >= 2L * m.nk ? 200 : (int)(100L * m.nq / m.nk);
+}
+
 // The forward: fwd_pair_kernel (two waves per 32 queries, 64-query workgroups) serves
-// 2-byte types at D = 256, and fp32 while its grid has at most one workgroup per
-// CU, or four (D = 64) or three (D = 128) when causal; fp32's two kernels give the same
-// bits (us, fwd / pair: causal N2048 H8 D64 B2 (512 workgroups) 142 / 99, B4
-// (1024) 196 / 165, B4 H16 (2048) 287 / 312; non-causal B1 (256) 142 / 97, B2
-// (512) 144 / 157; D128 causal B3 (768) 273 / 237, B4 (1024) 300 / 309).
+// 2-byte types at D = 256, and fp32 on grids that do not fill the chip; fp32's two
+// kernels give the same bits. Up to one workgroup per CU it halves the chain of a
+// block; beyond, it pays where short causal blocks share a CU with long ones (us, fwd /
+// pair; fp32 H8):
+// - two per CU, unless two nearly full blocks meet (D = 64, N2048 B2 142 / 99; 1024
+//   queries of 2048 keys bottom-right (150 %) B4 144 / 127; but 512 of 4096 bottom-right
+//   (187 %) B8 285 / 296, 2048 of 1024 (200 %) B4 H4 74.5 / 81.3; D = 128, 512 of 4096 (187 %)
+//   B8 552 / 531; but 2048 of 1024 (200 %) B4 H4 143 / 145; non-causal D = 64 N2048 144 / 157);
+// - three near a square (D = 64, 1536 queries of 1024 keys B4 102 / 96; D = 128, N2048 B3
+//   273 / 237, 1280 of 1024 B4 143 / 126; but 1536 of 1024 B4 164 / 169);
+// - four in a square at D = 64 (N2048 B4 196 / 165, 1024 queries of 1152 keys B8 118 / 110; but
+//   of 1280 134 / 139; B4 H16, eight per CU, 287 / 312; D = 128 B4 300 / 309).
 inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
-  return (long)((m.nq + 63) / 64) * npairs <= (long)(!m.causal ? 1 : head_dim == 64 ? 4 : 3) * cus;
+  const long grid = (long)((m.nq + 63) / 64) * npairs;
+  if (grid <= cus) return true;
+  if (grid <= 2L * cus && folded_percent(m) <= (head_dim == 64 ? 175 : 190)) return true;
+  if (grid <= 3L * cus && near_square(m, head_dim == 64 ? 2 : 4)) return true;
+  return grid <= 4L * cus && head_dim == 64 && near_square(m, 8);
 }
 
 // The first backward for 2-byte types at D = 64 has several kernels for each

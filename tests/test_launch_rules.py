@@ -39,6 +39,7 @@ int pairing(int c, int nq, int nk, int nb, int np, int resident, int waves) {
   return fhog::block_pairing(mask(c, nq, nk), nb, np, resident, waves);
 }
 long sees(int c, int nq, int nk, int rows, int keys) { return fhog::blocks_see(mask(c, nq, nk), rows, keys != 0); }
+int folded_percent(int c, int nq, int nk) { return fhog::folded_percent(mask(c, nq, nk)); }
 int near_square(int c, int nq, int nk, int parts) { return fhog::near_square(mask(c, nq, nk), parts); }
 int fold(int c, int nb, int np, int cus) { return fhog::fold_rank(c != 0, nb, np, cus); }
 int chunk(int np, int nranks, int resident) { return fhog::grid_chunk(np, nranks, resident); }
@@ -271,3 +272,37 @@ STAGE2_ORDER = [
 def test_stage2_order(rules, row):
     batch, nq, nk, heads, causal, want = row
     assert stage2_order(rules, causal, nq, nk, batch * heads) == want
+
+
+def test_folded_percent(rules):
+    """Against the two blocks on each CU of a folded grid of two workgroups per CU."""
+    for nq in (64, 512, 1024, 4096):
+        for nk in (64, 512, 1024, 4096):
+            for causal in (1, 2):
+                coff = nk - nq if causal == 2 else 0
+                see = sorted((min(nk, max(0, q0 + 64 + coff)) for q0 in range(0, nq, 64)), reverse=True)
+                busiest = max(a + b for a, b in zip(see, reversed(see)))
+                want = 100 * (busiest - (64 if nq > 64 else 0)) / max(see)  # a block's own 64 rows
+                got = rules.folded_percent(causal, nq, nk)
+                assert abs(got - want) <= 100 * 128 / max(see) or nq == 64, (nq, nk, causal, got, want)
+    assert rules.folded_percent(0, 512, 512) == 200
+
+
+# batch, n_q, n_k, heads, head_dim, causal: whether the fp32 forward takes its pair kernel
+FORWARD = [
+    (2, 2048, 2048, 8, 64, 1, True), (4, 2048, 2048, 8, 64, 1, True), (4, 2048, 2048, 16, 64, 1, False),
+    (4, 1024, 2048, 8, 64, 2, True), (4, 1536, 1024, 8, 64, 1, True), (8, 1024, 1152, 8, 64, 2, True),
+    (4, 512, 2048, 8, 64, 2, True), (1, 4096, 512, 4, 64, 1, True),
+    (8, 512, 4096, 8, 64, 2, False), (16, 512, 4096, 8, 64, 2, False), (4, 2048, 1024, 4, 64, 1, False),
+    (8, 1024, 1280, 8, 64, 2, False), (4, 4096, 2048, 4, 64, 1, False),
+    (3, 2048, 2048, 8, 128, 1, True), (8, 512, 4096, 8, 128, 2, True), (4, 1024, 2048, 8, 128, 2, True),
+    (4, 1280, 1024, 8, 128, 1, True), (4, 1536, 1024, 8, 128, 1, False), (6, 1024, 2048, 8, 128, 2, False),
+    (4, 2048, 1024, 4, 128, 1, False), (4, 2048, 2048, 8, 128, 1, False),
+    (1, 2048, 2048, 8, 64, 0, True), (2, 2048, 2048, 8, 64, 0, False),
+]
+
+
+@pytest.mark.parametrize("row", FORWARD, ids=str)
+def test_forward(rules, row):
+    batch, nq, nk, heads, d, causal, want = row
+    assert bool(rules.fwd_pair(causal, nq, nk, batch * heads, d, CUS)) == want
