@@ -247,13 +247,17 @@ inline bool stage1_fused_rule(Mask m) {
 // Stage 1 for fp32 runs bwdbwd_q_kernel (fhog_bwdbwd.hip, one wave per 32 queries) on grids
 // that fill the chip and bwdbwd_qpair_kernel (fhog_bwdbwd_qpair.hip, two waves per
 // 32 queries, half the time per block and twice the workgroups) on smaller ones;
-// both give the same bits. The line is two of the latter's workgroups per CU
-// when causal, one otherwise (stage 1, us, q / qpair: causal D = 64 N2048 H8 B2
-// (512 workgroups) 887 / 631, B3 (768) 890 / 840-885, B4 (1024) 970 / 1093;
-// non-causal B1 (256) 902 / 626, B2 (512) 910 / 1021; D = 128 causal B2 (512)
-// 1620 / 1296, B4 (1024) 1783 / 2538, non-causal B1 (256) 1647 / 1255).
+// both give the same bits. The line is one of the latter's workgroups per CU, two
+// where folded blocks even out (stage 1, us, q / qpair: causal D = 64 N2048 H8 B2 (512
+// workgroups) 887 / 631, B3 (768) 890 / 840-885, B4 (1024) 970 / 1093; 512 of them, 768
+// queries of 1024 keys bottom-right (125 %) B4 H10 454 / 434, 1280 of 1024 (125 %) B4 H6 455 / 433,
+// 1024 of 2048 bottom-right (150 %) B4 H8 902 / 828, but 1536 of 1024 (150 %) B4 H5 456 / 458, 2048 of
+// 1024 (200 %) B4 H4 456 / 533, 512 of 4096 bottom-right (187 %) B8 H8 1798 / 2002; non-causal B1
+// (256) 902 / 626, B2 (512) 910 / 1021; D = 128 causal B2 (512) 1620 / 1296, B4 (1024) 1783 /
+// 2538, 1280 of 1024 (125 %) B4 H6 833 / 804, 1024 of 2048 bottom-right (150 %) B4 H8 1650 / 1863, 512
+// of 4096 (187 %) B8 H8 3324 / 4645, non-causal B1 (256) 1647 / 1255).
 inline bool stage1_qpair_rule(Mask m, int npairs, int cus) {
-  return (long)((m.nq + 63) / 64) * npairs <= (long)(m.causal ? 2 : 1) * cus;
+  return (long)((m.nq + 63) / 64) * npairs <= (folded_percent(m) <= 140 ? 2L : 1L) * cus;
 }
 
 // Stage 2 runs bwdbwd_pair_kernel (fhog_bwdbwd_pair.hip, two waves per 32 keys)

@@ -306,3 +306,18 @@ FORWARD = [
 def test_forward(rules, row):
     batch, nq, nk, heads, d, causal, want = row
     assert bool(rules.fwd_pair(causal, nq, nk, batch * heads, d, CUS)) == want
+
+
+# batch, n_q, n_k, heads, causal: whether the fp32 stage 1 takes its pair kernel
+STAGE1_FP32 = [
+    (2, 2048, 2048, 8, 1, True), (4, 768, 1024, 10, 2, True), (4, 1280, 1024, 6, 1, True), (4, 512, 512, 8, 2, True),
+    (1, 2048, 1024, 8, 1, True), (1, 2048, 2048, 8, 0, True),
+    (8, 512, 4096, 8, 2, False), (4, 2048, 1024, 4, 1, False), (4, 1536, 1024, 5, 1, False),
+    (4, 2048, 2048, 8, 1, False), (2, 2048, 2048, 8, 0, False),
+]
+
+
+@pytest.mark.parametrize("row", STAGE1_FP32, ids=str)
+def test_stage1_fp32(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert bool(rules.stage1_qpair(causal, nq, nk, batch * heads, CUS)) == want
