@@ -282,28 +282,37 @@ inline bool stage2_pair_rule(Mask m, int npairs, int cus) {
 
 // Whether a causal grid deals its blocks one by one instead of folding them
 // (bwdbwd_q32_kernel; both give the same bits): when every block can have a CU of
-// its own, or when the folded items' rounds take over 8 % longer than the longest
-// block or an even share of all blocks (their keys vary linearly, from first to
-// last). Stage 1, us, folded / dealt: one round of blocks, B1 N512 H12 28.6 / 20.5,
-// B1 N1024 H12 41.8 / 33.7, B1 N2048 H12 67.5 / 62.0; estimated gain 12 %, B4 N1024
-// H12 46.0 / 44.6; 11 %, B24 N1024 H12 258 / 248; 33 %, B1 N8192 H12 650 / 518; 36 %,
-// B8 N1500 H12 fp16 218 / 176; 50 %, B3 N2048 H12 155 / 115; but 7 %, B40 N1024 H12
-// 414 / 422; 6 %, B2 N2048 H12 77.0 / 78.4; 3 %, B1 N4096 H12 141 / 149 (fewer CUs
-// run faster); none, B32 N1024 H12 324 / 332, B4 N2048 H16 182 / 183.
+// its own, or when the folded items' rounds take so much longer than the dealt blocks:
+// 8 % near a square, 19 % on rectangles, where dealing gives up more of the tiles that a
+// pair's blocks share in L2. Dealt blocks take at least the longest block, an even share
+// of all, and as many shortest blocks as some CU gets. Stage 1, us, folded / dealt: one
+// round of blocks, B1 N512 H12 28.6 / 20.5, B1 N1024 H12 41.8 / 33.7, B1 N2048 H12 67.5 / 62.0;
+// estimated gain 12 %, B4 N1024 H12 46.0 / 44.6; 11 %, B24 N1024 H12 258 / 248; 33 %, B1
+// N8192 H12 650 / 518; 36 %, B8 N1500 H12 fp16 218 / 176; 50 %, B3 N2048 H12 155 / 115; but
+// 7 %, B40 N1024 H12 414 / 422; 6 %, B2 N2048 H12 77.0 / 78.4; 3 %, B1 N4096 H12 141 / 149
+// (fewer CUs run faster); none, B32 N1024 H12 324 / 332, B4 N2048 H16 182 / 183.
+// Rectangles, H12: 42 %, 1024 queries of 8192 keys bottom-right B7 1105 / 870, 600 of 3000
+// B12 378 / 312; 25 %, 4096 of 1024 B6 371 / 329; 20 %, 900 of 2000 bottom-right B13 371 / 328;
+// but 18 %, 5000 of 1000 B2 153 / 155; 14 %, 1024 of 4096 bottom-right B28 1578 / 1631, B4 H10
+// 209 / 220; 6 %, 1024 of 8192 B4 462 / 475; none, 1024 of 4096 B32 1618 / 1839.
 inline bool q32_deal_rule(Mask m, int npairs, int cus) {
   constexpr int kRows = 128;
-  const int nqb = (int)(((long)m.nq + kRows - 1) / kRows);
-  const long blocks = (long)npairs * nqb;
+  const long nqb = ((long)m.nq + kRows - 1) / kRows, blocks = npairs * nqb;
   if (!m.causal) return false;
   if (blocks <= cus) return true;
-  auto keys = [&](int qb) {
-    const long e = (long)(qb + 1) * kRows + m.coff;
+  if (cus <= 0) return false;
+  auto keys = [&](long qb) {
+    const long e = (qb + 1) * kRows + m.coff;
     return (double)(e < 0 ? 0 : e < m.nk ? e : m.nk);
   };
+  auto most = [](double a, double b) { return a > b ? a : b; };
   const double first = keys(0), last = keys(nqb - 1);
-  const long rounds = ((long)npairs * ((nqb + 1) / 2) + cus - 1) / (cus > 0 ? cus : 1);
-  const double share = 0.5 * (first + last) * (double)blocks / cus;
-  return cus > 0 && (double)rounds * (first + last) > 1.08 * (last > share ? last : share);
+  const long mid = (nqb - 1) / 2;
+  const double item = most(first + last, keys(mid) + keys(nqb - 1 - mid));  // the longest of the folded items
+  const double rounds = (double)((npairs * ((nqb + 1) / 2) + cus - 1) / cus);
+  const double share = (double)npairs * blocks_see(m, kRows, false) / cus;
+  const double dealt = most(most(last, share), (double)((blocks + cus - 1) / cus) * first);
+  return rounds * item > (near_square(m, 4) ? 1.08 : 1.19) * dealt;
 }
 
 }  // namespace fhog

@@ -321,3 +321,23 @@ STAGE1_FP32 = [
 def test_stage1_fp32(rules, row):
     batch, nq, nk, heads, causal, want = row
     assert bool(rules.stage1_qpair(causal, nq, nk, batch * heads, CUS)) == want
+
+
+# batch, n_q, n_k, heads, causal: whether stage 1's 32-query kernel deals its blocks
+DEAL = [
+    (1, 512, 512, 12, 1, True), (4, 1024, 1024, 12, 1, True), (24, 1024, 1024, 12, 1, True),
+    (1, 8192, 8192, 12, 1, True), (8, 1500, 1500, 12, 1, True), (3, 2048, 2048, 12, 1, True),
+    (40, 1024, 1024, 12, 1, False), (2, 2048, 2048, 12, 1, False), (1, 4096, 4096, 12, 1, False),
+    (32, 1024, 1024, 12, 1, False), (4, 2048, 2048, 16, 1, False),
+    (7, 1024, 8192, 12, 2, True), (12, 600, 3000, 12, 2, True), (6, 4096, 1024, 12, 1, True),
+    (13, 900, 2000, 12, 2, True), (1, 8192, 4096, 12, 1, True), (24, 2048, 1024, 12, 2, True),
+    (28, 1024, 4096, 12, 2, False), (4, 1024, 4096, 10, 2, False), (4, 1024, 8192, 12, 2, False),
+    (3, 1024, 8192, 16, 2, False), (2, 5000, 1000, 12, 1, False), (32, 1024, 4096, 12, 2, False),
+    (3, 2048, 2048, 12, 0, False),
+]
+
+
+@pytest.mark.parametrize("row", DEAL, ids=str)
+def test_deal(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert bool(rules.q32_deal(causal, nq, nk, batch * heads, CUS)) == want
