@@ -141,7 +141,7 @@ bwdbwd_q_kernel(BwdBwdParams<T> p, int chunk) {
   if (CAUSAL) wend = max(0, min(wend, q0 + 32 + p.coff));
   const int wkt = q0 < p.nq ? (wend + BK - 1) / BK : 0;  // tiles with work for this wave
 
-  SwzFrags<T, D> fr;
+  WaveFrags<T, D> fr;
   fr.init(lane);
 
   // Wave w streams tensor w; the key sequence is streamed twice (iterations

@@ -401,6 +401,45 @@ template <typename T, int D, int COLS = 64> struct SwzFrags {
   }
 };
 
+// The same operands for fp32, addressed from the tile's pointer: the swizzle of an
+// element is formed where it is read. In the kernels that keep one or two fp32 waves
+// per SIMD at D = 64 the compiler hides that in the matrix instructions' shadow, and
+// the registers of SwzFrags' offsets cost more: stage 1 at B4 N2048 H16 1910 us against
+// 1931 with them, non-causal 3546 / 3591, forward non-causal 510 / 513. (At D = 128
+// the offsets win: stage 1 at B4 N2048 H16 3540 against 4277.)
+template <typename T, int D> struct PointerFrags {
+  static_assert(sizeof(T) == 4, "fp32 only");
+  int lane;
+  __device__ __forceinline__ void init(int l) { lane = l; }
+  __device__ __forceinline__ V8<T> rowf(uint32_t stage, int off, int ks) const {
+    const int n = lane & 31, g = lane >> 5;
+    const T* row = tile(stage, off) + n * D;
+    const V4<T> a = *reinterpret_cast<const V4<T>*>(row + 4 * phys_chunk(n, 4 * ks + 2 * g));
+    const V4<T> b = *reinterpret_cast<const V4<T>*>(row + 4 * phys_chunk(n, 4 * ks + 2 * g + 1));
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+  __device__ __forceinline__ V8<T> trf(uint32_t stage, int off, int dt, int s) const {
+    const T* t = tile(stage, off);
+    const int g = lane >> 5, col = 32 * dt + (lane & 31);
+    V8<T> v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int row = 16 * s + 8 * (e >> 2) + 4 * g + (e & 3);
+      v[e] = t[row * D + 4 * phys_chunk(row, col >> 2) + (col & 3)];
+    }
+    return v;
+  }
+
+ private:
+  __device__ __forceinline__ static const T* tile(uint32_t stage, int off) {
+    // an address-space conversion, which only a C-style cast expresses
+    return (const T*)((const lds_cchar*)(uintptr_t)stage + off);
+  }
+};
+// The operands of the kernels with one wave per 32 queries.
+template <typename T, int D, int COLS = 64>
+using WaveFrags = std::conditional_t<sizeof(T) == 4 && D == 64, PointerFrags<T, D>, SwzFrags<T, D, COLS>>;
+
 // ---------------------------------------------------------------------------
 // The 16x16x32 matrix instruction (v_mfma_f32_16x16x32_{bf16,f16}), used by
 // the kernels that give each wave 16 rows (lane l, n = l % 16, g = l / 16):

@@ -95,7 +95,7 @@ fwd_kernel(FwdParams<T> p, int chunk) {
   const int wkt = q0 < p.nq ? (wend + BK - 1) / BK : 0;
 
   // (offsets of its own for every column: with shared ones D = 128 was 1-2 % slower)
-  SwzFrags<T, D, sizeof(T) == 2 ? D : 64> fr;
+  WaveFrags<T, D, sizeof(T) == 2 ? D : 64> fr;
   fr.init(lane);
   const int tensor = wave >> 1;  // 0 = K, 1 = V
   const T* src = (tensor == 0 ? p.k : p.v) + kbase;
