@@ -40,9 +40,9 @@ SHAPES = [
     ("empty_key_blocks", 16, 1024, 2304, 2, 2, 1, 64),
     # bottom-right causal with N_Q > N_K: leading query rows see no key
     ("bottom_right", 16, 2600, 2304, 2, 2, 2, 64),
-    # D = 128 (one wave per SIMD, 256 resident workgroups): two rounds
+    # D = 128: 64-key workgroups of two waves per 32 keys, 128-query ones for dQ
     ("d128", 16, 2048, 2048, 2, 2, 1, 128),
-    # D = 256: the dK/dV kernel runs twice, for the two halves of the output columns
+    # D = 256: the kernels with two waves per 32 rows, grouped heads
     ("d256_gqa2", 4, 1100, 1100, 4, 2, 1, 256),
 ]
 

@@ -7,8 +7,8 @@ D = 64 on small grids or with FLASH_HOG_BWD=pair; the second fp32 and head dim
 Sizes are where they can go wrong: one row, one tile and its neighbours, a
 ragged last tile on either side, blocks of 64 that are half empty or see
 nothing, grouped heads, and grids above the sizes where the launch folds the
-block order (257 to 512 workgroups on 256 CUs) and takes three workgroups per
-CU (over 1024). Against the closed form in fp64 at the tolerances of
+block order (257 to 512 workgroups on 256 CUs) and takes more waves per SIMD, with
+a mask and without (over 512 and over 1024 workgroups). Against the closed form in fp64 at the tolerances of
 tests/helpers.py (fp32 products here sum at most 1300 terms). They must give
 the bits of bwd_k_kernel (D = 64) and bwd_q_kernel (2-byte D = 64 and 128).
 """
@@ -33,6 +33,8 @@ SHAPES = [
     ("bottom_right_long_q", 1, 300, 100, 2, 2, 2),
     ("folded_order", 37, 450, 450, 1, 1, 1),
     ("over_1024_workgroups", 26, 600, 600, 4, 4, 1),
+    ("over_512_workgroups_no_mask", 15, 600, 600, 4, 4, 0),
+    ("over_1024_workgroups_no_mask", 26, 600, 600, 4, 4, 0),
 ]
 KINDS = [(torch.bfloat16, 64), (torch.bfloat16, 128), (torch.float16, 256), (torch.float32, 64), (torch.float32, 128)]
 

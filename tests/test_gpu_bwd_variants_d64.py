@@ -4,9 +4,9 @@ The dK/dV work runs in the kernel with 64 keys per wave and a generated sweep
 (fhog_bwd_k64.hip) or in the compiled one (bwd_k_kernel in fhog_bwd.hip, 32
 keys per wave at two waves per SIMD), the dQ work in the kernel with 64
 queries per wave and a generated sweep (fhog_bwd_q64.hip) or in the compiled
-bwd_q_kernel: by default the one-wave kernel when its grid fills whole rounds
-of resident workgroups, else the compiled one; FLASH_HOG_BWD = k64 or
-compiled and FLASH_HOG_BWDQ = q64 or compiled force either kernel.
+bwd_q_kernel; fhog_grid.h's rules choose by the problem's size (and small grids run the
+kernels of test_gpu_bwd_pair.py). FLASH_HOG_BWD = k64 or compiled and FLASH_HOG_BWDQ =
+q64 or compiled force either kernel.
 
 The other suites run the defaults. Here every D = 64 bf16 and fp16 case of
 the parity, scale and random-sweep suites and every D = 64 shape of the
@@ -23,6 +23,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+import rules_host
 import test_gpu_bwd_grids as grids
 import test_gpu_parity as parity
 import test_gpu_sweep as sweep
@@ -127,3 +128,32 @@ def test_q64_matches_compiled_full_size(case, cuda_device, monkeypatch):
         assert torch.isfinite(a).all(), label
         print(f"  {label}: max abs diff {(a.float() - b.float()).abs().max().item():.3e}", flush=True)
         assert torch.equal(a, b), f"{label}: q64 and compiled differ"
+
+
+# Mirrored blocks in whole rounds of the one-wave kernels (four or six 256-row blocks), with
+# grouped heads, key blocks that no query sees and queries that see no key.
+MIRRORED = [("square_gqa2", 64, 1000, 1000, 4, 2, 1), ("empty_key_blocks_gqa2", 64, 300, 1000, 4, 2, 1),
+            ("bottom_right_long_q_gqa2", 64, 1300, 1000, 4, 2, 2)]
+
+
+@pytest.mark.parametrize("case", MIRRORED, ids=[c[0] for c in MIRRORED])
+def test_mirrored_blocks_match_compiled(case, cuda_device, monkeypatch, tmp_path):
+    name, B, Nq, Nk, H, Hk, causal = case
+    print(f"[case] one-wave kernels, mirrored blocks: {name}", flush=True)
+    from flash_hog import _hip
+
+    rules = rules_host.load(tmp_path)
+    assert rules_host.one_wave_order(rules, causal, Nq, Nk, Nk, B * Hk) == 1
+    assert rules_host.one_wave_order(rules, causal, Nq, Nk, Nq, B * H) == 1
+    x = make_inputs(B, Nq, Nk, H, 64, torch.bfloat16, seed=29, kv_heads=Hk, device=cuda_device)
+    scale = default_scale(64)
+    o, lse = _hip.attention_fwd(x["q"], x["k"], x["v"], causal, scale)
+    outs = {}
+    for kv, q in (("compiled", "compiled"), ("k64", "q64")):
+        monkeypatch.setenv("FLASH_HOG_BWD", kv)
+        monkeypatch.setenv("FLASH_HOG_BWDQ", q)
+        outs[kv] = _hip.attention_bwd(x["q"], x["k"], x["v"], o, x["do"], lse, causal, scale)
+        torch.cuda.synchronize()
+    for a, b, label in zip(outs["k64"], outs["compiled"], ("dq", "dk", "dv", "D")):
+        assert torch.isfinite(a).all(), label
+        assert torch.equal(a, b), label

@@ -20,6 +20,8 @@ from test_gpu_bwd_pair import SHAPES, _probs
 pytestmark = pytest.mark.gpu
 
 D = 128
+# grids of 128-query workgroups, which compute a power-of-two scale in another instance
+LARGE = [s for s in SHAPES if s[0].startswith("over_")]
 SCALES = {"default": None, "pow2": 0.125, "negative": -0.11}
 
 
@@ -51,8 +53,10 @@ def _run(x, o, lse, causal, scale, b=slice(None)):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("shape,scale", [(s, "default") for s in SHAPES] + [(SHAPES[4], "pow2"), (SHAPES[6], "negative")],
-                         ids=[s[0] for s in SHAPES] + ["pow2_scale", "negative_scale"])
+@pytest.mark.parametrize("shape,scale", [(s, "default") for s in SHAPES] + [(SHAPES[4], "pow2"), (SHAPES[6], "negative")]
+                         + [(s, "pow2") for s in LARGE],
+                         ids=[s[0] for s in SHAPES] + ["pow2_scale", "negative_scale"]
+                         + ["pow2_scale_" + s[0] for s in LARGE])
 def test_stage1_pair(shape, scale, dtype, cuda_device):
     name, B, Nq, Nk, H, Hk, causal = shape
     print("[case] stage 1 at D = 128, two waves per 32 queries:", name, scale, dtype, flush=True)

@@ -1,15 +1,17 @@
 """The double backward on shapes that select each of stage 2's grid layouts.
 
-Stage 2 (pass 4, tiled over key blocks: 128 keys at D = 64 and 256, 64 keys
-in the 16-key-per-wave kernel used for 2-byte types at D = 128, which keeps
-plain rank-major or chunked order) lays its grid out by the problem's
-size: one key block per workgroup when the grid fits on the GPU at once; for
-larger causal grids a workgroup takes key block r and then its mirror
-nkb - 1 - r (odd nkb leaves the middle block alone); and when that paired grid
-is exactly two workgroups per CU the pairs are skewed (the standard
-configuration in test_gpu_configs.py). A workgroup streams the query tiles
-of both its blocks through one ring, and a block no query sees (top-left
-causal with N_K > N_Q) streams nothing and writes zeros. Each shape here is
+Stage 2 (pass 4, tiled over key blocks) runs 2-byte types at D = 64 on grids that fill
+the chip in bwdbwd_k_kernel, 128 keys per workgroup, and lays that grid out by the
+problem's size (block_pairing): one key block per workgroup, longest first; or a
+workgroup takes key block r and then its mirror nkb - 1 - r (odd nkb leaves the
+middle block alone), where such a grid fills whole rounds of the resident
+workgroups, or half a round of many blocks; exactly one round of a multiple of four
+blocks is skewed. A workgroup streams the query tiles of both its blocks through one
+ring, and a block no query sees (top-left causal with N_K > N_Q) streams nothing and
+writes zeros. ORDERS holds the layout that each D = 64 shape is here for, and the
+launch rule is asked for it, so that a changed rule cannot leave a layout untested.
+D = 128 and 256 run bwdbwd_pair_kernel, 64 keys per workgroup, one block per
+workgroup in rank-major or chunked order. Each shape is
 checked on every (batch, head) against tests/gpu_reference.py (fp32 closed
 form on the GPU, pinned to the fp64 oracle in test_gpu_parity.py), with the
 residual (O, L) from gpu_reference.fwd. Tolerance: max|a - r| / max|r| < 2e-2
@@ -24,6 +26,7 @@ import pytest
 import torch
 
 import gpu_reference
+import rules_host
 from helpers import make_inputs, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -32,17 +35,17 @@ TOL = 2e-2
 
 # id, batch, n_q, n_k, heads, kv_heads, causal (C ABI code), head_dim
 SHAPES = [
-    # 18 key blocks x 32 (batch, head) pairs > 512 resident workgroups: mirror pairs
-    ("mirror_pairs_even", 16, 2304, 2304, 2, 2, 1, 64),
-    # 17 key blocks: the middle block has no mirror
-    ("mirror_pairs_odd", 16, 2176, 2176, 2, 2, 1, 64),
-    # grouped heads (4 query heads per key/value head) with mirror pairs
-    ("mirror_pairs_gqa4", 8, 2304, 2304, 16, 4, 1, 64),
-    # top-left causal, N_K > N_Q: key blocks past N_Q see no query (empty blocks in pairs)
-    ("mirror_pairs_empty_blocks", 16, 1024, 2304, 2, 2, 1, 64),
+    # 18 key blocks x 32 (batch, head) pairs, 1.1 rounds of 512 resident workgroups: single blocks
+    ("single_blocks_even", 16, 2304, 2304, 2, 2, 1, 64),
+    # 17 key blocks
+    ("single_blocks_odd", 16, 2176, 2176, 2, 2, 1, 64),
+    # grouped heads (4 query heads per key/value head)
+    ("single_blocks_gqa4", 8, 2304, 2304, 16, 4, 1, 64),
+    # top-left causal, N_K > N_Q: key blocks past N_Q see no query
+    ("single_blocks_empty_blocks", 16, 1024, 2304, 2, 2, 1, 64),
     # bottom-right causal with N_Q > N_K
-    ("mirror_pairs_bottom_right", 16, 2600, 2304, 2, 2, 2, 64),
-    # D = 128 (64-key blocks, no mirror pairs): 32 blocks x 32 pairs, rank-major
+    ("single_blocks_bottom_right", 16, 2600, 2304, 2, 2, 2, 64),
+    # D = 128 (64-key blocks): 32 blocks x 32 pairs, rank-major
     ("d128_rank_major", 16, 2048, 2048, 2, 2, 1, 128),
     # 33 blocks, the last one ragged
     ("d128_ragged_last_block", 16, 2100, 2100, 2, 2, 1, 128),
@@ -52,10 +55,26 @@ SHAPES = [
     ("d128_empty_blocks", 16, 1024, 2304, 2, 2, 1, 128),
     # 16 blocks x 288 pairs = 9 rounds of 512 workgroups: chunked grid order
     ("d128_chunked", 144, 1024, 1024, 2, 2, 1, 128),
-    # D = 256 (the 32-key kernel at one wave per SIMD, 256 resident workgroups):
-    # 18 key blocks x 32 pairs, mirror pairs without the skew
-    ("d256_mirror_pairs", 16, 2304, 2304, 2, 2, 1, 256),
+    # D = 256 (one wave per SIMD, 256 resident workgroups): 36 blocks x 32 pairs
+    ("d256_rank_major", 16, 2304, 2304, 2, 2, 1, 256),
+    # D = 64, mirrored: exactly one round of pairs of four blocks, skewed; grouped heads, with
+    # blocks that no query sees, and with leading queries that see no key
+    ("skewed_pairs_gqa2", 64, 512, 512, 8, 4, 1, 64),
+    ("skewed_pairs_empty_blocks", 64, 200, 512, 4, 4, 1, 64),
+    ("skewed_pairs_bottom_right", 64, 700, 512, 4, 4, 2, 64),
+    # one round of three blocks: the middle one has no mirror
+    ("mirror_pairs_odd_gqa2", 64, 330, 330, 8, 4, 1, 64),
+    # two rounds
+    ("mirror_pairs_two_rounds_gqa2", 128, 300, 300, 8, 4, 1, 64),
+    # 31/32 of a round
+    ("mirror_pairs_near_a_round", 31, 2048, 2048, 2, 2, 1, 64),
+    # 32 blocks x 16 pairs: one paired workgroup per CU
+    ("mirror_pairs_one_per_cu_gqa2", 4, 4096, 4096, 8, 4, 1, 64),
+    ("mirror_pairs_one_per_cu_empty_blocks", 4, 3000, 4096, 4, 4, 1, 64),
+    ("mirror_pairs_one_per_cu_bottom_right", 4, 5000, 4096, 4, 4, 2, 64),
 ]
+# `pairs` of block_pairing: 0 single blocks, 1 mirrored, 2 skewed
+ORDERS = {"single": 0, "mirror": 1, "skewed": 2}
 
 
 def _reference_residual(x, scale, causal, dtype):
@@ -107,12 +126,20 @@ def _bwdbwd_head(q, k, v, o, do, ddq, ddk, ddv, lse, scale, causal):
         mm(ddp.t().contiguous(), do), mm(p, ddv) + mm(ddp, v)
 
 
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    return rules_host.load(tmp_path_factory.mktemp("rules"))
+
+
 @pytest.mark.parametrize("shape", SHAPES, ids=[s[0] for s in SHAPES])
-def test_stage2_grid_layouts(shape, cuda_device):
+def test_stage2_grid_layouts(shape, cuda_device, rules):
     from flash_hog import _hip
 
     name, B, Nq, Nk, H, Hk, causal, D = shape
     print("[case] stage-2 grid", name, flush=True)
+    if D == 64:
+        assert not rules.stage2_pair(causal, Nq, Nk, B * Hk, rules_host.CUS)
+        assert rules_host.stage2_order(rules, causal, Nq, Nk, B * Hk) == ORDERS[name.split("_")[0]]
     dtype = torch.bfloat16
     scale = 1.0 / math.sqrt(D)
     x = make_inputs(B, Nq, Nk, H, D, dtype, seed=71, kv_heads=Hk, device=cuda_device)

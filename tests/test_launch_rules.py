@@ -8,58 +8,14 @@ measured the faster one there; the times stand beside the rules.
 
 from __future__ import annotations
 
-import ctypes
-import pathlib
-import shutil
-import subprocess
-
 import pytest
 
-CSRC = pathlib.Path(__file__).resolve().parent.parent / "flash-hog_amd" / "csrc"
-CUS = 256
-
-WRAPPERS = r"""
-#include "fhog_grid.h"
-using fhog::Mask;
-static Mask mask(int causal, int nq, int nk) { return Mask{causal != 0, nq, nk, causal == 2 ? nk - nq : 0}; }
-extern "C" {
-int fwd_pair(int c, int nq, int nk, int np, int d, int cus) { return fhog::fwd_pair_rule(mask(c, nq, nk), np, d, cus); }
-int bwd_pair(int c, int nq, int nk, int np, int cus) { return fhog::bwd_pair_rule(mask(c, nq, nk), np, cus); }
-int bwd_k64(int c, int nq, int nk, int np, int cus) { return fhog::bwd_k64_rule(mask(c, nq, nk), np, cus); }
-int bwd_qpair(int c, int nq, int nk, int np, int cus) { return fhog::bwd_qpair_rule(mask(c, nq, nk), np, cus); }
-int bwd_q64(int c, int nq, int nk, int np, int cus) { return fhog::bwd_q64_rule(mask(c, nq, nk), np, cus); }
-int bwd_waves(int c, int nq, int nk, int np, int d, int bytes, int cus) {
-  return fhog::bwd_pair_waves(mask(c, nq, nk), np, d, bytes, cus);
-}
-int stage1_fused(int c, int nq, int nk) { return fhog::stage1_fused_rule(mask(c, nq, nk)); }
-int stage1_qpair(int c, int nq, int nk, int np, int cus) { return fhog::stage1_qpair_rule(mask(c, nq, nk), np, cus); }
-int stage2_pair(int c, int nq, int nk, int np, int cus) { return fhog::stage2_pair_rule(mask(c, nq, nk), np, cus); }
-int q32_deal(int c, int nq, int nk, int np, int cus) { return fhog::q32_deal_rule(mask(c, nq, nk), np, cus); }
-int pairing(int c, int nq, int nk, int nb, int np, int resident, int waves) {
-  return fhog::block_pairing(mask(c, nq, nk), nb, np, resident, waves);
-}
-long sees(int c, int nq, int nk, int rows, int keys) { return fhog::blocks_see(mask(c, nq, nk), rows, keys != 0); }
-int folded_percent(int c, int nq, int nk) { return fhog::folded_percent(mask(c, nq, nk)); }
-int near_square(int c, int nq, int nk, int parts) { return fhog::near_square(mask(c, nq, nk), parts); }
-int fold(int c, int nb, int np, int cus) { return fhog::fold_rank(c != 0, nb, np, cus); }
-int chunk(int np, int nranks, int resident) { return fhog::grid_chunk(np, nranks, resident); }
-}
-"""
+from rules_host import CUS, load, one_wave_order, stage2_order
 
 
 @pytest.fixture(scope="module")
 def rules(tmp_path_factory):
-    cxx = shutil.which("g++") or shutil.which("c++") or shutil.which("clang++")
-    if cxx is None:
-        pytest.skip("no host C++ compiler")
-    d = tmp_path_factory.mktemp("rules")
-    (d / "rules.cpp").write_text(WRAPPERS)
-    cmd = [cxx, "-std=c++20", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}", str(d / "rules.cpp"), "-o",
-           str(d / "rules.so")]
-    subprocess.run(cmd, check=True)
-    lib = ctypes.CDLL(str(d / "rules.so"))
-    lib.sees.restype = ctypes.c_long
-    return lib
+    return load(tmp_path_factory.mktemp("rules"))
 
 
 def dkdv(r, causal, nq, nk, npairs):
@@ -72,16 +28,6 @@ def dq(r, causal, nq, nk, npairs):
     if r.bwd_qpair(causal, nq, nk, npairs, CUS):
         return "pair"
     return "q64" if r.bwd_q64(causal, nq, nk, npairs, CUS) else "compiled"
-
-
-def stage2_order(r, causal, nq, nk, npairs):
-    """`pairs` of bwdbwd_k_kernel: 128-key blocks, two workgroups per CU."""
-    return r.pairing(causal, nq, nk, (nk + 127) // 128, npairs, 2 * CUS, 2)
-
-
-def one_wave_order(r, causal, nq, nk, n, npairs):
-    """`pairs` of the kernels with 256-row blocks, one workgroup per CU."""
-    return r.pairing(causal, nq, nk, (n + 255) // 256, npairs, CUS, 1)
 
 
 # batch, length, heads (square, top-left causal): dK/dV, dQ, stage 2, its block order
@@ -341,3 +287,16 @@ DEAL = [
 def test_deal(rules, row):
     batch, nq, nk, heads, causal, want = row
     assert bool(rules.q32_deal(causal, nq, nk, batch * heads, CUS)) == want
+
+
+# batch, n_q, n_k, rows blocked, heads, causal: `pairs` of the kernels with 256-row blocks
+ONE_WAVE_ORDER = [
+    (4, 2048, 2048, 2048, 16, 1, 1), (8, 2048, 2048, 2048, 12, 1, 0), (16, 1536, 1536, 1536, 16, 1, 1),
+    (2, 2048, 2048, 2048, 16, 1, 0), (24, 2048, 2048, 2048, 16, 1, 1), (4, 2048, 2048, 2048, 16, 0, 0),
+]
+
+
+@pytest.mark.parametrize("row", ONE_WAVE_ORDER, ids=str)
+def test_one_wave_order(rules, row):
+    batch, nq, nk, n, heads, causal, want = row
+    assert one_wave_order(rules, causal, nq, nk, n, batch * heads) == want
