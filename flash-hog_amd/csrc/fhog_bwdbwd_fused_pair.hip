@@ -130,9 +130,7 @@ bwdbwd_fused_pair_kernel(BwdBwdParams<T> p, int chunk, int fold) {
         r1[ks] = *reinterpret_cast<const V8<T>*>(p.ddq + off);
       } else {
         r0[ks] = *reinterpret_cast<const V8<T>*>(p.dout + off);
-        const V8<T> of = *reinterpret_cast<const V8<T>*>(p.o + off);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) dpart += (float)of[e] * (float)r0[ks][e];
+        dpart = dot8<T>(*reinterpret_cast<const V8<T>*>(p.o + off), r0[ks], dpart);
       }
     }
     if constexpr (PRE && role == 0) {
