@@ -18,9 +18,10 @@
 // takes half the time per tile, and a workgroup is 64 keys instead of 128, so
 // small and grouped-head grids spread over twice as many CUs. The price is the
 // exchange: 8 KiB of LDS traffic beside 32 KiB of operand reads per 32 x 32
-// tile at D = 128 (at D = 64 beside 16 KiB). What bounds it is LDS bandwidth: 40 KiB
-// and the row constants take about 380 cycles per tile and CU at D = 128,
-// against 256 cycles of matrix work.
+// tile at D = 128 (at D = 64 beside 16 KiB). What bounds it is latency: at B2
+// N8192 H16 D = 128 the matrix pipes are busy 47 % of the cycles and the LDS 63 %, 24
+// points of it bank conflicts, while a wave waits half of its time for operands, the
+// exchange and the barriers.
 //
 // First backward (dQ kernel included), us, before -> with this kernel, causal
 // bf16 unless named: B2 N2048 H32 over 8 key heads D128 642 -> 364; B4 N2048
@@ -32,6 +33,9 @@
 // one in its middle the exchange, which needs one buffer per pair and a ring of
 // two stages, so that two or three workgroups share a CU (a wave B one tile
 // behind A needs one barrier, but a ring stage and a buffer more: 0-3 % slower).
+// The two roles run separate copies of the sweep and must reach the same barriers:
+// every one of them stands outside the role's and the mask's branches, and the number
+// of tiles is the workgroup's.
 #pragma once
 
 #include "fhog_device.h"

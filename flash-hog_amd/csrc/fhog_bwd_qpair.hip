@@ -18,6 +18,10 @@
 // N2048 H8 D256 causal bf16 247 -> 199, B4 N2048 H16 D256 642 -> 600, fp32 B2
 // N2048 H8 D64 causal 378 -> 289, B4 N2048 H16 D64 1015 -> 976, B1 N2048 H8 D128
 // non-causal 680 -> 494; 2-byte small grids: B1 N2048 H8 D128 118 -> 109.
+//
+// The two roles run separate copies of the sweep and must reach the same barriers:
+// every one of them stands outside the role's and the mask's branches, and the number
+// of tiles is the workgroup's.
 #include "fhog_device.h"
 #include "fhog_params.h"
 

@@ -12,9 +12,10 @@
 // kernel gives a wave 16 queries on the 16x16x32 instruction and reads each
 // key-side tile from LDS once per 16 queries: 128 KiB per 32 x 32 tile. Two waves
 // share the accumulators of 32 queries (two each, 256 registers) on the 32x32x16
-// instruction and read 72 KiB, with 16 KiB of exchange. Bound by the matrix pipe
-// and LDS bandwidth, about 700-800 cycles per tile and CU each, which two waves
-// per SIMD overlap by half.
+// instruction and read 72 KiB, with 16 KiB of exchange. What bounds it is
+// latency: at B2 N8192 H16 the matrix pipes are busy 51 % of the cycles and the LDS
+// 49 %, 21 points of it bank conflicts; two waves per SIMD each wait 43 % of their time,
+// and 20-92 bytes per lane are spilled, part of them in the loop.
 //
 // Two workgroup shapes give the same bits: two pairs (two workgroups per CU) for
 // grids that do not fill the chip, four (waves w and w + 4, the two of a pair,
@@ -22,6 +23,10 @@
 // Stage 1, us, before -> with this kernel: B2 N8192 H16 causal bf16 2924 -> 2743, B4
 // N2048 H16 non-causal 759 -> 679, B2 N2048 H32 over 8 key heads 397 -> 372, B1
 // N1024 H8 73 -> 66.
+//
+// The two roles run separate copies of the sweep and must reach the same barriers:
+// every one of them stands outside the role's and the mask's branches, and the number
+// of tiles is the workgroup's.
 #include <cmath>
 #include <type_traits>
 

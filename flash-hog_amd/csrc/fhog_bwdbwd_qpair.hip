@@ -27,10 +27,14 @@
 // registers) lets two waves share a SIMD, and a block is 64 queries at half the
 // time per tile. Two waves wait for each other in every tile, though, and wave A
 // has more to do in sweep 1: on grids that fill the chip bwdbwd_q_kernel
-// (fhog_bwdbwd.hip) is faster, and the launch chooses by grid size (the figures
-// are there). Bound by the fp32 matrix rate and, small grids, by the chain of a
+// (fhog_bwdbwd.hip) is faster, and the launch chooses by grid size
+// (stage1_qpair_rule). Bound by the fp32 matrix rate and, small grids, by the chain of a
 // block: stage 1 at B2 N2048 H8 D64 causal 887 -> 631 us, at B1 N2048 H8 D128
 // non-causal 1647 -> 1255.
+//
+// The two roles run separate copies of the sweep and must reach the same barriers:
+// every one of them stands outside the role's and the mask's branches, and the number
+// of tiles is the workgroup's.
 #include "fhog_device.h"
 #include "fhog_params.h"
 

@@ -1,6 +1,6 @@
 // Flash attention forward with two waves per 32 queries, for 2-byte types at
-// D = 256 and for fp32 on small grids (fhog_fwd.hip holds the other kernel, the
-// rule between them and the definitions of O and L). Each wave of a pair holds half of Q's and
+// D = 256 and for fp32 on small grids (fhog_fwd.hip holds the other kernel and
+// the definitions of O and L, fhog_grid.h the rule between them). Each wave of a pair holds half of Q's and
 // half of O's columns: it forms its half of the contraction of S^T = K Q^T, adds
 // its partner's half through LDS (fp32, accumulator layout: lane l reads what
 // lane l of the partner wrote), takes the softmax of the whole tile and
@@ -15,6 +15,10 @@
 // beside 32 KiB of operand reads at D = 256. us, before -> with this kernel: B2
 // N2048 H8 D256 causal bf16 107 -> 77, B4 N2048 H16 D256 248 -> 212, fp32 B2 N2048
 // H8 D64 causal 140 -> 99, fp32 B1 N2048 H8 D128 non-causal 271 -> 166.
+//
+// The two halves run separate copies of the sweep and must reach the same barriers:
+// every one of them stands outside the half's and the mask's branches, and the number
+// of tiles is the workgroup's.
 #include "fhog_device.h"
 #include "fhog_params.h"
 

@@ -86,11 +86,13 @@ hipError_t launch_bwdbwd_stage1_q32(const BwdBwdParams<T>& p, hipStream_t s);
 template <bool CAUSAL>
 hipError_t launch_bwdbwd_stage2_k32(const BwdBwdParams<__bf16>& p, hipStream_t s);
 // The first backward's dK/dV kernel with 64 keys per wave at one wave per SIMD
-// (2-byte types, D = 64); launch_bwd selects it for grids of whole rounds.
+// (2-byte types, D = 64); launch_bwd selects it where its blocks cover little more than
+// 128-key ones, on causal grids and on others of whole rounds (bwd_k64_rule).
 template <typename T, bool CAUSAL>
 hipError_t launch_bwd_k64(const BwdParams<T>& p, hipStream_t s);
 // The first backward's dQ kernel with 64 queries per wave at one wave per SIMD
-// (2-byte types, D = 64); launch_bwd selects it for grids of whole rounds.
+// (2-byte types, D = 64); launch_bwd selects it where its blocks cover little more than
+// 128-query ones, on grids of whole rounds (bwd_q64_rule).
 template <typename T, bool CAUSAL>
 hipError_t launch_bwd_q64(const BwdParams<T>& p, hipStream_t s);
 // dQ and D of the first backward with two waves per 32 queries (all types and
@@ -98,7 +100,8 @@ hipError_t launch_bwd_q64(const BwdParams<T>& p, hipStream_t s);
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd_qpair(const BwdParams<T>& p, hipStream_t s);
 // dK and dV of the first backward with two waves per 32 keys (all types and
-// head dims; at 2-byte D = 64 launch_bwd selects it for small grids).
+// head dims; at 2-byte D = 64 launch_bwd selects it for small grids and short causal
+// problems, bwd_pair_rule).
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd_pair(const BwdParams<T>& p, hipStream_t s);
 // Stage 1 for fp32 with two waves per 32 queries; launch_bwdbwd selects it for
