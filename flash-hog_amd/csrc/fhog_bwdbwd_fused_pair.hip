@@ -15,7 +15,7 @@
 // instruction and read 72 KiB, with 16 KiB of exchange. What bounds it is
 // latency: at B2 N8192 H16 the matrix pipes are busy 51 % of the cycles and the LDS
 // 49 %, 21 points of it bank conflicts; two waves per SIMD each wait 43 % of their time,
-// and 20-92 bytes per lane are spilled, part of them in the loop.
+// and 20-88 bytes per lane are spilled, part of them in the loop.
 //
 // Two workgroup shapes give the same bits: two pairs (two workgroups per CU) for
 // grids that do not fill the chip, four (waves w and w + 4, the two of a pair,
