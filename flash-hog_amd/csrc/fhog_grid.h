@@ -185,8 +185,15 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 inline bool one_wave_grid(int workgroups, int resident) {
   return resident > 0 && workgroups > 0 && (workgroups % resident == 0 || workgroups >= 6 * resident);
 }
-// Whether 256-row blocks cover at most `percent` of what 128-row ones do.
+// Whether 256-row blocks cover at most `percent` of what 128-row ones do. Blocks that see
+// nothing (keys past the last query, queries before the first key) cost their launch
+// and a store of zeros each, half as many with 256 rows; with any of them a grid counts
+// as the square of all its rows (first backward, us, k64 / compiled dK/dV: 512 queries of
+// 4096 keys B16 H12 85.4 / 107, of 2048 B32 135 / 144; q64 / compiled dQ: 4096 queries of 512
+// keys bottom-right B16 128 / 148, 2048 of 512 B32 168 / 180).
 inline bool one_wave_cover(Mask m, bool key_tiled, int percent) {
+  const bool empty = m.causal && (key_tiled ? m.nk > m.nq + (long)m.coff : m.coff < 0);
+  if (empty) m.nq = m.nk = key_tiled ? m.nk : m.nq, m.coff = 0;
   return 100 * 2 * blocks_see(m, 256, key_tiled) <= percent * blocks_see(m, 128, key_tiled);
 }
 // Whether the whole rounds of q64 or k64 are there (n: the blocked side).

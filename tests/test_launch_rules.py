@@ -121,6 +121,7 @@ DQ = [
     (8, 512, 8192, 16, 2, "q64"),
     (64, 512, 640, 12, 2, "compiled"), (64, 256, 512, 12, 2, "compiled"), (128, 512, 512, 12, 1, "compiled"),
     (1, 512, 512, 12, 1, "pair"), (2, 512, 4096, 12, 2, "pair"),
+    (16, 4096, 512, 12, 2, "q64"), (32, 2048, 512, 12, 2, "q64"),
 ]
 
 
@@ -154,6 +155,7 @@ DKDV = [
     (64, 1000, 1000, 12, 1, "pair"), (32, 1100, 1100, 16, 1, "compiled"),
     (2, 8192, 2048, 12, 1, "k64"), (4, 4096, 1024, 12, 1, "k64"), (1, 1024, 4096, 12, 2, "k64"),
     (2, 3072, 2048, 12, 1, "pair"), (2, 8192, 2048, 8, 1, "pair"),
+    (16, 512, 4096, 12, 1, "k64"), (32, 512, 2048, 12, 1, "k64"), (32, 1024, 2048, 12, 1, "k64"),
 ]
 
 
