@@ -122,6 +122,7 @@ DQ = [
     (64, 512, 640, 12, 2, "compiled"), (64, 256, 512, 12, 2, "compiled"), (128, 512, 512, 12, 1, "compiled"),
     (1, 512, 512, 12, 1, "pair"), (2, 512, 4096, 12, 2, "pair"),
     (16, 4096, 512, 12, 2, "q64"), (32, 2048, 512, 12, 2, "q64"),
+    (32, 1024, 512, 16, 1, "q64"), (32, 1024, 512, 8, 1, "q64"), (32, 1500, 1500, 12, 1, "compiled"),
 ]
 
 
