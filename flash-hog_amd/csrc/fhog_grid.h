@@ -71,7 +71,8 @@ inline int fold_rank(bool causal, int nb, int npairs, int cus) {
 // 442 / 387; 0.88, B4 N2048 H14, 145 / 144; 1.06, B2 N4096 H17, 411 / 314; 1.5, B16 N1024
 // H12, 132 / 122; 2.25, B24 N1024 H12, 216 / 194). At two workgroups per CU that is
 // - one round, skewed if nb allows (B4 N2048 H16 138 / 148, B1 N16384 H8 944 / 1021), or
-//   15/16 of one (B2 N4096 H15 274 / 282, B4 N2048 H15 150 / 153);
+//   15/16 of one near a square (B2 N4096 H15 274 / 282, B4 N2048 H15 150 / 153; but 1200
+//   queries of 2500 keys bottom-right B7 H7 143 / 132);
 // - more rounds of few blocks per pair. What decides is which of the two orders is
 //   chunked (grid_chunk, over 8 rounds), so that a pair's blocks run close together.
 //   Neither (up to 8 rounds of single blocks): fewer than 8 (nb = 2, B128 N256 H16 204 /
@@ -97,7 +98,7 @@ inline int block_pairing(Mask m, int nb, int npairs, int resident, int waves) {
   if (!m.causal || resident <= 0) return 0;
   if (waves == 2 && nb >= 32 && single == resident && 2 * paired == resident) return near_square(m, 32);
   if (single <= resident) return 0;
-  if (waves == 2 && paired < resident) return 16 * paired >= 15L * resident;
+  if (waves == 2 && paired < resident) return near_square(m, 4) && 16 * paired >= 15L * resident;
   if (paired % resident != 0) return 0;
   if (waves != 2) return 1;
   if (paired == resident) return nb % 4 == 0 ? 2 : 1;

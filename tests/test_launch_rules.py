@@ -207,6 +207,7 @@ STAGE2_ORDER = [
     (1, 8192, 8192, 8, 1, 1), (2, 4096, 4096, 8, 1, 1), (1, 8192, 8192, 8, 2, 1), (1, 6144, 8192, 8, 1, 1),
     (2, 16384, 4096, 8, 1, 0), (2, 5120, 4096, 8, 1, 0), (2, 2048, 4096, 8, 2, 0), (4, 512, 4096, 4, 2, 0),
     (1, 9216, 8192, 8, 1, 0), (2, 4096, 4096, 9, 1, 0), (2, 4096, 4096, 15, 1, 1), (4, 2048, 2048, 15, 1, 1),
+    (7, 1200, 2500, 7, 2, 0), (31, 4096, 2048, 2, 1, 0), (31, 2400, 2048, 2, 1, 1),
     (4, 2048, 2048, 14, 1, 0), (4, 2048, 2048, 17, 1, 0), (4, 2048, 2048, 16, 1, 2), (3, 2048, 2048, 12, 1, 0),
     # several whole rounds: neither order chunked, the single blocks only, both
     (128, 256, 256, 16, 1, 1), (64, 512, 512, 8, 1, 1), (16, 1024, 1024, 16, 1, 0), (8, 2048, 2048, 16, 1, 0),
