@@ -214,7 +214,9 @@ STAGE2_ORDER = [
     (192, 256, 256, 16, 1, 1), (96, 384, 384, 16, 1, 1), (128, 512, 512, 12, 1, 0), (96, 512, 512, 16, 1, 0),
     (64, 768, 768, 16, 1, 0), (1, 32768, 32768, 8, 1, 0),
     (384, 256, 256, 16, 1, 1), (160, 512, 512, 16, 1, 1), (96, 1024, 1024, 16, 1, 1), (64, 1536, 1536, 16, 1, 1),
-    (64, 2048, 2048, 16, 1, 0), (4, 2048, 2048, 8, 1, 0), (1, 8192, 8192, 8, 0, 0),
+    (64, 2048, 2048, 16, 1, 0),
+    # half of the key blocks and more see no query
+    (16, 512, 4096, 12, 1, 1), (32, 1024, 2048, 12, 1, 1), (8, 1024, 2048, 16, 1, 0), (32, 1500, 2048, 12, 1, 0), (4, 2048, 2048, 8, 1, 0), (1, 8192, 8192, 8, 0, 0),
 ]
 
 
