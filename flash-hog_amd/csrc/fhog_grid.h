@@ -152,9 +152,9 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 // The one-wave kernels (k64, q64) are the fastest per tile, but run one 256-row
 // block per CU at a time and gain nothing when a CU is left alone. They are taken
 // when their blocks cover little more than 128-row ones, in padding and, causal,
-// past the diagonal: up to 6 % more for dQ (8 % on causal rectangles, whose rows are
-// not ragged by it: 1024 queries of 512 keys B32 H8 137 / 144, H16 270 / 276, B64 H16 547 /
-// 543), 10 % for dK/dV (first backward, us, causal
+// past the diagonal: up to 6 % more for dQ (8 % where queries outnumber the keys of a
+// top-left mask: 1024 of 512 B32 H8 137 / 144, H16 270 / 276, B64 H16 547 / 543; but 512 of
+// 1024 bottom-right B64 H12 416 / 409), 10 % for dK/dV (first backward, us, causal
 // bf16, one-wave / compiled for dQ: 6 % more, B8 N2048 H16 280 / 297 with both halves;
 // 8 %, B8 N4736 H12 977 / 977; 11 %, B8 N3200 H12 506 / 503; 16 %, B32 N2117 H16 fp16 1446 /
 // 1386; 23 %, B24 N1300 H12 348 / 319; 24 %, B32 N1408 H16 681 / 633; for dK/dV: 4 %, B8
@@ -210,7 +210,7 @@ inline bool one_wave_rounds(Mask m, int n, int npairs, int cus) {
   return one_wave_grid((mirrored ? (nb + 1) / 2 : nb) * npairs, cus);
 }
 inline bool bwd_q64_rule(Mask m, int npairs, int cus) {
-  return one_wave_cover(m, false, near_square(m, 4) || !m.causal ? 106 : 108) && one_wave_rounds(m, m.nq, npairs, cus);
+  return one_wave_cover(m, false, m.causal && m.coff == 0 && !near_square(m, 4) ? 108 : 106) && one_wave_rounds(m, m.nq, npairs, cus);
 }
 inline bool bwd_k64_rule(Mask m, int npairs, int cus) {
   return one_wave_cover(m, true, 110) && (m.causal || one_wave_rounds(m, m.nk, npairs, cus));
