@@ -4,6 +4,8 @@
 // Figures in the comments are from one MI355X (256 CUs).
 #pragma once
 
+#include <initializer_list>
+
 namespace fhog {
 
 // Query i sees key j iff j <= i + coff (causal), or always. coff is 0 (top-left)
@@ -294,39 +296,79 @@ inline bool stage2_pair_rule(Mask m, int npairs, int cus) {
   return (long)((m.nk + 63) / 64) * npairs <= (!m.causal ? 1L : near_square(m, 4) ? 3L : 2L) * cus;
 }
 
-// Whether a causal grid deals its blocks one by one instead of folding them
-// (bwdbwd_q32_kernel; both give the same bits): when every block can have a CU of
-// its own, or when the folded items' rounds take so much longer than the dealt blocks:
-// 8 % near a square, 19 % on rectangles, where dealing gives up more of the tiles that a
-// pair's blocks share in L2. Dealt blocks take at least the longest block, an even share
-// of all, and as many shortest blocks as some CU gets. Stage 1, us, folded / dealt: one
-// round of blocks, B1 N512 H12 28.6 / 20.5, B1 N1024 H12 41.8 / 33.7, B1 N2048 H12 67.5 / 62.0;
-// estimated gain 12 %, B4 N1024 H12 46.0 / 44.6; 11 %, B24 N1024 H12 258 / 248; 33 %, B1
-// N8192 H12 650 / 518; 36 %, B8 N1500 H12 fp16 218 / 176; 50 %, B3 N2048 H12 155 / 115; but
-// 7 %, B40 N1024 H12 414 / 422; 6 %, B2 N2048 H12 77.0 / 78.4; 3 %, B1 N4096 H12 141 / 149
-// (fewer CUs run faster); none, B32 N1024 H12 324 / 332, B4 N2048 H16 182 / 183.
-// Rectangles, H12: 42 %, 1024 queries of 8192 keys bottom-right B7 1105 / 870, 600 of 3000
-// B12 378 / 312; 25 %, 4096 of 1024 B6 371 / 329; 20 %, 900 of 2000 bottom-right B13 371 / 328;
-// but 18 %, 5000 of 1000 B2 153 / 155; 14 %, 1024 of 4096 bottom-right B28 1578 / 1631, B4 H10
-// 209 / 220; 6 %, 1024 of 8192 B4 462 / 475; none, 1024 of 4096 B32 1618 / 1839.
-inline bool q32_deal_rule(Mask m, int npairs, int cus) {
+// Keys that the busiest workgroup of a causal grid of bwdbwd_q32_kernel sweeps, in each of
+// its two block lists: `cus` workgroups (or one per item) walk the list in strides of their
+// number, see fhog_bwdbwd_q32.hip.
+struct Q32Load {
+  double folded, dealt;
+};
+inline Q32Load q32_load(Mask m, int npairs, int cus) {
   constexpr int kRows = 128;
-  const long nqb = ((long)m.nq + kRows - 1) / kRows, blocks = npairs * nqb;
-  if (!m.causal) return false;
-  if (blocks <= cus) return true;
-  if (cus <= 0) return false;
+  const long nqb = ((long)m.nq + kRows - 1) / kRows, npr = (nqb + 1) / 2;
   auto keys = [&](long qb) {
     const long e = (qb + 1) * kRows + m.coff;
     return (double)(e < 0 ? 0 : e < m.nk ? e : m.nk);
   };
   auto most = [](double a, double b) { return a > b ? a : b; };
-  const double first = keys(0), last = keys(nqb - 1);
-  const long mid = (nqb - 1) / 2;
-  const double item = most(first + last, keys(mid) + keys(nqb - 1 - mid));  // the longest of the folded items
-  const double rounds = (double)((npairs * ((nqb + 1) / 2) + cus - 1) / cus);
-  const double share = (double)npairs * blocks_see(m, kRows, false) / cus;
-  const double dealt = most(most(last, share), (double)((blocks + cus - 1) / cus) * first);
-  return rounds * item > (near_square(m, 4) ? 1.08 : 1.19) * dealt;
+  // Item r: the r-th block from either end. Workgroup w gets items w, w + cus, ..., so the
+  // items r of each pair come round with period npr / gcd(cus, npr). In a square all
+  // items are equal; with very many the mean serves.
+  auto item = [&](long r) { return keys(nqb - 1 - r) + (2 * r + 1 == nqb ? 0.0 : keys(r)); };
+  const long items = npairs * npr, rounds = (items + cus - 1) / cus;
+  double folded = 0;
+  if (m.coff >= 0 && near_square(m, 1 << 20)) {
+    folded = (double)rounds * (nqb > 1 ? item(0) : keys(0));
+  } else if (npr * rounds > 4096) {
+    folded = (double)rounds * blocks_see(m, kRows, false) / (double)npr;
+  } else {
+    for (long w = 0; w < npr && w < items && w < cus; ++w) {
+      double sum = 0;
+      for (long i = w; i < items; i += cus) sum += item(i % npr);
+      folded = most(folded, sum);
+    }
+  }
+  // Blocks longest first, every other round in reverse: the busiest workgroup is the first
+  // or the last of the rounds, or the last one that gets a block of the final round.
+  const long blocks = npairs * nqb, full = blocks / cus, rest = blocks % cus;
+  const long mean = 64;  // rounds after which the share is near enough
+  double dealt = (double)npairs * blocks_see(m, kRows, false) / cus;
+  if (full < mean) {
+    const long last = full & 1 ? cus - rest : rest - 1;
+    for (const long w : {0L, cus - 1L, rest > 0 ? last : 0L}) {
+      double sum = 0;
+      for (long k = 0;; ++k) {
+        const long i = k * cus + (k & 1 ? cus - 1 - w : w);
+        if (i >= blocks) break;
+        sum += keys(nqb - 1 - i / npairs);
+      }
+      dealt = most(dealt, sum);
+    }
+  }
+  return Q32Load{folded, dealt};
+}
+
+// Whether a causal grid deals its blocks one by one instead of folding them
+// (bwdbwd_q32_kernel; both give the same bits): when every block can have a CU of
+// its own, or when the busiest workgroup of the folded list has so much more to sweep than
+// that of the dealt one: 7 % near a square, 15 % on rectangles, where dealing gives up more
+// of the tiles that a pair's blocks share in L2. Stage 1, us, folded / dealt: one
+// round of blocks, B1 N512 H12 28.6 / 20.5, B1 N1024 H12 41.8 / 33.7, B1 N2048 H12 67.5 / 62.0;
+// 12 % more in the folded list, B4 N1024 H12 46.0 / 44.6; 10 %, B24 N1024 H12 258 / 248; 20 %,
+// B1 N8192 H12 650 / 518; 31 %, B8 N1500 H12 fp16 218 / 176; 62 %, B3 N2048 H12 155 / 115; but
+// 6 %, B2 N2048 H12 77.0 / 78.4; 3 %, B1 N4096 H12 141 / 149 (fewer CUs run faster); 1 %, B40
+// N1024 H12 414 / 422; none, B32 N1024 H12 324 / 332, B4 N2048 H16 182 / 183.
+// Rectangles, H12: 34 %, 1024 queries of 8192 keys bottom-right B7 1105 / 870, 600 of 3000
+// B12 378 / 312; 23 %, 4096 of 1024 B6 371 / 329; 21 %, 900 of 2000 bottom-right B13 371 / 328;
+// but 12 %, 4096 of 1024 B4 H16 300 / 288; 10 %, 1024 of 4096 bottom-right B28 1578 / 1631; 7 %,
+// B4 H10 209 / 220; 2 %, 1024 of 8192 B4 462 / 475; none, 1024 of 4096 B32 1618 / 1839. With rows that
+// see no key: 76 %, 2048 of 1024 bottom-right B24 330 / 273; 6 %, 1664 of 768 B35 H16 354 / 374.
+inline bool q32_deal_rule(Mask m, int npairs, int cus) {
+  const long blocks = npairs * (((long)m.nq + 127) / 128);
+  if (!m.causal) return false;
+  if (blocks <= cus) return true;
+  if (cus <= 0) return false;
+  const Q32Load load = q32_load(m, npairs, cus);
+  return load.folded > (near_square(m, 4) ? 1.07 : 1.15) * load.dealt;
 }
 
 }  // namespace fhog

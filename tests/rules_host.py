@@ -34,6 +34,8 @@ int stage1_fused(int c, int nq, int nk) { return fhog::stage1_fused_rule(mask(c,
 int stage1_qpair(int c, int nq, int nk, int np, int cus) { return fhog::stage1_qpair_rule(mask(c, nq, nk), np, cus); }
 int stage2_pair(int c, int nq, int nk, int np, int cus) { return fhog::stage2_pair_rule(mask(c, nq, nk), np, cus); }
 int q32_deal(int c, int nq, int nk, int np, int cus) { return fhog::q32_deal_rule(mask(c, nq, nk), np, cus); }
+double q32_folded(int c, int nq, int nk, int np, int cus) { return fhog::q32_load(mask(c, nq, nk), np, cus).folded; }
+double q32_dealt(int c, int nq, int nk, int np, int cus) { return fhog::q32_load(mask(c, nq, nk), np, cus).dealt; }
 int pairing(int c, int nq, int nk, int nb, int np, int resident, int waves) {
   return fhog::block_pairing(mask(c, nq, nk), nb, np, resident, waves);
 }
@@ -56,6 +58,7 @@ def load(directory):
     subprocess.run(cmd, check=True)
     lib = ctypes.CDLL(str(directory / "rules.so"))
     lib.sees.restype = ctypes.c_long
+    lib.q32_folded.restype = lib.q32_dealt.restype = ctypes.c_double
     return lib
 
 

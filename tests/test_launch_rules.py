@@ -8,6 +8,8 @@ measured the faster one there; the times stand beside the rules.
 
 from __future__ import annotations
 
+import random
+
 import pytest
 
 from rules_host import CUS, load, one_wave_order, stage2_order
@@ -283,6 +285,8 @@ DEAL = [
     (32, 1024, 1024, 12, 1, False), (4, 2048, 2048, 16, 1, False),
     (7, 1024, 8192, 12, 2, True), (12, 600, 3000, 12, 2, True), (6, 4096, 1024, 12, 1, True),
     (13, 900, 2000, 12, 2, True), (1, 8192, 4096, 12, 1, True), (24, 2048, 1024, 12, 2, True),
+    (9, 1500, 3000, 10, 2, True), (9, 3000, 1500, 10, 1, True), (32, 2048, 512, 12, 2, True),
+    (35, 1664, 768, 16, 2, False), (66, 1152, 128, 4, 2, False), (487, 681, 681, 1, 1, False),
     (28, 1024, 4096, 12, 2, False), (4, 1024, 4096, 10, 2, False), (4, 1024, 8192, 12, 2, False),
     (3, 1024, 8192, 16, 2, False), (2, 5000, 1000, 12, 1, False), (32, 1024, 4096, 12, 2, False),
     (3, 2048, 2048, 12, 0, False),
@@ -306,3 +310,42 @@ ONE_WAVE_ORDER = [
 def test_one_wave_order(rules, row):
     batch, nq, nk, n, heads, causal, want = row
     assert one_wave_order(rules, causal, nq, nk, n, batch * heads) == want
+
+
+def _walk(causal, nq, nk, npairs):
+    """The most keys that a workgroup sweeps in the folded and in the dealt list, walked as the kernel does."""
+    coff = nk - nq if causal == 2 else 0
+    nqb = -(-nq // 128)
+    npr = (nqb + 1) // 2
+    keys = [min(nk, max(0, (i + 1) * 128 + coff)) for i in range(nqb)]
+    item = [keys[nqb - 1 - r] + (keys[r] if 2 * r + 1 != nqb else 0) for r in range(npr)]
+    n = npairs * npr
+    folded = max(sum(item[i % npr] for i in range(w, n, CUS)) for w in range(min(CUS, n)))
+    n = npairs * nqb
+    grid = min(CUS, n)
+    dealt = [0] * grid
+    for k in range(-(-n // grid)):
+        for w in range(grid):
+            i = k * grid + (((grid // 8 - 1 - w // 8) * 8 + w % 8 if grid % 8 == 0 else grid - 1 - w) if k % 2 else w)
+            if i < n:
+                dealt[w] += keys[nqb - 1 - i // npairs]
+    return folded, max(dealt)
+
+
+def test_q32_load(rules):
+    """The estimate of the rule is the walk's: exactly for folded lists of up to 4096 steps, to the
+    reversed groups of eight workgroups (a block more or less in the last round) for dealt ones."""
+    rng = random.Random(3)
+    for _ in range(300):
+        causal, nq, npairs = rng.choice((1, 2)), rng.randint(1, 40) * 128, rng.randint(1, 400)
+        nk = nq if rng.random() < 0.3 else rng.randint(1, 40) * 128
+        if npairs * nq // 128 <= CUS:
+            continue
+        folded, dealt = _walk(causal, nq, nk, npairs)
+        got = rules.q32_folded(causal, nq, nk, npairs, CUS), rules.q32_dealt(causal, nq, nk, npairs, CUS)
+        npr, coff = (nq // 128 + 1) // 2, nk - nq if causal == 2 else 0
+        equal = coff >= 0 and max(coff, nq - nk + coff) <= 0  # every item but a middle one
+        if npr * (-(-npairs * npr // CUS)) <= 4096 and not equal:
+            assert got[0] == folded, (causal, nq, nk, npairs)
+        assert abs(got[0] - folded) <= 0.05 * folded + nq, (causal, nq, nk, npairs, got, folded)
+        assert abs(got[1] - dealt) <= 0.05 * dealt + 128, (causal, nq, nk, npairs, got, dealt)
