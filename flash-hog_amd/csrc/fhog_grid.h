@@ -85,9 +85,10 @@ inline int fold_rank(bool causal, int nb, int npairs, int cus) {
 //   N32768 H8 3795 / 3720). Both: fewer than 16 (2, B384 N256 H16 565 / 580; 3, B192 N384 H16
 //   461 / 487; 4, B160 N512 H16 585 / 595; 8, B96 N1024 H16 1051 / 1067; 12, B64 N1536 H16
 //   1427 / 1447; but 14, B64 N1792 H16 1865 / 1845; 16, B64 N2048 H16 2398 / 2373). Where half
-//   of the blocks or more see no query, pairs spare the chunked order their launches (512
-//   queries of 4096 keys B16 H12 101 / 113, 1024 of 2048 B32 283 / 294; not chunked, 1024 of 2048
-//   B8 H16 95 / 93);
+//   of the blocks or more see no query, the chunked order starts later pairs' longest blocks
+//   late, and pairs, half as many, are taken in any number of rounds (512 queries of 4096 keys
+//   B16 H12 101 / 113, 1024 of 2048 B32 283 / 294, 2325 of 16384 B9 H4 139 / 193; not chunked,
+//   1024 of 2048 B8 H16 95 / 93);
 // - one paired workgroup per CU, from 32 blocks per pair in a square (64, B1 N8192 H8
 //   309 / 320, B2 N8192 H16 over 4 key heads 1230 / 1260; 32, B4 N4096 H16 over 4 key heads
 //   623 / 634; but 16, B4 N2048 H8 92.6 / 90.1). Equal blocks run better two to a CU (B2 H8,
@@ -104,11 +105,11 @@ inline int block_pairing(Mask m, int nb, int npairs, int resident, int waves) {
   if (waves == 2 && nb >= 32 && single == resident && 2 * paired == resident) return near_square(m, 32);
   if (single <= resident) return 0;
   if (waves == 2 && paired < resident) return near_square(m, 4) && 16 * paired >= 15L * resident;
+  if (single > 8L * resident && m.nk >= 2 * (m.nq + (long)m.coff)) return 1;
   if (paired % resident != 0) return 0;
   if (waves != 2) return 1;
   if (paired == resident) return nb % 4 == 0 ? 2 : 1;
   const bool chunked = single > 8L * resident, chunked_pairs = paired > 8L * resident;
-  if (chunked && m.nk >= 2 * (m.nq + (long)m.coff)) return 1;
   return nb < (chunked_pairs ? 16 : chunked ? 4 : 8);
 }
 

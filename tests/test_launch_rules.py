@@ -218,6 +218,7 @@ STAGE2_ORDER = [
     (384, 256, 256, 16, 1, 1), (160, 512, 512, 16, 1, 1), (96, 1024, 1024, 16, 1, 1), (64, 1536, 1536, 16, 1, 1),
     (64, 2048, 2048, 16, 1, 0),
     # half of the key blocks and more see no query
+    (9, 2325, 16384, 4, 1, 1), (13, 1664, 11392, 8, 1, 1),
     (16, 512, 4096, 12, 1, 1), (32, 1024, 2048, 12, 1, 1), (8, 1024, 2048, 16, 1, 0), (32, 1500, 2048, 12, 1, 0), (4, 2048, 2048, 8, 1, 0), (1, 8192, 8192, 8, 0, 0),
 ]
 
