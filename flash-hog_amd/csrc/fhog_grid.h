@@ -312,14 +312,13 @@ inline Q32Load q32_load(Mask m, int npairs, int cus) {
   };
   auto most = [](double a, double b) { return a > b ? a : b; };
   // Item r: the r-th block from either end. Workgroup w gets items w, w + cus, ..., so the
-  // items r of each pair come round with period npr / gcd(cus, npr). In a square all
-  // items are equal; with very many the mean serves.
+  // items r of each pair come round with period npr / gcd(cus, npr). A middle item is one
+  // block, so that three items of a square (five blocks) even out where four do not. With
+  // very many items the mean serves.
   auto item = [&](long r) { return keys(nqb - 1 - r) + (2 * r + 1 == nqb ? 0.0 : keys(r)); };
   const long items = npairs * npr, rounds = (items + cus - 1) / cus;
   double folded = 0;
-  if (m.coff >= 0 && near_square(m, 1 << 20)) {
-    folded = (double)rounds * (nqb > 1 ? item(0) : keys(0));
-  } else if (npr * rounds > 4096) {
+  if (npr * rounds > 4096) {
     folded = (double)rounds * blocks_see(m, kRows, false) / (double)npr;
   } else {
     for (long w = 0; w < npr && w < items && w < cus; ++w) {
