@@ -428,20 +428,20 @@ inline Dkdv dkdv_selected(Mask m, int npairs) {
   return bwd_pair_rule(m, npairs, cus) ? Dkdv::pair : bwd_k64_rule(m, npairs, cus) ? Dkdv::k64 : Dkdv::compiled;
 }
 enum class Dq { compiled, q64, pair };
-inline Dq dq_selected(Mask m, int npairs) {
+inline Dq dq_selected(Mask m, int npairs, int head_dim) {
   const char* v = std::getenv("FLASH_HOG_BWDQ");
   if (v != nullptr && std::strcmp(v, "pair") == 0) return Dq::pair;
   if (v != nullptr && std::strcmp(v, "q64") == 0) return Dq::q64;
   if (v != nullptr && std::strcmp(v, "compiled") == 0) return Dq::compiled;
   const int cus = resident_workgroups(1);
-  return bwd_qpair_rule(m, npairs, cus) ? Dq::pair : bwd_q64_rule(m, npairs, cus) ? Dq::q64 : Dq::compiled;
+  return bwd_qpair_rule(m, npairs, head_dim, cus) ? Dq::pair : bwd_q64_rule(m, npairs, cus) ? Dq::q64 : Dq::compiled;
 }
 
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd_dq(const BwdParams<T>& p, hipStream_t stream) {
   if constexpr (sizeof(T) == 2 && D <= 128) {
     const int npairs = p.batch * p.heads;
-    const Dq sel = dq_selected(mask_of(CAUSAL, p), npairs);
+    const Dq sel = dq_selected(mask_of(CAUSAL, p), npairs, D);
     if (sel != Dq::pair) {
       if constexpr (D == 64) {
         if (sel == Dq::q64) return launch_bwd_q64<T, CAUSAL>(p, stream);

@@ -187,8 +187,10 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 // 8192 of 1024 B8 H16 923 / 1100; non-causal B1 N2048 H16 (512) 95.2 / 92.9, B2 N2048
 // H12 (768) 120 / 117, B8 N1000 H12 fp16 (1536) 122.8 / 124.0). dQ gains less and takes its pair kernel,
 // at D = 64 and 128, up to one workgroup per CU (B1 N512 H12 27.0 / 26.1, B1
-// N2048 H8 D128 non-causal 118 / 109; B2 N1000 H12 fp16, 384 workgroups, 51.2 /
-// 55.7). Short causal sequences gain nothing on fuller grids (compiled / pair: B128 N256
+// N2048 H8 D128 non-causal 119 / 109; B2 N1000 H12 fp16, 384 workgroups, 51.2 /
+// 55.7), at D = 64 up to 2048 keys: it starts 1 us earlier and takes longer per tile (B1 N1024
+// H12 45.5 / 44.9, N2048 H8 81.7 / 81.8, N4096 H4 154 / 155, N8192 H2 298 / 309, 1024 queries of 7168
+// keys bottom-right B6 H1 147 / 158; D128 B6 H1 253 / 232). Short causal sequences gain nothing on fuller grids (compiled / pair: B128 N256
 // H12 168 / 166, B128 N384 H12 292 / 296, B32 N512 H12 101 / 99, B128 N512 H12 408 / 423, over
 // 4 key heads 442 / 467), and a chunk of queries against more keys loses (512 queries
 // of 1024 keys bottom-right B64 H12 409 / 448, of 4096 B32 877 / 1036).
@@ -223,7 +225,11 @@ inline bool bwd_pair_rule(Mask m, int npairs, int cus) {
   if (!m.causal || m.nk > 1024) return false;
   return 1000 * 2 * blocks_see(m, 128, true) >= (near_square(m, 16) ? 1058 : 1065) * blocks_see(m, 64, true);
 }
-inline bool bwd_qpair_rule(Mask m, int npairs, int cus) { return (long)((m.nq + 63) / 64) * npairs <= cus; }
+inline bool bwd_qpair_rule(Mask m, int npairs, int head_dim, int cus) {
+  if ((long)((m.nq + 63) / 64) * npairs > cus) return false;
+  const long last = m.causal && m.nq + (long)m.coff < m.nk ? m.nq + (long)m.coff : m.nk;  // keys of the last query
+  return head_dim > 64 || last <= 2048;
+}
 
 // Waves per SIMD of bwd_pair_kernel. Three workgroups per CU at 256-byte rows (168
 // registers): for fp32 always (D = 64 B4 N2048 H16 1031 -> 1013 us, B2 N2048 H8

@@ -25,7 +25,7 @@ extern "C" {
 int fwd_pair(int c, int nq, int nk, int np, int d, int cus) { return fhog::fwd_pair_rule(mask(c, nq, nk), np, d, cus); }
 int bwd_pair(int c, int nq, int nk, int np, int cus) { return fhog::bwd_pair_rule(mask(c, nq, nk), np, cus); }
 int bwd_k64(int c, int nq, int nk, int np, int cus) { return fhog::bwd_k64_rule(mask(c, nq, nk), np, cus); }
-int bwd_qpair(int c, int nq, int nk, int np, int cus) { return fhog::bwd_qpair_rule(mask(c, nq, nk), np, cus); }
+int bwd_qpair(int c, int nq, int nk, int np, int d, int cus) { return fhog::bwd_qpair_rule(mask(c, nq, nk), np, d, cus); }
 int bwd_q64(int c, int nq, int nk, int np, int cus) { return fhog::bwd_q64_rule(mask(c, nq, nk), np, cus); }
 int bwd_waves(int c, int nq, int nk, int np, int d, int bytes, int cus) {
   return fhog::bwd_pair_waves(mask(c, nq, nk), np, d, bytes, cus);

@@ -26,8 +26,8 @@ def dkdv(r, causal, nq, nk, npairs):
     return "k64" if r.bwd_k64(causal, nq, nk, npairs, CUS) else "compiled"
 
 
-def dq(r, causal, nq, nk, npairs):
-    if r.bwd_qpair(causal, nq, nk, npairs, CUS):
+def dq(r, causal, nq, nk, npairs, d=64):
+    if r.bwd_qpair(causal, nq, nk, npairs, d, CUS):
         return "pair"
     return "q64" if r.bwd_q64(causal, nq, nk, npairs, CUS) else "compiled"
 
@@ -122,7 +122,8 @@ DQ = [
     (64, 512, 1024, 12, 2, "compiled"), (32, 512, 4096, 12, 2, "compiled"),
     (8, 512, 8192, 16, 2, "q64"),
     (64, 512, 640, 12, 2, "compiled"), (64, 256, 512, 12, 2, "compiled"), (128, 512, 512, 12, 1, "compiled"),
-    (1, 512, 512, 12, 1, "pair"), (2, 512, 4096, 12, 2, "pair"),
+    (1, 512, 512, 12, 1, "pair"), (2, 512, 2048, 12, 2, "pair"), (1, 512, 4096, 12, 1, "pair"),
+    (2, 512, 4096, 12, 2, "compiled"), (16, 443, 4058, 2, 2, "compiled"), (1, 8192, 8192, 2, 1, "compiled"),
     (16, 4096, 512, 12, 2, "q64"), (32, 2048, 512, 12, 2, "q64"),
     (32, 1024, 512, 16, 1, "q64"), (32, 1024, 512, 8, 1, "q64"), (32, 1500, 1500, 12, 1, "compiled"),
 ]
@@ -132,6 +133,8 @@ DQ = [
 def test_dq(rules, row):
     batch, nq, nk, heads, causal, want = row
     assert dq(rules, causal, nq, nk, batch * heads) == want
+    small = -(-nq // 64) * batch * heads <= CUS
+    assert (dq(rules, causal, nq, nk, batch * heads, 128) == "pair") == small
 
 
 # batch, n_q, n_k, heads, causal: whether dK/dV's 256-row kernel may run
