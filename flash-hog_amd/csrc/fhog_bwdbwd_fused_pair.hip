@@ -17,9 +17,10 @@
 // 49 %, 21 points of it bank conflicts; two waves per SIMD each wait 43 % of their time,
 // and 20-88 bytes per lane are spilled, part of them in the loop.
 //
-// Two workgroup shapes give the same bits: two pairs (two workgroups per CU) for
-// grids that do not fill the chip, four (waves w and w + 4, the two of a pair,
-// share a SIMD; the key-side tiles are streamed half as often) for the others.
+// Two workgroup shapes give the same bits (stage1_pairs_rule): two pairs (two
+// workgroups per CU) for grids that do not fill the chip and where 128-query blocks would
+// waste rows, four (waves w and w + 4, the two of a pair, share a SIMD; the key-side
+// tiles are streamed half as often) for the others.
 // Stage 1, us, before -> with this kernel: B2 N8192 H16 causal bf16 2924 -> 2743, B4
 // N2048 H16 non-causal 759 -> 679, B2 N2048 H32 over 8 key heads 397 -> 372, B1
 // N1024 H8 73 -> 66.
@@ -339,10 +340,7 @@ hipError_t launch_pairs(const BwdBwdParams<T>& p, int cus, hipStream_t stream) {
 template <typename T, bool CAUSAL>
 hipError_t launch_bwdbwd_stage1_fused_pair(const BwdBwdParams<T>& p, hipStream_t stream) {
   const int cus = resident_workgroups(1);
-  // (64-query workgroups; four pairs against two, us: causal B1 N1024 H8 (128 of
-  // them) 76 / 66, B2 N2048 H32 (2048) 372 / 389; non-causal B1 N2048 H8 (256) 141 /
-  // 127, B4 N2048 H16 (2048) 679 / 734)
-  if ((long)((p.nq + 63) / 64) * p.batch * p.heads <= 2L * cus) return launch_pairs<T, 128, CAUSAL, 2>(p, cus, stream);
+  if (stage1_pairs_rule(mask_of(CAUSAL, p), p.batch * p.heads, cus) == 2) return launch_pairs<T, 128, CAUSAL, 2>(p, cus, stream);
   return launch_pairs<T, 128, CAUSAL, 4>(p, cus, stream);
 }
 

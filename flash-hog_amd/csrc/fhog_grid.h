@@ -267,6 +267,23 @@ inline bool stage1_fused_rule(Mask m) {
   return 100 * 2 * blocks_see(m, 128, false) >= (near_square(m, 16) ? 112 : 115) * blocks_see(m, 64, false);
 }
 
+// Pairs of waves (32 queries each) per workgroup of the D = 128 stage 1,
+// fhog_bwdbwd_fused_pair.hip: two (two workgroups per CU) while the chip is not full of
+// them; where 128-query blocks cover 30 % more than 64-query ones; and where four pairs (one
+// workgroup per CU) make two rounds and less than a third of one. Four otherwise.
+// Stage 1, us, two / four, H16 bf16: small grids, causal B1 N1024 H8 (128 workgroups of 64
+// queries) 66 / 76, non-causal B1 N2048 H8 (256) 127 / 141; cover 100 % more, N64 B64 42 /
+// 60; 46 %, N300 B16 H12 fp16 58 / 73; 33 %, N128 B64 98 / 102; 58 %, 1288 queries of 169 keys
+// bottom-right B84 H8 444 / 480; rounds, 327 queries of 100 keys B23 H8 (2.16) 52 / 62; but 20 %,
+// N256 B64 257 / 254; 14 %, N384 B32 204 / 208; 11 %, N512 B32 335 / 320, B128 H12 897 / 923; N1024
+// B16 505 / 517; B2 N2048 H32 389 / 372; non-causal B4 N2048 734 / 679, N256 B64 352 / 296; 256 of
+// 1024 bottom-right B64 H8 495 / 403.
+inline int stage1_pairs_rule(Mask m, int npairs, int cus) {
+  const long two = (long)((m.nq + 63) / 64) * npairs, four = (long)((m.nq + 127) / 128) * npairs;
+  if (two <= 2L * cus || 10 * 2 * blocks_see(m, 128, false) >= 13 * blocks_see(m, 64, false)) return 2;
+  return four > 2L * cus && 3 * four < 7L * cus ? 2 : 4;
+}
+
 // Stage 1 for fp32 runs bwdbwd_q_kernel (fhog_bwdbwd.hip, one wave per 32 queries) on grids
 // that fill the chip and bwdbwd_qpair_kernel (fhog_bwdbwd_qpair.hip, two waves per
 // 32 queries, half the time per block and twice the workgroups) on smaller ones;

@@ -31,6 +31,7 @@ int bwd_waves(int c, int nq, int nk, int np, int d, int bytes, int cus) {
   return fhog::bwd_pair_waves(mask(c, nq, nk), np, d, bytes, cus);
 }
 int stage1_fused(int c, int nq, int nk) { return fhog::stage1_fused_rule(mask(c, nq, nk)); }
+int stage1_pairs(int c, int nq, int nk, int np, int cus) { return fhog::stage1_pairs_rule(mask(c, nq, nk), np, cus); }
 int stage1_qpair(int c, int nq, int nk, int np, int cus) { return fhog::stage1_qpair_rule(mask(c, nq, nk), np, cus); }
 int stage2_pair(int c, int nq, int nk, int np, int cus) { return fhog::stage2_pair_rule(mask(c, nq, nk), np, cus); }
 int q32_deal(int c, int nq, int nk, int np, int cus) { return fhog::q32_deal_rule(mask(c, nq, nk), np, cus); }

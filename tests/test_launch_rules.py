@@ -353,3 +353,18 @@ def test_q32_load(rules):
             assert got[0] == folded, (causal, nq, nk, npairs)
         assert abs(got[0] - folded) <= 0.05 * folded + nq, (causal, nq, nk, npairs, got, folded)
         assert abs(got[1] - dealt) <= 0.05 * dealt + 128, (causal, nq, nk, npairs, got, dealt)
+
+
+# batch, n_q, n_k, heads, causal: pairs of waves per workgroup of the D = 128 stage 1
+STAGE1_PAIRS = [
+    (1, 1024, 1024, 8, 1, 2), (1, 2048, 2048, 8, 0, 2), (64, 64, 64, 16, 1, 2), (16, 300, 300, 12, 1, 2),
+    (64, 128, 128, 16, 1, 2), (84, 1288, 169, 8, 2, 2), (23, 327, 100, 8, 1, 2),
+    (64, 256, 256, 16, 1, 4), (32, 512, 512, 16, 1, 4), (2, 2048, 2048, 32, 1, 4), (2, 8192, 8192, 16, 1, 4),
+    (4, 2048, 2048, 16, 0, 4), (64, 256, 256, 16, 0, 4), (64, 256, 1024, 8, 2, 4),
+]
+
+
+@pytest.mark.parametrize("row", STAGE1_PAIRS, ids=str)
+def test_stage1_pairs(rules, row):
+    batch, nq, nk, heads, causal, want = row
+    assert rules.stage1_pairs(causal, nq, nk, batch * heads, CUS) == want
