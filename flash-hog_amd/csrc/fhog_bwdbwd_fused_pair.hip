@@ -340,7 +340,8 @@ hipError_t launch_pairs(const BwdBwdParams<T>& p, int cus, hipStream_t stream) {
 template <typename T, bool CAUSAL>
 hipError_t launch_bwdbwd_stage1_fused_pair(const BwdBwdParams<T>& p, hipStream_t stream) {
   const int cus = resident_workgroups(1);
-  if (stage1_pairs_rule(mask_of(CAUSAL, p), p.batch * p.heads, cus) == 2) return launch_pairs<T, 128, CAUSAL, 2>(p, cus, stream);
+  if (stage1_pairs_rule(mask_of(CAUSAL, p), p.batch * p.heads, cus) == 2)
+    return launch_pairs<T, 128, CAUSAL, 2>(p, cus, stream);
   return launch_pairs<T, 128, CAUSAL, 4>(p, cus, stream);
 }
 

@@ -190,8 +190,8 @@ inline bool fwd_pair_rule(Mask m, int npairs, int head_dim, int cus) {
 // N2048 H8 D128 non-causal 119 / 109; B2 N1000 H12 fp16, 384 workgroups, 51.2 /
 // 55.7), at D = 64 up to 2048 keys: it starts 1 us earlier and takes longer per tile (B1 N1024
 // H12 45.5 / 44.9, N2048 H8 81.7 / 81.8, N4096 H4 154 / 155, N8192 H2 298 / 309, 1024 queries of 7168
-// keys bottom-right B6 H1 147 / 158; D128 B6 H1 253 / 232). Short causal sequences gain nothing on fuller grids (compiled / pair: B128 N256
-// H12 168 / 166, B128 N384 H12 292 / 296, B32 N512 H12 101 / 99, B128 N512 H12 408 / 423, over
+// keys bottom-right B6 H1 147 / 158; D128 B6 H1 253 / 232). Short causal sequences gain
+// nothing on fuller grids (compiled / pair: B128 N256 H12 168 / 166, B128 N384 H12 292 / 296, B32 N512 H12 101 / 99, B128 N512 H12 408 / 423, over
 // 4 key heads 442 / 467), and a chunk of queries against more keys loses (512 queries
 // of 1024 keys bottom-right B64 H12 409 / 448, of 4096 B32 877 / 1036).
 inline bool one_wave_grid(int workgroups, int resident) {
@@ -215,7 +215,8 @@ inline bool one_wave_rounds(Mask m, int n, int npairs, int cus) {
   return one_wave_grid((mirrored ? (nb + 1) / 2 : nb) * npairs, cus);
 }
 inline bool bwd_q64_rule(Mask m, int npairs, int cus) {
-  return one_wave_cover(m, false, m.causal && m.coff == 0 && !near_square(m, 4) ? 108 : 106) && one_wave_rounds(m, m.nq, npairs, cus);
+  const int percent = m.causal && m.coff == 0 && !near_square(m, 4) ? 108 : 106;
+  return one_wave_cover(m, false, percent) && one_wave_rounds(m, m.nq, npairs, cus);
 }
 inline bool bwd_k64_rule(Mask m, int npairs, int cus) {
   return one_wave_cover(m, true, 110) && (m.causal || one_wave_rounds(m, m.nk, npairs, cus));

@@ -222,7 +222,8 @@ STAGE2_ORDER = [
     (64, 2048, 2048, 16, 1, 0),
     # half of the key blocks and more see no query
     (9, 2325, 16384, 4, 1, 1), (13, 1664, 11392, 8, 1, 1),
-    (16, 512, 4096, 12, 1, 1), (32, 1024, 2048, 12, 1, 1), (8, 1024, 2048, 16, 1, 0), (32, 1500, 2048, 12, 1, 0), (4, 2048, 2048, 8, 1, 0), (1, 8192, 8192, 8, 0, 0),
+    (16, 512, 4096, 12, 1, 1), (32, 1024, 2048, 12, 1, 1), (8, 1024, 2048, 16, 1, 0), (32, 1500, 2048, 12, 1, 0),
+    (4, 2048, 2048, 8, 1, 0), (1, 8192, 8192, 8, 0, 0),
 ]
 
 
